@@ -17,19 +17,31 @@
 // grid ride on the GEMM's output instead of making their own HBM passes.
 //
 // Shape: Y^T = W X^T on v_mfma_f32_16x16x32_bf16 (A = weight rows from the
-// fragment-packed layout of terra_swin_pack_linear, B = token rows), so an
-// accumulator lane holds four consecutive output features of one token and
-// stores 8 contiguous bytes.  A workgroup (8 waves, one per CU) computes a
-// 256-feature x 256-token tile; wave w owns features 64 (w & 3) .. + 64 of
-// tokens 128 (w >> 2) .. + 128: 4 x 8 accumulator tiles, each weight fragment
-// feeding 8 MFMAs and each token fragment 4.  Per 64-wide stage (two
-// k-steps) the tile's weights (32 packed 1 KB blocks) and token rows (256
-// whole 128-byte lines) stream straight into LDS by global->LDS loads, two
-// 64 KB buffers, one stage ahead, as one stream across a workgroup's tiles;
-// a k-step's fragments are read out of LDS while the previous k-step's MFMAs
-// run.  Measured (MI355X, 156672 rows): 1024 -> 1024 at 34 % of the bf16
-// MFMA peak, 4096 -> 1024 at 40 %, about hipBLASLt's rate for the plain
-// product; the fused epilogues are what it adds.
+// fragment-packed layout of terra_swin_pack_linear, B = token rows).  A
+// workgroup (8 waves, one per CU) computes a 256-feature x 256-token tile;
+// wave w owns features 128 (w >> 2) .. + 128 of tokens 64 (w & 3) .. + 64: 8 x
+// 4 accumulator tiles.  Per 64-wide stage (two k-steps) the tile's weights (32
+// packed 1 KB blocks) and token rows (256 whole 128-byte lines) stream
+// straight into LDS by global->LDS loads, two 64 KB buffers, as one stream
+// across a workgroup's tiles.
+//
+// What bounds it: the matrix cores, fed from LDS, at the clock the power limit
+// leaves (1.5-1.9 GHz under this kernel).  A stage is four phases of 16 MFMAs
+// per wave (one 64 x 32 quadrant each).  The order of MFMAs, fragment reads and
+// loads is pinned (sched_barrier): a phase reads the fragments of the next one
+// right after their registers' last use, so no LDS latency is exposed, and
+// issues a quarter stage (16 KB) into LDS that the phase before last has read
+// out, so eight quarter stages are in flight and the wait at a phase's end
+// (vmcnt(10), with an LDS-only barrier) is for the one issued five phases
+// earlier.  The order before left the reads to the compiler, which placed each
+// next to its MFMA, and waited for a whole stage at once.  Rates (156672 rows,
+// us; before -> after; hipBLASLt's plain product in brackets):
+//   1024 -> 1024  380 -> 325-340 [350-370]     4096 -> 1024 1218 -> 980-1060 [980-1020]
+//   1024 -> 4096 + GELU 1441 -> 1200-1270 [1030-1090 without GELU]
+//   1024 -> 1024 + scatter + residual 440 -> 362
+// A tile's stores (64 contiguous bytes per row and instruction, nontemporal:
+// 192 -> 768 of 524288 rows 290 -> 226 us, the others within 1 %) are waited
+// for only at the end of the next tile's first stage.
 //
 // Tiles are walked persistently and XCD-aware: workgroup b runs on XCD b % 8
 // (the hardware's round-robin), XCD x takes token blocks x, x + 8, ... and
@@ -50,6 +62,8 @@ constexpr int kLinF = 256;                         // output features per tile
 constexpr int kLinT = 256;                         // token rows per tile
 constexpr int kLinKS = 64;                         // input features per stage (two k-steps)
 constexpr int kLinStages = 2;
+constexpr uint32_t kLinDrop = 0xffff0000u;         // byte offset outside every output descriptor (plus a row's column)
+constexpr int kLinStores = 16;                    // output stores per wave and tile (16 bytes per lane)
 constexpr int kLinThreads = 512;
 constexpr int kLinWBytes = kLinF * kLinKS * 2;     // 16 feature tiles x 2 packed 1 KB blocks
 constexpr int kLinXBytes = kLinT * kLinKS * 2;     // 256 rows x 128 bytes
@@ -68,6 +82,7 @@ struct LinParams {
   const uint8_t* res;     // residual (kEpiResidual / kEpiScatter), row stride y_ld
   uint8_t* y;             // output rows, row stride y_ld bytes
   int64_t x_ld, y_ld;
+  int64_t y_bytes;        // kEpiScatter: bytes of y (and res)
   int32_t M, N, K;
   int32_t tiles_m, tiles_n;
   // kEpiScatter: window-order rows of 8x8 windows -> grid tokens
@@ -84,10 +99,10 @@ __device__ __forceinline__ int lin_lane() {
 }
 
 // 16-byte slot of (row, chunk c < 8) in a stage's token rows: 128-byte rows,
-// the chunk XOR-swizzled by (row ^ (row >> 3)) & 7, so that the rows of a
-// fragment read hit distinct banks whether the LDS serves 8 lanes from 128
+// the chunk XOR-swizzled within aligned groups of 16 rows, so that the rows of
+// a fragment read hit distinct banks whether the LDS serves 8 lanes from 128
 // bytes of banks or 16 lanes from 256 bytes per cycle.
-__device__ __forceinline__ int lin_swz(int row) { return (row ^ (row >> 3)) & 7; }
+__device__ __forceinline__ int lin_swz(int row) { return (row ^ ((row >> 3) & 1)) & 7; }
 __device__ __forceinline__ int lin_slot(int row, int c) { return row * 8 + (c ^ lin_swz(row)); }
 
 // Grid token of window-order row m (window m / 64, token m % 64 of an 8x8
@@ -120,17 +135,17 @@ __device__ __forceinline__ uint2 add_bf16x4(uint2 r, uint2 o) {
   return make_uint2(out[0], out[1]);
 }
 
-template <int kEpi>
+template <int kEpi, bool kFar>
 __global__ __launch_bounds__(kLinThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void linear_kernel(const LinParams p) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wf = wave & 3, wt = wave >> 2;
+  const int wn = wave & 3, wm = wave >> 2;  // token quarter, feature half
   float* s_bias = reinterpret_cast<float*>(smem + kLinBiasOff);
   const uint16_t* s_gelu = reinterpret_cast<const uint16_t*>(smem + kLinGeluOff);
   // Bias (and the GELU table) in LDS: a global load at a tile's start would
-  // complete only behind the loads already in flight for the next stage.
+  // complete only behind the loads already in flight for the next stages.
   for (int e = tid; e < p.N; e += kLinThreads) s_bias[e] = p.bias != nullptr ? p.bias[e] : 0.f;
   if constexpr (kEpi == kEpiGelu) gelu_table_fill(reinterpret_cast<uint16_t*>(smem + kLinGeluOff), tid, kLinThreads);
   __syncthreads();
@@ -149,168 +164,317 @@ void linear_kernel(const LinParams p) {
     f0 = (s - tq * p.tiles_n) * kLinF;
     return tb < p.tiles_m;
   };
+  int m0, f0;
+  if (!tile_of(0, m0, f0)) return;  // uniform
 
-  // One stream of stages over all of this workgroup's tiles (stage g in LDS
-  // buffer g % 2), issued one stage ahead, so the loads run on across tile
-  // boundaries.  A stage is 64 input features: every token row contributes
-  // one whole 128-byte line (a 64-byte half line per request halves what the
-  // L2 delivers), and each feature tile its two adjacent packed blocks.
-  // This thread's part: 1 KB blocks wave + 8q (q < 4) of the weights (tile
-  // blk / 2, k-step 2 st + blk % 2) and of the token rows (rows 8 blk .. + 8,
-  // lane l taking slot l of the block).
+  // One stream of units over all stages of all of this workgroup's tiles.
+  // Unit 4 s + {0: B0, 1: A0, 2: B1, 3: A1} of stage s (LDS buffer s & 1) is
+  // 16 KB, two 1 KB blocks per wave; phase P issues unit P + 8.  A half h:
+  // features 128 wm + 64 h + .., i.e. packed row tiles rt = 8 wm + 4 h + ..;
+  // this wave loads both k-steps of rt = 8 (wave >> 2) + 4 h + (wave & 3).
+  // B half h: token rows 64 wn + 32 h + ..; this wave loads the 8-row blocks
+  // 8 (wave >> 1) + 4 h + 2 (wave & 1) + {0, 1}.
   const uint8_t* xbase = nullptr;  // token row m0 of the issue tile (wave-uniform)
   const uint8_t* wbase = nullptr;  // first packed block of the issue tile's features (wave-uniform)
-  uint32_t xoff[4];
-  int issue_tile = 0, issue_st = 0;
+  uint32_t xoff[2][2];
+  const uint32_t woff = (uint32_t)((tid & 63) ^ (4 * (wave & 1))) * 16u;
+  int issue_tile = 0, issue_st = 0, issue_buf = 0;
   auto set_sources = [&](int t) -> bool {
-    int m0, f0;
-    if (!tile_of(t, m0, f0)) return false;
+    int im, jf;
+    if (!tile_of(t, im, jf)) return false;
     const int lane = lin_lane();
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int row = 8 * (wave + 8 * q) + (lane >> 3);
-      const int c = (lane & 7) ^ lin_swz(row);
-      const int r = m0 + row < p.M ? row : p.M - 1 - m0;  // rows past the end: a valid row, never stored
-      xoff[q] = (uint32_t)r * (uint32_t)p.x_ld + (uint32_t)c * 16u;
-    }
-    xbase = p.x + (int64_t)m0 * p.x_ld;
-    wbase = p.w + (int64_t)(f0 / 16) * ksteps * 1024;
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int row = 8 * (8 * (wave >> 1) + 4 * h + 2 * (wave & 1) + q) + (lane >> 3);
+        const int c = (lane & 7) ^ lin_swz(row);
+        const int r = im + row < p.M ? row : p.M - 1 - im;  // rows past the end: a valid row, never stored
+        xoff[h][q] = (uint32_t)r * (uint32_t)p.x_ld + (uint32_t)c * 16u;
+      }
+    xbase = p.x + (int64_t)im * p.x_ld;
+    wbase = p.w + (int64_t)(jf / 16) * ksteps * 1024;
     return true;
   };
   bool issue_valid = set_sources(0);
-  auto issue_next = [&](int buf) {
-    if (!issue_valid) return;  // uniform: the stream has ended
-    const uint32_t base = lds0 + buf * kLinStage;
-    const uint32_t woff = (uint32_t)lin_lane() * 16u;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int blk = wave + 8 * q;
-      dma_to_lds16_at(wbase + ((int64_t)(blk >> 1) * ksteps + 2 * issue_st + (blk & 1)) * 1024, woff, base + blk * 1024);
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) dma_to_lds16_at(xbase + issue_st * 128, xoff[q], base + kLinWBytes + (wave + 8 * q) * 1024);
+  auto issue_b = [&](int h, int q) {
+    dma_to_lds16_at(xbase + issue_st * 128, xoff[h][q],
+                    lds0 + issue_buf * kLinStage + kLinWBytes + (8 * (wave >> 1) + 4 * h + 2 * (wave & 1) + q) * 1024);
+  };
+  auto issue_a = [&](int h, int q) {
+    const int rt = 8 * (wave >> 2) + 4 * h + (wave & 3);
+    dma_to_lds16_at(wbase + ((int64_t)rt * ksteps + 2 * issue_st + q) * 1024, woff,
+                    lds0 + issue_buf * kLinStage + rt * 2048 + q * 1024);
+  };
+  auto issue_advance = [&]() {  // after the stage's last unit
+    issue_buf ^= 1;
     if (++issue_st == nst) {
       issue_st = 0;
       issue_valid = set_sources(++issue_tile);
     }
   };
 
-  // Fragments of k-step kk of the stage in buffer buf.
-  auto read_frags = [&](int buf, int kk, uint4 (&wfr)[4], uint4 (&xfr)[8]) {
-    const int lane = lin_lane();
-    const int g = lane >> 4, c16 = lane & 15;
-    const uint8_t* stg = smem + buf * kLinStage;
+  // Fragment addresses in buffer 0 (loop-invariant).  Row c16 of A tile i is
+  // feature 32 (i >> 1) + 8 (c16 >> 2) + 4 (i & 1) + (c16 & 3) of the half, so
+  // an accumulator lane g holds 8 consecutive features of a token in tiles
+  // 2 q and 2 q + 1, and the four lanes g 64 contiguous bytes of the output
+  // row.  Packed row tiles of odd index have their 64-byte row groups stored
+  // pairwise swapped (woff), so a fragment's 16 rows hit distinct banks.
+  uint32_t aaddr[2], baddr[2];
+  {
+    const int lane = tid & 63, g = lane >> 4, c16 = lane & 15;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      wfr[i] = *reinterpret_cast<const uint4*>(stg + (2 * (4 * wf + i) + kk) * 1024 + lane * 16);
+    for (int i = 0; i < 2; ++i)
+      aaddr[i] = (8 * wm + (c16 >> 3)) * 2048 +
+                 (16 * g + 8 * ((c16 >> 2) & 1) + 4 * (i ^ (c16 >> 3)) + (c16 & 3)) * 16;
 #pragma unroll
-    for (int jj = 0; jj < 8; ++jj)
-      xfr[jj] = *reinterpret_cast<const uint4*>(stg + kLinWBytes + lin_slot(128 * wt + 16 * jj + c16, 4 * kk + g) * 16);
+    for (int kk = 0; kk < 2; ++kk) baddr[kk] = kLinWBytes + lin_slot(64 * wn + c16, 4 * kk + g) * 16;
+  }
+  auto frag_a = [&](uint32_t bo, int h, int kk, int i) {
+    return *reinterpret_cast<const uint4*>(smem + bo + aaddr[i & 1] + h * 8192 + (i >> 1) * 4096 + kk * 1024);
   };
-  auto mfmas = [&](f32x4 (&acc)[4][8], const uint4 (&wfr)[4], const uint4 (&xfr)[8]) {
-#pragma unroll
-    for (int jj = 0; jj < 8; ++jj)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        acc[i][jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wfr[i]),
-                                                             __builtin_bit_cast(bf16x8, xfr[jj]), acc[i][jj], 0, 0, 0);
+  auto frag_b = [&](uint32_t bo, int h, int kk, int j) {
+    return *reinterpret_cast<const uint4*>(smem + bo + baddr[kk] + (32 * h + 16 * j) * 128);
   };
 
-  // Stage g + 1 is issued right after the barrier that ends the reads of
-  // stage g - 1 (its buffer), so the only loads outstanding at the wait for a
-  // stage are its own (and an epilogue's, which the wait then also covers).
-  issue_next(0);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  f32x4 acc[8][4];
+  auto mma = [&](int ah, int bh, int n, const uint4 (&a)[2][4], const uint4 (&b)[2][2]) {  // n-th of a quadrant's 16
+    const int kk = n >> 3, j = (n >> 2) & 1, i = n & 3;
+    f32x4& c = acc[4 * ah + i][2 * bh + j];
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[kk][i]),
+                                                __builtin_bit_cast(bf16x8, b[kk][j]), c, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // End of phase P: units up to P + 3 have landed (all but the five newest, of
+  // two loads each).  In a tile's first stage the previous tile's kLinStores
+  // output stores (issued by every wave whatever its rows) lie between units
+  // P + 4 and P + 8, so as many more may be open: the stores drain under the
+  // MFMAs instead of being waited for.
+  auto phase_end = [&](bool live, bool after_stores) {
+    if (!live)
+      asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    else if (after_stores)
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(10 + kLinStores) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(10)\n\ts_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  uint4 a[2][4], bx[2][2], by[2][2];
+  int buf = 0;
+  // One stage: four phases of 16 MFMAs (a quadrant each), with the fragment
+  // reads of the next phase and one unit's loads between them, in program
+  // order.  A fragment is reloaded right after its last use: a[kk][i] after
+  // MFMA 8 kk + 4 + i, b[kk][j] after MFMA 8 kk + 4 j + 3.  Fragments read in
+  // one phase are waited for by the next phase's MFMAs, so a unit's place is
+  // free from the phase after that on (B0's, read by MFMA 0 of the phase
+  // before, from the next one on: lgkmcnt(4) leaves only the four newest A
+  // reads open there).  On entry b0 holds B0; on exit b1 holds the next
+  // stage's B0 and a its A0.
+  auto stage = [&](uint4 (&b0)[2][2], uint4 (&b1)[2][2], bool after_stores) {
+    const bool live = issue_valid;  // uniform
+    const uint32_t cur = buf * kLinStage, nxt = cur ^ kLinStage;
+#pragma unroll
+    for (int n = 0; n < 16; ++n) {  // A0 B0; reads B1
+      mma(0, 0, n, a, b0);
+      if (n < 4) b1[n >> 1][n & 1] = frag_b(cur, 1, n >> 1, n & 1);
+      if ((n == 6 || n == 10) && live) issue_b(0, n == 10);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    phase_end(live, after_stores);
+#pragma unroll
+    for (int n = 0; n < 16; ++n) {  // A0 B1; reads A1
+      mma(0, 1, n, a, b1);
+      if (n & 4) a[n >> 3][n & 3] = frag_a(cur, 1, n >> 3, n & 3);
+      if ((n == 1 || n == 9) && live) issue_a(0, n == 9);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    phase_end(live, after_stores);
+#pragma unroll
+    for (int n = 0; n < 16; ++n) {  // A1 B1; reads the next stage's B0
+      mma(1, 1, n, a, b1);
+      if ((n & 3) == 3 && n < 15) b1[n >> 3][(n >> 2) & 1] = frag_b(nxt, 0, n >> 3, (n >> 2) & 1);
+      if ((n == 5 || n == 9) && live) issue_b(1, n == 9);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    phase_end(live, after_stores);
+#pragma unroll
+    for (int n = 0; n < 16; ++n) {  // A1 B0; reads the next stage's A0 (and the last of its B0)
+      mma(1, 0, n, a, b0);
+      if (n == 0) b1[1][1] = frag_b(nxt, 0, 1, 1);
+      if (n & 4) a[n >> 3][n & 3] = frag_a(nxt, 0, n >> 3, n & 3);
+      if ((n == 2 || n == 9) && live) issue_a(1, n == 9);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (live) issue_advance();
+    asm volatile("s_waitcnt lgkmcnt(4)" ::: "memory");
+    phase_end(live, after_stores);
+    buf ^= 1;
+  };
+  // Units 0 .. 7; unit 8 takes unit 0's place only once every wave has read it.
+  auto issue_stage = [&]() {
+    if (!issue_valid) return;  // uniform
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) issue_b(h, q);
+#pragma unroll
+      for (int q = 0; q < 2; ++q) issue_a(h, q);
+    }
+    issue_advance();
+  };
+  issue_stage();
+  const bool second = issue_valid;
+  issue_stage();
+  phase_end(second, false);
+#pragma unroll
+  for (int n = 0; n < 8; ++n) a[n >> 2][n & 3] = frag_a(0, 0, n >> 2, n & 3);
+#pragma unroll
+  for (int n = 0; n < 4; ++n) bx[n >> 1][n & 1] = frag_b(0, 0, n >> 1, n & 1);
   lds_barrier();
-  issue_next(1);
-  uint4 wa[4], xa[8], wb[4], xb[8];  // fragments of k-steps 2 st (a) and 2 st + 1 (b)
-  read_frags(0, 0, wa, xa);
-  int sg = 0;  // stream index of the stage being computed
   for (int t = 0;; ++t) {
-    int m0, f0;
-    if (!tile_of(t, m0, f0)) break;  // uniform
-    int m1, f1;
-    const bool next_tile = tile_of(t + 1, m1, f1);
-    f32x4 acc[4][8];
     {
       const int g = lin_lane() >> 4;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const f32x4 b = *reinterpret_cast<const f32x4*>(s_bias + f0 + 64 * wf + 16 * i + 4 * g);
+      for (int i = 0; i < 8; ++i) {
+        const f32x4 bv = *reinterpret_cast<const f32x4*>(s_bias + f0 + 128 * wm + 32 * (i >> 1) + 8 * g + 4 * (i & 1));
 #pragma unroll
-        for (int jj = 0; jj < 8; ++jj) acc[i][jj] = b;
+        for (int j = 0; j < 4; ++j) acc[i][j] = bv;
       }
     }
-    for (int st = 0; st < nst; ++st, ++sg) {
-      read_frags(sg & 1, 1, wb, xb);
-      mfmas(acc, wa, xa);
-      if (st + 1 < nst || next_tile) {  // uniform: stage sg + 1 exists
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        lds_barrier();  // stage sg + 1 is in LDS; every wave has read stage sg out
-        issue_next(sg & 1);
-        read_frags((sg + 1) & 1, 0, wa, xa);
-      }
-      mfmas(acc, wb, xb);
+    for (int st = 0; st + 1 < nst; st += 2) {
+      stage(bx, by, !kFar && st == 0 && t > 0);
+      stage(by, bx, false);
+    }
+    if (nst & 1) {  // uniform
+      stage(bx, by, !kFar && nst == 1 && t > 0);
+#pragma unroll
+      for (int n = 0; n < 4; ++n) bx[n >> 1][n & 1] = by[n >> 1][n & 1];
     }
     const int lane = lin_lane();
     const int g = lane >> 4, c16 = lane & 15;
 
-    // Epilogue: lane (c16, g) of tile (i, jj) holds features f0 + 64 wf +
-    // 16 i + 4 g .. + 3 of token row m0 + 128 wt + 16 jj + c16.
+    // Epilogue: lane (c16, g) of tiles (2 q + i, j), i < 2, holds the 8
+    // features f0 + 128 wm + 32 q + 8 g .. of token row m0 + 64 wn + 16 j + c16:
+    // 16 bytes at byte offset off[j] + 64 q of the output.  Through a
+    // descriptor, rows past the end and frame padding take an offset outside
+    // it: their loads give 0, their stores are dropped, and every wave issues
+    // kLinStores stores.  Outputs of more bytes than a descriptor covers
+    // (kFar) go through 64-bit addresses under a predicate.
+    uint2 o[4][8];
 #pragma unroll
-    for (int jj = 0; jj < 8; ++jj) {
-      uint2 o[4];
+    for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = make_uint2(pack_bf16x2(acc[i][jj][0], acc[i][jj][1]),
-                                                    pack_bf16x2(acc[i][jj][2], acc[i][jj][3]));
+      for (int i = 0; i < 8; ++i)
+        o[j][i] = make_uint2(pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3]));
+    __builtin_amdgcn_sched_barrier(0);  // the fp32 accumulators end here
+    constexpr bool kScatter = kEpi == kEpiScatter;
+    constexpr bool kRes = kEpi == kEpiResidual || kScatter;
+    const int64_t tile0 = kScatter ? 0 : (int64_t)m0 * p.y_ld;
+    const int left = p.M - m0 < kLinT ? p.M - m0 : kLinT;
+    const uint32_t span = kScatter ? (uint32_t)p.y_bytes : (uint32_t)((left - 1) * p.y_ld + p.N * 2);
+    const __amdgpu_buffer_rsrc_t yr = buffer_rsrc(p.y + tile0, span);
+    const __amdgpu_buffer_rsrc_t rr = buffer_rsrc(p.res + tile0, span);
+    using Off = std::conditional_t<kFar, int64_t, uint32_t>;
+    Off off[4];
+    bool ok[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int row = 64 * wn + 16 * j + c16;
+      int64_t orow = row;
+      ok[j] = row < left;
+      if constexpr (kScatter) {
+        orow = ok[j] ? lin_grid_row(p, m0 + row) : -1;
+        ok[j] = orow >= 0;  // frame padding
+      }
+      const uint32_t col = (uint32_t)(f0 + 128 * wm + 8 * g) * 2u;
+      if constexpr (kFar)
+        off[j] = orow * p.y_ld + col;
+      else
+        off[j] = (ok[j] ? (uint32_t)(orow * p.y_ld) : kLinDrop) + col;
+    }
+    if constexpr (kRes) {
+      // Every residual load before the first store (a later load would wait
+      // for the stores ahead of it), in two batches for the registers' sake.
+#pragma unroll
+      for (int jb = 0; jb < 4; jb += 2) {
+        u32x4 r[2][4];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            if constexpr (kFar) {
+              r[j][q] = u32x4{0, 0, 0, 0};
+              if (ok[jb + j]) {
+                const uint2* src = reinterpret_cast<const uint2*>(p.res + tile0 + off[jb + j] + 64 * q);
+                r[j][q] = u32x4{src[0].x, src[0].y, src[1].x, src[1].y};
+              }
+            } else {
+              r[j][q] = __builtin_amdgcn_raw_buffer_load_b128(rr, off[jb + j] + 64 * q, 0, 0);
+            }
+          }
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            uint2(&v)[8] = o[jb + j];
+            v[2 * q] = add_bf16x4(make_uint2(r[j][q][0], r[j][q][1]), v[2 * q]);
+            v[2 * q + 1] = add_bf16x4(make_uint2(r[j][q][2], r[j][q][3]), v[2 * q + 1]);
+          }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
       if constexpr (kEpi == kEpiGelu) {
-        // Table lookups; a wave holding a value outside the table (|x| < 2^-22
-        // or >= 32) redoes the row exactly.
-        u16x2 dmax = {0, 0};
-        uint2 gv[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          asm volatile("" : "+v"(o[i].x), "+v"(o[i].y));
-          gv[i].x = gelu_pair_table(o[i].x, s_gelu, dmax);
-          gv[i].y = gelu_pair_table(o[i].y, s_gelu, dmax);
-        }
-        const uint32_t dm = dmax.x > dmax.y ? dmax.x : dmax.y;
-        if (__builtin_amdgcn_ballot_w64(dm >= (uint32_t)kGeluSpan) != 0) {
+        for (int ah = 0; ah < 2; ++ah) {
+          // Table lookups; a wave holding a value outside the table (|x| < 2^-22
+          // or >= 32) redoes the values exactly.
+          u16x2 dmax = {0, 0};
+          uint2 gv[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            gv[i].x = gelu_bf16(o[i].x & 0xffffu, s_gelu) | (gelu_bf16(o[i].x >> 16, s_gelu) << 16);
-            gv[i].y = gelu_bf16(o[i].y & 0xffffu, s_gelu) | (gelu_bf16(o[i].y >> 16, s_gelu) << 16);
+            uint2& v = o[j][4 * ah + i];
+            asm volatile("" : "+v"(v.x), "+v"(v.y));
+            gv[i].x = gelu_pair_table(v.x, s_gelu, dmax);
+            gv[i].y = gelu_pair_table(v.y, s_gelu, dmax);
           }
+          const uint32_t dm = dmax.x > dmax.y ? dmax.x : dmax.y;
+          if (__builtin_amdgcn_ballot_w64(dm >= (uint32_t)kGeluSpan) != 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const uint2 v = o[j][4 * ah + i];
+              gv[i].x = gelu_bf16(v.x & 0xffffu, s_gelu) | (gelu_bf16(v.x >> 16, s_gelu) << 16);
+              gv[i].y = gelu_bf16(v.y & 0xffffu, s_gelu) | (gelu_bf16(v.y >> 16, s_gelu) << 16);
+            }
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[j][4 * ah + i] = gv[i];
         }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = gv[i];
-      }
-      const int m = m0 + 128 * wt + 16 * jj + c16;
-      if (m >= p.M) continue;
-      int64_t orow = m;
-      if constexpr (kEpi == kEpiScatter) {
-        orow = lin_grid_row(p, m);
-        if (orow < 0) continue;  // frame padding
-      }
-      uint8_t* yr = p.y + orow * p.y_ld + (f0 + 64 * wf + 4 * g) * 2;
-      if constexpr (kEpi == kEpiResidual || kEpi == kEpiScatter) {
-        const uint8_t* rr = p.res + orow * p.y_ld + (f0 + 64 * wf + 4 * g) * 2;
-        uint2 r[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) r[i] = *reinterpret_cast<const uint2*>(rr + 32 * i);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = add_bf16x4(r[i], o[i]);
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) *reinterpret_cast<uint2*>(yr + 32 * i) = o[i];
+      for (int q = 0; q < 4; ++q) {
+        const int d = 64 * q;
+        const uint2 lo = o[j][2 * q], hi = o[j][2 * q + 1];
+        if constexpr (kFar) {
+          if (ok[j]) {
+            uint2* dst = reinterpret_cast<uint2*>(p.y + tile0 + off[j] + d);
+            dst[0] = lo;
+            dst[1] = hi;
+          }
+        } else {
+          __builtin_amdgcn_raw_buffer_store_b128(u32x4{lo.x, lo.y, hi.x, hi.y}, yr, off[j] + d, 0, kCacheNt);
+        }
+      }
     }
+    if (!tile_of(t + 1, m0, f0)) break;  // uniform
   }
 }
 
-template <int kEpi>
+template <int kEpi, bool kFar>
 int launch_linear(const LinParams& p, hipStream_t s) {
   constexpr int lds = kEpi == kEpiGelu ? kLinGeluOff + kGeluBytes : kLinGeluOff;
-  auto kern = linear_kernel<kEpi>;
+  auto kern = linear_kernel<kEpi, kFar>;
   static const hipError_t attr =
       hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (attr != hipSuccess) return fail(TERRA_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(attr));
@@ -331,6 +495,18 @@ int launch_linear(const LinParams& p, hipStream_t s) {
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(TERRA_ERR_LAUNCH, "linear kernel launch failed: %s", hipGetErrorString(e));
   return TERRA_OK;
+}
+
+// Outputs whose tiles (scatter: the whole grid) a buffer descriptor covers take
+// the descriptor form: all but grids of 4 GiB and more, or row strides of 16
+// MiB and more (a residual's rows are contiguous, so never those).
+template <int kEpi>
+int dispatch_linear(const LinParams& p, hipStream_t s) {
+  if constexpr (kEpi != kEpiResidual) {
+    const int64_t bytes = kEpi == kEpiScatter ? p.y_bytes : (int64_t)kLinT * p.y_ld;
+    if (bytes >= (int64_t)kLinDrop) return launch_linear<kEpi, true>(p, s);
+  }
+  return launch_linear<kEpi, false>(p, s);
 }
 
 bool lin_overlap(const void* a, int64_t abytes, const void* b, int64_t bbytes) {
@@ -395,7 +571,7 @@ extern "C" int terra_swin_linear(const void* x, void* y, int dtype, int64_t rows
   if (rows > 0 && lin_overlap(x, xb, y, yb)) return fail(TERRA_ERR_SHAPE, "y overlaps x");
   if (rows == 0) return TERRA_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return epilogue == TERRA_LINEAR_GELU ? launch_linear<kEpiGelu>(p, s) : launch_linear<kEpiStore>(p, s);
+  return epilogue == TERRA_LINEAR_GELU ? dispatch_linear<kEpiGelu>(p, s) : dispatch_linear<kEpiStore>(p, s);
 }
 
 extern "C" int terra_swin_linear_residual(const void* x, const void* residual, void* y, int dtype, int64_t rows,
@@ -438,5 +614,6 @@ extern "C" int terra_swin_linear_residual(const void* x, const void* residual, v
     return fail(TERRA_ERR_SHAPE, "y overlaps residual without being residual");
   if (rows == 0) return TERRA_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return geom != nullptr ? launch_linear<kEpiScatter>(p, s) : launch_linear<kEpiResidual>(p, s);
+  p.y_bytes = yb;
+  return geom != nullptr ? dispatch_linear<kEpiScatter>(p, s) : dispatch_linear<kEpiResidual>(p, s);
 }

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from oracle import swin_oracle as so
+from terra_amd import _lib as L
 from terra_amd import kernels, workloads
 from terra_amd.kernels import WindowGeometry
 
@@ -165,6 +166,56 @@ def test_linear_scatter_matches_proj_then_reverse(dev, shape):
     assert (d.norm() / want.float().norm()).item() < 4e-3
     y = (want.float() - x.float())
     assert ((got.float() - x.float() - y).norm() / y.norm()).item() < 2e-2
+
+
+@pytest.mark.parametrize("k", [64, 128, 192, 320])
+def test_linear_many_tiles_per_workgroup(dev, k):
+    """1028 tiles over 256 workgroups: the load stream runs across tile
+    boundaries with 1, 2, 3 and 5 stages per tile (odd counts swap the token
+    fragment registers), past output stores still in flight, into a last tile
+    of 77 rows; against the same rows computed as one small call each."""
+    rows, n = 256 * 513 + 77, 512
+    x = torch.randn(rows, k, device=dev, dtype=torch.bfloat16, generator=torch.Generator(dev).manual_seed(30))
+    w, b = _weights(n, k, 31)
+    pk, bd = kernels.pack_linear(w.to(dev)), b.to(dev)
+    got = kernels.linear(x, pk, n, bd)
+    ref = x.double() @ w.to(dev).double().t() + bd.double()
+    # one fp32 sum of k products in another order: within a bf16 step of the exact sum's rounding
+    assert ((got.double() - ref).abs() <= ref.abs() * 2.0 ** -7 + 1e-5).all()
+    for r0 in (0, 256 * 255, rows - 333):
+        assert torch.equal(got[r0:r0 + 333], kernels.linear(x[r0:r0 + 333].contiguous(), pk, n, bd))
+    r = torch.randn(rows, n, device=dev, dtype=torch.bfloat16, generator=torch.Generator(dev).manual_seed(32))
+    assert torch.equal(kernels.linear_residual(x, pk, n, r, bd), r + got)
+
+
+def test_linear_row_stride_past_the_descriptor(dev):
+    """A 16.8 MB output row stride: 256 rows span more than a buffer
+    descriptor, so the 64-bit store form runs; the same values as contiguous."""
+    rows, k, n, stride = 300, 64, 256, (1 << 23) + 8
+    x = workloads.activations((rows, k), 33).to(torch.bfloat16).to(dev)
+    w, b = _weights(n, k, 34)
+    pk, bd = kernels.pack_linear(w.to(dev)), b.to(dev)
+    y = torch.empty((rows - 1) * stride + n, dtype=torch.bfloat16, device=dev)
+    for gelu in (0, 1):
+        st = L.load().terra_swin_linear(x.data_ptr(), y.data_ptr(), L.DTYPE_BF16, rows, k, n, k, stride,
+                                        pk.data_ptr(), bd.data_ptr(), gelu, None)
+        torch.cuda.synchronize()
+        assert st == 0, L.last_error()
+        assert torch.equal(y.as_strided((rows, n), (stride, 1)), kernels.linear(x, pk, n, bd, gelu=bool(gelu)))
+
+
+def test_linear_scatter_grid_past_the_descriptor(dev):
+    """A grid of 4.3 GB (2904 x 2904 tokens of 256 channels): the 64-bit
+    addresses of the scatter, bit for bit the reverse kernel's (W = I)."""
+    H = W = 2904
+    C = 256
+    geom = WindowGeometry(1, H, W, C, 8, 4, 4)
+    g = torch.Generator(dev).manual_seed(35)
+    win = torch.randn(geom.num_windows, 64, C, device=dev, dtype=torch.bfloat16, generator=g)
+    r = torch.randn(1, H, W, C, device=dev, dtype=torch.bfloat16, generator=g)
+    eye = torch.eye(C, dtype=torch.bfloat16, device=dev)
+    got = kernels.linear_residual(win, kernels.pack_linear(eye), C, r, None, geom=geom)
+    assert torch.equal(got, kernels.swin_reverse(win, geom, residual=r))
 
 
 def test_linear_empty_rows(dev):
