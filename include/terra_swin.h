@@ -465,6 +465,40 @@ int terra_swin_linear_residual(const void* x, const void* residual, void* y,
                                const void* weight_packed, const float* bias,
                                const terra_swin_geom* geom, void* stream);
 
+/* terra_swin_pack_linear of a weight that still has to be cast or transposed
+ * (the training step's linear layers): packs P [out_features, in_features]
+ * (multiples of 16 and 32), P = weight (row-major [out, in]) or, transposed
+ * != 0, P = weight^T (row-major [in, out]); weight_dtype bf16, or f32 rounded
+ * once to bf16 (autocast's cast of the Linear's weight).
+ */
+int terra_swin_pack_weight(const void* weight, void* packed, int weight_dtype, int transposed,
+                           int out_features, int in_features, void* stream);
+
+/* terra_swin_linear with TERRA_LINEAR_GELU that also writes the layer's own
+ * output, for a training step whose backward needs both (contiguous rows):
+ *   h[m] = bf16(x[m] W^T + b),  y[m] = GELU(h[m])
+ * Replaces  self.fc1(x); self.act(x)        models/mlp.py:162-165
+ */
+int terra_swin_linear_gelu_keep(const void* x, void* h, void* y, int dtype, int64_t rows,
+                                int in_features, int out_features,
+                                const void* weight_packed, const float* bias, void* stream);
+
+/* The gradient of fc1's output in one kernel (contiguous rows):
+ *   dh[m] = bf16((dy[m] W^T) * slope(h[m])),  slope(h) = Phi(h) + h phi(h)
+ * with dy the gradient of fc2's output [rows, in_features], W^T the packed
+ * transpose of fc2's weight (P [out_features, in_features] = fc2.weight^T:
+ * terra_swin_pack_weight with transposed), h fc1's output [rows,
+ * out_features]; the product stays in fp32 until the one rounding.  When
+ * column_sums is not NULL each column's sum of the dh written is ADDED into it
+ * (fp32 [out_features], float atomics): fc1's bias gradient.  Sizes as
+ * terra_swin_linear.  dh must not overlap dy or h.
+ * Replaces the autograd backward of self.act and of the input of self.fc2
+ *           models/mlp.py:162-168
+ */
+int terra_swin_linear_gelu_bwd(const void* dy, const void* h, void* dh, int dtype, int64_t rows,
+                               int in_features, int out_features,
+                               const void* weight_packed, float* column_sums, void* stream);
+
 /* Backward of the MLP half's activation in the training step
  * (core/runtime/run_model.py:362-617): for rows x features tensors
  *   dh = dout * (Phi(h) + h phi(h)),

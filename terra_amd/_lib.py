@@ -62,6 +62,9 @@ EXPORTED_SYMBOLS = (
     "terra_swin_gelu_bwd",
     "terra_swin_linear",
     "terra_swin_linear_residual",
+    "terra_swin_linear_gelu_keep",
+    "terra_swin_linear_gelu_bwd",
+    "terra_swin_pack_weight",
 )
 
 
@@ -235,6 +238,14 @@ def load() -> ctypes.CDLL:
         lib.terra_swin_linear_residual.restype = ctypes.c_int
         lib.terra_swin_linear_residual.argtypes = [vp, vp, vp, ctypes.c_int, i64, ctypes.c_int, ctypes.c_int, vp, vp,
                                                    ctypes.POINTER(SwinGeom), vp]
+        lib.terra_swin_pack_weight.restype = ctypes.c_int
+        lib.terra_swin_pack_weight.argtypes = [vp, vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp]
+        lib.terra_swin_linear_gelu_keep.restype = ctypes.c_int
+        lib.terra_swin_linear_gelu_keep.argtypes = [vp, vp, vp, ctypes.c_int, i64, ctypes.c_int, ctypes.c_int, vp, vp,
+                                                    vp]
+        lib.terra_swin_linear_gelu_bwd.restype = ctypes.c_int
+        lib.terra_swin_linear_gelu_bwd.argtypes = [vp, vp, vp, ctypes.c_int, i64, ctypes.c_int, ctypes.c_int, vp, vp,
+                                                   vp]
         version = lib.terra_abi_version()
         if version != ABI_VERSION:
             raise RuntimeError(f"terra_amd: {LIB_PATH} has ABI version {version}, expected {ABI_VERSION}; rebuild it")

@@ -192,7 +192,7 @@ class _Linear(torch.autograd.Function):
         dy2 = dy.reshape(-1, dy.shape[-1]).to(wc.dtype)
         dx = dw = db = None
         if ctx.needs_input_grad[0]:
-            dx = (dy2 @ wc).view(xc.shape).to(xd)
+            dx = _input_grad(dy2, wc).view(xc.shape).to(xd)
         if ctx.needs_input_grad[1]:
             dw = weight_grad(dy2, xc.reshape(-1, xc.shape[-1])).to(wd)
         sums = None
@@ -213,16 +213,46 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
     return torch.nn.functional.linear(x, weight, bias)
 
 
+def _bf16_linears(x: torch.Tensor, *params: torch.Tensor) -> bool:
+    """Whether F.linear of bf16 rows like x with these parameters is a bf16
+    product: under bf16 autocast, or with bf16 parameters and no autocast."""
+    if torch.is_autocast_enabled(x.device.type):
+        return kernels.autocast_bf16(x)
+    return all(p.dtype == torch.bfloat16 for p in params)
+
+
+def _linear_kernel(x: torch.Tensor, out_features: int) -> bool:
+    """The token-row linear kernels serve and fill the chip with rows like x."""
+    return (x.is_contiguous() and kernels.linear_supported(x, x.shape[-1], out_features)
+            and kernels.linear_fills(x.numel() // x.shape[-1], out_features))
+
+
+def _input_grad(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """dy @ weight for dy [T, out] in the GEMMs' dtype and a Linear's weight
+    [out, in] of any dtype: on the linear kernel where it serves the shape
+    (156672 rows, 4096 -> 1024: 980-1060 us against 1130-1240 for the
+    library's product with an untransposed weight)."""
+    if _linear_kernel(dy, weight.shape[1]):
+        return kernels.linear(dy, kernels.pack_weight(weight, transpose=True), weight.shape[1])
+    return dy @ weight.to(dy.dtype)
+
+
 class _Mlp(torch.autograd.Function):
     """SequentialMlp.forward (models/mlp.py:152-172) for training:
     y = x + fc2(GELU(fc1(LayerNorm(x)))).  The LayerNorm forward and its
     backward (with the residual gradient added in the same kernel) run on
-    terra_swin_partition_ln / _bwd over the token rows; the four GEMMs of
-    the backward on hipBLASLt through torch, in the dtypes autocast gave the
-    forward's GEMMs.  The GELU derivative (the exact, erf one) runs on
-    terra_swin_gelu_bwd with fc1's bias gradient summed in the same pass;
-    under autocast the output gradient's cast to bf16 sums fc2's bias
-    gradient in its pass (terra_swin_partition_mixed over the token rows)."""
+    terra_swin_partition_ln / _bwd over the token rows.  With bf16 GEMMs that
+    fill the chip, fc1 and the GELU are one linear kernel that keeps fc1's
+    output (156672 rows, C = 1024: 1576 us against 1673 for the library's
+    product and torch's GELU; 524288 rows, C = 192: 503 against 631), a bf16
+    residual is added in fc2's, and in the backward the product with fc2's
+    weight, the GELU derivative and fc1's bias gradient are one
+    (1446 against 1972 us; 451 against 778).  Smaller or other shapes run the
+    products on hipBLASLt through torch, in the dtypes autocast gave them, and
+    the exact (erf) GELU derivative on terra_swin_gelu_bwd with fc1's bias
+    gradient summed in the same pass.  Under autocast the output gradient's
+    cast to bf16 sums fc2's bias gradient in its pass
+    (terra_swin_partition_mixed over the token rows)."""
 
     @staticmethod
     def forward(ctx, x, ln_w, ln_b, w1, b1, w2, b2, eps):
@@ -233,17 +263,24 @@ class _Mlp(torch.autograd.Function):
         # output: the kernel writes that copy directly.
         xn = kernels.swin_partition_ln(rows.view(1, -1, 1, C), geom, ln_w, ln_b, eps,
                                        out_dtype=linear_input_dtype(rows)).view(-1, C)
-        h1 = torch.nn.functional.linear(xn, w1, b1)
-        a = torch.nn.functional.gelu(h1)
-        h2 = torch.nn.functional.linear(a, w2, b2)
-        if h2.dtype == torch.bfloat16 and rows.dtype == torch.float32 and C % 4 == 0 and h2.shape[-1] == C:
-            # x + fc2(...) under autocast: the bf16 h2 widened and added to the
-            # fp32 rows in one pass (the mixed scatter over an identity frame;
-            # bit for bit torch's promoted add).
-            y = kernels.swin_reverse(h2.contiguous(), geom, residual=rows.view(1, -1, 1, C),
-                                     out_dtype=torch.float32).view(rows.shape)
+        y = None
+        if _bf16_linears(xn, w1, b1, w2, b2) and _linear_kernel(xn, w1.shape[0]):
+            h1, a = kernels.linear_gelu_keep(xn, kernels.pack_weight(w1), w1.shape[0], b1.float())
+            if rows.dtype == torch.bfloat16 and w2.shape[0] == C and _linear_kernel(a, C):
+                y = kernels.linear_residual(a, kernels.pack_weight(w2), C, rows, b2.float())
         else:
-            y = rows + h2
+            h1 = torch.nn.functional.linear(xn, w1, b1)
+            a = torch.nn.functional.gelu(h1)
+        if y is None:
+            h2 = torch.nn.functional.linear(a, w2, b2)
+            if h2.dtype == torch.bfloat16 and rows.dtype == torch.float32 and C % 4 == 0 and h2.shape[-1] == C:
+                # x + fc2(...) under autocast: the bf16 h2 widened and added to the
+                # fp32 rows in one pass (the mixed scatter over an identity frame;
+                # bit for bit torch's promoted add).
+                y = kernels.swin_reverse(h2.contiguous(), geom, residual=rows.view(1, -1, 1, C),
+                                         out_dtype=torch.float32).view(rows.shape)
+            else:
+                y = rows + h2
         ctx.eps, ctx.geom, ctx.shape = eps, geom, x.shape
         ctx.autocast = torch.is_autocast_enabled(x.device.type)
         ctx.save_for_backward(rows, ln_w, ln_b, xn, h1, a, w1, w2)
@@ -267,19 +304,26 @@ class _Mlp(torch.autograd.Function):
         else:
             dh2 = dy.to(gemm_dtype)
             db2 = dh2.sum(0, dtype=torch.float32) if ctx.needs_input_grad[6] else None
-        w2c, w1c = w2.to(gemm_dtype), w1.to(gemm_dtype)
-        da = dh2 @ w2c
         dw2 = weight_grad(dh2, a.to(gemm_dtype)) if ctx.needs_input_grad[5] else None
         db1 = None
-        if kernels.gelu_backward_supported(h1):
-            # The GELU derivative and fc1's bias gradient in one pass.
+        dh2 = dh2.contiguous()
+        if _linear_kernel(dh2, h1.shape[-1]):
+            # fc2's input gradient, the GELU derivative and fc1's bias gradient in one kernel.
             if ctx.needs_input_grad[4]:
                 db1 = torch.zeros(h1.shape[-1], dtype=torch.float32, device=h1.device)
-            dh1 = kernels.gelu_backward(da.contiguous(), h1.contiguous(), column_sums=db1)
+            dh1 = kernels.linear_gelu_backward(dh2, kernels.pack_weight(w2, transpose=True), h1.shape[-1], h1,
+                                               column_sums=db1)
         else:
-            dh1 = torch.ops.aten.gelu_backward(da, h1)
-            db1 = dh1.sum(0, dtype=torch.float32) if ctx.needs_input_grad[4] else None
-        dxn = dh1 @ w1c
+            da = dh2 @ w2.to(gemm_dtype)
+            if kernels.gelu_backward_supported(h1):
+                # The GELU derivative and fc1's bias gradient in one pass.
+                if ctx.needs_input_grad[4]:
+                    db1 = torch.zeros(h1.shape[-1], dtype=torch.float32, device=h1.device)
+                dh1 = kernels.gelu_backward(da.contiguous(), h1.contiguous(), column_sums=db1)
+            else:
+                dh1 = torch.ops.aten.gelu_backward(da, h1)
+                db1 = dh1.sum(0, dtype=torch.float32) if ctx.needs_input_grad[4] else None
+        dxn = _input_grad(dh1, w1)
         dw1 = weight_grad(dh1, xn.to(gemm_dtype)) if ctx.needs_input_grad[3] else None
         dlw = torch.zeros(C, dtype=torch.float32, device=rows.device) if (
             ln_w is not None and ctx.needs_input_grad[1]) else None

@@ -61,5 +61,15 @@ __device__ __forceinline__ uint32_t gelu_bf16(uint32_t b, const uint16_t* table)
   return mag < kGeluLo ? half : (mag < kGeluHi ? tab : big);
 }
 
+// d/dh GELU(h) in fp32 (the erf form's exact derivative, before the
+// multiplication by the incoming gradient).
+__device__ __forceinline__ float gelu_slope(float h) {
+  constexpr float kAlpha = 0.70710678118654752f;  // 1 / sqrt(2)
+  constexpr float kBeta = 0.39894228040143268f;   // 1 / sqrt(2 pi)
+  const float cdf = 0.5f * (1.f + erff(h * kAlpha));
+  const float pdf = expf(-0.5f * h * h) * kBeta;
+  return cdf + h * pdf;
+}
+
 }  // namespace
 }  // namespace terra

@@ -12,6 +12,11 @@
 //             reverse + inverse roll + shortcut: row m of window-order x goes
 //             back to the grid token t(m) it was gathered from; frame-padding
 //             rows are dropped)
+//   gelu-keep h[m]    = bf16(acc), y[m] = GELU(h[m])           (fc1 + nn.GELU
+//             of the training step, whose backward needs both)
+//   gelu-bwd  y[m]    = bf16(acc * slope(h[m])), colsum += sum_m y[m]   (the
+//             gradient of fc1's output: fc2's input-gradient product times the
+//             GELU's derivative, and fc1's bias gradient)
 //
 // so that the activation, the residual add and the permutation back to the
 // grid ride on the GEMM's output instead of making their own HBM passes.
@@ -73,13 +78,62 @@ constexpr int kLinBiasOff = kLinStages * kLinStage;
 constexpr int kLinGeluOff = kLinBiasOff + kLinMaxN * 4;
 static_assert(kLinGeluOff + kGeluBytes <= 160 * 1024, "LDS");
 
-enum { kEpiStore = 0, kEpiGelu = 1, kEpiResidual = 2, kEpiScatter = 3 };
+// LDS of each epilogue past the stages: bias (or, gelu-bwd, the column sums),
+// then the GELU or slope table.
+enum { kEpiStore = 0, kEpiGelu = 1, kEpiResidual = 2, kEpiScatter = 3, kEpiGeluKeep = 4, kEpiGeluBwd = 5 };
+
+// The GELU's slope Phi(h) + h phi(h) of a bf16 h: an fp32 table for 2^-13 <=
+// |h| < 8 filled with gelu_slope; from 8 on the last entries (1, and -8e-14 for
+// negative h) stand for the limits 1 and 0 to fp32 rounding; below 2^-13 the
+// slope is 1/2 + 2 phi(0) h to fp32 rounding (the next term is below 2^-40).
+// +-inf and NaN give NaN (inf * 0).  16 KB: with the stages and the column
+// sums exactly the 160 KB of a CU.
+constexpr uint32_t kSlopeTabLo = 0x3900;  // bf16 bits of 2^-13
+constexpr uint32_t kSlopeTabHi = 0x4100;  // bf16 bits of 8
+constexpr int kSlopeTabSpan = (int)(kSlopeTabHi - kSlopeTabLo);
+constexpr int kSlopeTabBytes = 2 * kSlopeTabSpan * 4;
+static_assert(kLinGeluOff + kSlopeTabBytes <= 160 * 1024, "LDS");
+
+template <int kEpi>
+constexpr int lin_lds_bytes() {
+  return kLinGeluOff + (kEpi == kEpiGeluBwd ? kSlopeTabBytes : (kEpi == kEpiGelu || kEpi == kEpiGeluKeep) ? kGeluBytes : 0);
+}
+
+__device__ __forceinline__ float slope_exact(uint32_t b) {
+  const uint32_t mag = b & 0x7fffu;
+  const float h = __uint_as_float(b << 16);
+  if (mag >= 0x7f80u) return __uint_as_float(0x7fc00000u);
+  if (mag < kSlopeTabLo) return fmaf(0.79788456080286536f, h, 0.5f);
+  return mag >= kSlopeTabHi ? (b >> 15 ? 0.f : 1.f) : gelu_slope(h);
+}
+
+// Byte offsets into the slope table of the two bf16 values of `p`; `dmax`
+// collects mag - kSlopeTabLo per half (wrapping below it): from kSlopeRare on
+// a value is tiny, infinite or NaN and its lookup is wrong.
+constexpr uint32_t kSlopeRare = 0x7f80u - kSlopeTabLo;
+__device__ __forceinline__ void slope_pair(uint32_t p, const uint8_t* table, u16x2& dmax, float& lo, float& hi) {
+  const u16x2 v = __builtin_bit_cast(u16x2, p);
+  const u16x2 d = (v & (u16x2)0x7fff) - (u16x2)(uint16_t)kSlopeTabLo;
+  dmax = __builtin_elementwise_max(dmax, d);
+  const u16x2 off = (__builtin_elementwise_min(d, (u16x2)(uint16_t)(kSlopeTabSpan - 1)) +
+                     (v >> 15) * (u16x2)(uint16_t)kSlopeTabSpan) << 2;  // < 2^14
+  lo = *reinterpret_cast<const float*>(table + off.x);
+  hi = *reinterpret_cast<const float*>(table + off.y);
+}
+
+// Sum over the 16 aligned lanes of a row (every lane ends with it).
+__device__ __forceinline__ float row16_sum(float v) {
+  v = group8_sum(v);
+  return v + dpp_move<0x128>(v);  // row_ror:8
+}
 
 struct LinParams {
   const uint8_t* x;       // [M rows] x K bf16, row stride x_ld bytes
   const uint8_t* w;       // packed [N, K] bf16
   const float* bias;      // [N] or NULL
-  const uint8_t* res;     // residual (kEpiResidual / kEpiScatter), row stride y_ld
+  const uint8_t* res;     // residual (kEpiResidual / kEpiScatter) or h (kEpiGeluBwd), row stride y_ld
+  uint8_t* keep;          // kEpiGeluKeep: h, row stride y_ld
+  float* colsum;          // kEpiGeluBwd: [N] or NULL
   uint8_t* y;             // output rows, row stride y_ld bytes
   int64_t x_ld, y_ld;
   int64_t y_bytes;        // kEpiScatter: bytes of y (and res)
@@ -147,7 +201,15 @@ void linear_kernel(const LinParams p) {
   // Bias (and the GELU table) in LDS: a global load at a tile's start would
   // complete only behind the loads already in flight for the next stages.
   for (int e = tid; e < p.N; e += kLinThreads) s_bias[e] = p.bias != nullptr ? p.bias[e] : 0.f;
-  if constexpr (kEpi == kEpiGelu) gelu_table_fill(reinterpret_cast<uint16_t*>(smem + kLinGeluOff), tid, kLinThreads);
+  if constexpr (kEpi == kEpiGelu || kEpi == kEpiGeluKeep)
+    gelu_table_fill(reinterpret_cast<uint16_t*>(smem + kLinGeluOff), tid, kLinThreads);
+  if constexpr (kEpi == kEpiGeluBwd) {  // s_bias holds the column sums
+    float* table = reinterpret_cast<float*>(smem + kLinGeluOff);
+    for (int e = tid; e < 2 * kSlopeTabSpan; e += kLinThreads) {
+      const uint32_t bits = e < kSlopeTabSpan ? kSlopeTabLo + e : 0x8000u + kSlopeTabLo + (e - kSlopeTabSpan);
+      table[e] = gelu_slope(__uint_as_float(bits << 16));
+    }
+  }
   __syncthreads();
   const int xcd = (int)blockIdx.x & 7;
   const int nx = ((int)gridDim.x - xcd + 7) >> 3;  // workgroups with this blockIdx % 8
@@ -254,7 +316,7 @@ void linear_kernel(const LinParams p) {
     if (!live)
       asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
     else if (after_stores)
-      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(10 + kLinStores) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(10 + (kEpi == kEpiGeluKeep ? 2 : 1) * kLinStores) : "memory");
     else
       asm volatile("s_waitcnt vmcnt(10)\n\ts_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
@@ -336,7 +398,7 @@ void linear_kernel(const LinParams p) {
       const int g = lin_lane() >> 4;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const f32x4 bv = *reinterpret_cast<const f32x4*>(s_bias + f0 + 128 * wm + 32 * (i >> 1) + 8 * g + 4 * (i & 1));
+        const f32x4 bv = kEpi == kEpiGeluBwd ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(s_bias + f0 + 128 * wm + 32 * (i >> 1) + 8 * g + 4 * (i & 1));
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = bv;
       }
@@ -361,12 +423,14 @@ void linear_kernel(const LinParams p) {
     // kLinStores stores.  Outputs of more bytes than a descriptor covers
     // (kFar) go through 64-bit addresses under a predicate.
     uint2 o[4][8];
+    if constexpr (kEpi != kEpiGeluBwd) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        o[j][i] = make_uint2(pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3]));
-    __builtin_amdgcn_sched_barrier(0);  // the fp32 accumulators end here
+        for (int i = 0; i < 8; ++i)
+          o[j][i] = make_uint2(pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3]));
+      __builtin_amdgcn_sched_barrier(0);  // the fp32 accumulators end here
+    }
     constexpr bool kScatter = kEpi == kEpiScatter;
     constexpr bool kRes = kEpi == kEpiResidual || kScatter;
     const int64_t tile0 = kScatter ? 0 : (int64_t)m0 * p.y_ld;
@@ -423,9 +487,72 @@ void linear_kernel(const LinParams p) {
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    if constexpr (kEpi == kEpiGeluBwd) {
+      const uint8_t* s_slope = smem + kLinGeluOff;
+      // Two of the four 32-feature groups q at a time: their h, their products
+      // and column sums; every load before the first store.
+#pragma unroll
+      for (int qb = 0; qb < 4; qb += 2) {
+        u32x4 h[2][4];
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) h[q][j] = __builtin_amdgcn_raw_buffer_load_b128(rr, off[j] + 64 * (qb + q), 0, 0);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            float sl[8];
+            u16x2 dmax = {0, 0};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) slope_pair(h[q][j][e], s_slope, dmax, sl[2 * e], sl[2 * e + 1]);
+            const uint32_t dm = dmax.x > dmax.y ? dmax.x : dmax.y;
+            if (__builtin_amdgcn_ballot_w64(dm >= kSlopeRare) != 0) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                sl[2 * e] = slope_exact(h[q][j][e] & 0xffffu);
+                sl[2 * e + 1] = slope_exact(h[q][j][e] >> 16);
+              }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const f32x4& c = acc[2 * (qb + q) + (e >> 1)][j];
+              const uint32_t v = pack_bf16x2(c[2 * (e & 1)] * sl[2 * e], c[2 * (e & 1) + 1] * sl[2 * e + 1]);
+              uint2& d = o[j][2 * (qb + q) + (e >> 1)];
+              if (e & 1)
+                d.y = v;
+              else
+                d.x = v;
+              // the values as written; rows past the end add nothing (their h is 0, but their products are not)
+              if (ok[j]) {
+                sum[2 * e] += __uint_as_float(v << 16);
+                sum[2 * e + 1] += __uint_as_float(v & 0xffff0000u);
+              }
+            }
+          }
+          if (p.colsum != nullptr) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sum[e] = row16_sum(sum[e]);
+            if (c16 == 0) {
+#pragma unroll
+              for (int e = 0; e < 8; ++e) atomicAdd(&s_bias[f0 + 128 * wm + 32 * (qb + q) + 8 * g + e], sum[e]);
+            }
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      if constexpr (kEpi == kEpiGelu) {
+      if constexpr (kEpi == kEpiGeluKeep) {
+        const __amdgpu_buffer_rsrc_t kr = buffer_rsrc(p.keep + tile0, span);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          __builtin_amdgcn_raw_buffer_store_b128(
+              u32x4{o[j][2 * q].x, o[j][2 * q].y, o[j][2 * q + 1].x, o[j][2 * q + 1].y}, kr, off[j] + 64 * q, 0, kCacheNt);
+      }
+      if constexpr (kEpi == kEpiGelu || kEpi == kEpiGeluKeep) {
 #pragma unroll
         for (int ah = 0; ah < 2; ++ah) {
           // Table lookups; a wave holding a value outside the table (|x| < 2^-22
@@ -469,11 +596,17 @@ void linear_kernel(const LinParams p) {
     }
     if (!tile_of(t + 1, m0, f0)) break;  // uniform
   }
+  if constexpr (kEpi == kEpiGeluBwd) {
+    lds_barrier();  // every wave's column sums are in
+    if (p.colsum != nullptr)
+      for (int e = tid; e < p.N; e += kLinThreads)
+        if (s_bias[e] != 0.f) unsafeAtomicAdd(p.colsum + e, s_bias[e]);
+  }
 }
 
 template <int kEpi, bool kFar>
 int launch_linear(const LinParams& p, hipStream_t s) {
-  constexpr int lds = kEpi == kEpiGelu ? kLinGeluOff + kGeluBytes : kLinGeluOff;
+  constexpr int lds = lin_lds_bytes<kEpi>();
   auto kern = linear_kernel<kEpi, kFar>;
   static const hipError_t attr =
       hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -499,10 +632,10 @@ int launch_linear(const LinParams& p, hipStream_t s) {
 
 // Outputs whose tiles (scatter: the whole grid) a buffer descriptor covers take
 // the descriptor form: all but grids of 4 GiB and more, or row strides of 16
-// MiB and more (a residual's rows are contiguous, so never those).
+// MiB and more (the other epilogues' rows are contiguous, so never those).
 template <int kEpi>
 int dispatch_linear(const LinParams& p, hipStream_t s) {
-  if constexpr (kEpi != kEpiResidual) {
+  if constexpr (kEpi == kEpiStore || kEpi == kEpiGelu || kEpi == kEpiScatter) {
     const int64_t bytes = kEpi == kEpiScatter ? p.y_bytes : (int64_t)kLinT * p.y_ld;
     if (bytes >= (int64_t)kLinDrop) return launch_linear<kEpi, true>(p, s);
   }
@@ -616,4 +749,42 @@ extern "C" int terra_swin_linear_residual(const void* x, const void* residual, v
   hipStream_t s = static_cast<hipStream_t>(stream);
   p.y_bytes = yb;
   return geom != nullptr ? dispatch_linear<kEpiScatter>(p, s) : dispatch_linear<kEpiResidual>(p, s);
+}
+
+extern "C" int terra_swin_linear_gelu_keep(const void* x, void* h, void* y, int dtype, int64_t rows, int in_features,
+                                           int out_features, const void* weight_packed, const float* bias,
+                                           void* stream) {
+  clear_error();
+  LinParams p{};
+  const int st = lin_validate(x, weight_packed, bias, y, dtype, rows, in_features, out_features, in_features,
+                              out_features, &p);
+  if (st != TERRA_OK) return st;
+  if (h == nullptr) return fail(TERRA_ERR_NULL, "h must be non-NULL");
+  if (((uintptr_t)h & 7u) != 0) return fail(TERRA_ERR_ALIGN, "h must be 8-byte aligned");
+  const int64_t xb = rows * (int64_t)in_features * 2, yb = rows * (int64_t)out_features * 2;
+  if (rows > 0 && (lin_overlap(x, xb, y, yb) || lin_overlap(x, xb, h, yb) || lin_overlap(h, yb, y, yb)))
+    return fail(TERRA_ERR_SHAPE, "x, h and y must not overlap");
+  p.keep = static_cast<uint8_t*>(h);
+  if (rows == 0) return TERRA_OK;
+  return dispatch_linear<kEpiGeluKeep>(p, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int terra_swin_linear_gelu_bwd(const void* dy, const void* h, void* dh, int dtype, int64_t rows,
+                                          int in_features, int out_features, const void* weight_packed,
+                                          float* column_sums, void* stream) {
+  clear_error();
+  LinParams p{};
+  const int st = lin_validate(dy, weight_packed, nullptr, dh, dtype, rows, in_features, out_features, in_features,
+                              out_features, &p);
+  if (st != TERRA_OK) return st;
+  if (h == nullptr) return fail(TERRA_ERR_NULL, "h must be non-NULL");
+  if (((uintptr_t)h & 7u) != 0 || ((uintptr_t)column_sums & 3u) != 0)
+    return fail(TERRA_ERR_ALIGN, "h must be 8-byte and column_sums 4-byte aligned");
+  const int64_t xb = rows * (int64_t)in_features * 2, yb = rows * (int64_t)out_features * 2;
+  if (rows > 0 && (lin_overlap(dy, xb, dh, yb) || lin_overlap(h, yb, dh, yb)))
+    return fail(TERRA_ERR_SHAPE, "dh must not overlap dy or h");
+  p.res = static_cast<const uint8_t*>(h);
+  p.colsum = column_sums;
+  if (rows == 0) return TERRA_OK;
+  return dispatch_linear<kEpiGeluBwd>(p, static_cast<hipStream_t>(stream));
 }

@@ -9,6 +9,7 @@
 // activation dtype, and optionally  colsum[f] += sum_t dh[t, f]  over the
 // rounded values (fc1's bias gradient, models/mlp.py:162).
 #include "common.h"
+#include "gelu.h"
 
 namespace terra {
 namespace {
@@ -23,16 +24,6 @@ constexpr int kGeluMaxChunks = 512;  // 16-byte chunks per row: bf16 F <= 4096, 
 // each input per lane.
 template <int CPL>
 constexpr int gelu_rows() { return CPL >= 8 ? 1 : 8 / CPL; }
-
-// d/dh GELU(h) in fp32 (the erf form's exact derivative, before the
-// multiplication by the incoming gradient).
-__device__ __forceinline__ float gelu_slope(float h) {
-  constexpr float kAlpha = 0.70710678118654752f;  // 1 / sqrt(2)
-  constexpr float kBeta = 0.39894228040143268f;   // 1 / sqrt(2 pi)
-  const float cdf = 0.5f * (1.f + erff(h * kAlpha));
-  const float pdf = expf(-0.5f * h * h) * kBeta;
-  return cdf + h * pdf;
-}
 
 // The slope of a bf16 input by table.  fc1's output is rounded to bf16
 // before the activation, so the slope takes one of 2^16 values; for

@@ -2062,6 +2062,38 @@ __global__ __launch_bounds__(256) void pack_linear_kernel(const uint4* __restric
   packed[i] = w[(uint64_t)row * (uint32_t)k_chunks + col_chunk];
 }
 
+// The same order of the bf16 matrix P [rows, 8 k_chunks] with P = W or, kTrans,
+// P = W^T of a row-major W (bf16 or fp32, rounded once): the training step's
+// cast, transpose and packing of a weight in one pass.  Both directions read
+// whole 32- or 64-byte segments: 8 consecutive values of a row, or (kTrans)
+// the 16 lanes of a row tile consecutive values of each of 8 rows.
+template <typename T, bool kTrans>
+__global__ __launch_bounds__(256) void pack_weight_kernel(const T* __restrict__ w, uint4* __restrict__ packed,
+                                                          uint32_t chunks, int rows, int k_chunks) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= chunks) return;
+  const uint32_t lane = i & 63u, blk = i >> 6;
+  const uint32_t ksteps = (uint32_t)k_chunks / 4u;
+  const uint32_t rt = blk / ksteps, ks = blk - rt * ksteps;
+  const uint32_t row = 16u * rt + (lane & 15u), col = 8u * (4u * ks + (lane >> 4));
+  uint32_t out[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    uint32_t h[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const uint64_t c = col + 2 * q + e;
+      const T v = kTrans ? w[c * (uint32_t)rows + row] : w[(uint64_t)row * (8u * (uint32_t)k_chunks) + c];
+      if constexpr (sizeof(T) == 4)
+        h[e] = f32_to_bf16_bits(v);
+      else
+        h[e] = v;
+    }
+    out[q] = h[0] | (h[1] << 16);
+  }
+  packed[i] = make_uint4(out[0], out[1], out[2], out[3]);
+}
+
 bool ranges_overlap(const void* a, const void* b, int64_t bytes) {
   const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
   return x < y + (uintptr_t)bytes && y < x + (uintptr_t)bytes;
@@ -2196,6 +2228,45 @@ extern "C" int terra_swin_pack_linear(const void* weight, void* packed, int dtyp
   const uint32_t chunks = (uint32_t)(bytes / 16);
   pack_linear_kernel<<<(chunks + 255) / 256, 256, 0, static_cast<hipStream_t>(stream)>>>(
       static_cast<const uint4*>(weight), static_cast<uint4*>(packed), chunks, in_features / 8);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(TERRA_ERR_LAUNCH, "pack launch failed: %s", hipGetErrorString(e));
+  return TERRA_OK;
+}
+
+extern "C" int terra_swin_pack_weight(const void* weight, void* packed, int weight_dtype, int transposed,
+                                      int out_features, int in_features, void* stream) {
+  clear_error();
+  if (weight == nullptr || packed == nullptr) return fail(TERRA_ERR_NULL, "weight and packed must be non-NULL");
+  if (dtype_size(weight_dtype) == 0) return fail(TERRA_ERR_DTYPE, "unknown dtype %d", weight_dtype);
+  if (weight_dtype != TERRA_DTYPE_BF16 && weight_dtype != TERRA_DTYPE_F32)
+    return fail(TERRA_ERR_UNSUPPORTED, "weights are packed from bf16 or fp32");
+  if (out_features <= 0 || in_features <= 0 || out_features % 16 != 0 || in_features % 32 != 0)
+    return fail(TERRA_ERR_SHAPE, "packed weight [%d, %d] must be a multiple of [16, 32]", out_features, in_features);
+  if ((((uintptr_t)weight) & 15u) != 0 || (((uintptr_t)packed) & 15u) != 0)
+    return fail(TERRA_ERR_ALIGN, "weight and packed must be 16-byte aligned");
+  const int64_t bytes = (int64_t)out_features * in_features * 2;
+  if (bytes / 16 >= (1ll << 31)) return fail(TERRA_ERR_SHAPE, "weight too large");
+  const int64_t wbytes = bytes / 2 * dtype_size(weight_dtype);
+  const uintptr_t a = (uintptr_t)weight, b = (uintptr_t)packed;
+  if (a < b + (uintptr_t)bytes && b < a + (uintptr_t)wbytes) return fail(TERRA_ERR_SHAPE, "packed overlaps weight");
+  const uint32_t chunks = (uint32_t)(bytes / 16);
+  const dim3 grid((chunks + 255) / 256);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  uint4* out = static_cast<uint4*>(packed);
+  const int kc = in_features / 8;
+  if (weight_dtype == TERRA_DTYPE_F32) {
+    const float* w = static_cast<const float*>(weight);
+    if (transposed)
+      pack_weight_kernel<float, true><<<grid, 256, 0, s>>>(w, out, chunks, out_features, kc);
+    else
+      pack_weight_kernel<float, false><<<grid, 256, 0, s>>>(w, out, chunks, out_features, kc);
+  } else {
+    const uint16_t* w = static_cast<const uint16_t*>(weight);
+    if (transposed)
+      pack_weight_kernel<uint16_t, true><<<grid, 256, 0, s>>>(w, out, chunks, out_features, kc);
+    else
+      pack_weight_kernel<uint16_t, false><<<grid, 256, 0, s>>>(w, out, chunks, out_features, kc);
+  }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(TERRA_ERR_LAUNCH, "pack launch failed: %s", hipGetErrorString(e));
   return TERRA_OK;

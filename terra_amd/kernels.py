@@ -784,6 +784,13 @@ def linear_supported(x: torch.Tensor, in_features: int, out_features: int) -> bo
             and 0 < out_features <= LINEAR_MAX_OUT and out_features % LINEAR_OUT_MULTIPLE == 0)
 
 
+def linear_fills(rows: int, out_features: int) -> bool:
+    """Whether a linear-kernel launch has a 256 x 256 tile for each of the 256
+    compute units.  Below that the library's smaller tiles keep more of the
+    chip busy; at and above it the fused epilogues pay."""
+    return -(-rows // 256) * (out_features // LINEAR_OUT_MULTIPLE) >= 256
+
+
 def _linear_checks(x: torch.Tensor, weight_packed: torch.Tensor, out_features: int, bias: Optional[torch.Tensor]):
     dev = _require_device(x, weight_packed)
     code = _dtype_code(x, (torch.bfloat16,))
@@ -864,6 +871,66 @@ def linear_residual(x: torch.Tensor, weight_packed: torch.Tensor, out_features: 
                                                     None if c_geom is None else ctypes.byref(c_geom), _stream(dev))
     _lib.check(st, "terra_swin_linear_residual")
     return out.view(shape)
+
+
+def pack_weight(weight: torch.Tensor, transpose: bool = False) -> torch.Tensor:
+    """:func:`pack_linear` of a bf16 or fp32 weight [out, in] (rounded once to
+    bf16) or, with ``transpose``, of its transpose (the weight of the
+    input-gradient product), in one pass (terra_swin_pack_weight)."""
+    dev = _require_device(weight)
+    code = _dtype_code(weight, (torch.bfloat16, torch.float32))
+    if weight.dim() != 2:
+        raise ValueError("weight must be a 2-D tensor")
+    weight = weight.detach().contiguous()
+    n, k = (weight.shape[1], weight.shape[0]) if transpose else weight.shape
+    out = torch.empty(n * k, dtype=torch.bfloat16, device=dev)
+    with torch.cuda.device(dev):
+        st = _lib.load().terra_swin_pack_weight(_ptr(weight), _ptr(out), code, int(bool(transpose)), int(n), int(k),
+                                                _stream(dev))
+    _lib.check(st, "terra_swin_pack_weight")
+    return out
+
+
+def linear_gelu_keep(x: torch.Tensor, weight_packed: torch.Tensor, out_features: int,
+                     bias: Optional[torch.Tensor] = None):
+    """``h = bf16(x W^T + b)`` and ``GELU(h)`` over the token rows of ``x``
+    [rows, in] in one kernel (:func:`linear` with ``gelu`` that keeps its
+    pre-activation for the backward); returns (h, GELU(h))."""
+    dev, code, k, rows = _linear_checks(x, weight_packed, out_features, bias)
+    shape = (*x.shape[:-1], out_features)
+    h = torch.empty(shape, dtype=x.dtype, device=dev)
+    y = torch.empty(shape, dtype=x.dtype, device=dev)
+    if rows:
+        with torch.cuda.device(dev):
+            st = _lib.load().terra_swin_linear_gelu_keep(_ptr(x), _ptr(h), _ptr(y), code, int(rows), int(k),
+                                                         int(out_features), _ptr(weight_packed), _ptr(bias),
+                                                         _stream(dev))
+        _lib.check(st, "terra_swin_linear_gelu_keep")
+    return h, y
+
+
+def linear_gelu_backward(dy: torch.Tensor, weight_packed: torch.Tensor, out_features: int, h: torch.Tensor,
+                         column_sums: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``bf16((dy W^T) * (Phi(h) + h phi(h)))``: the gradient of fc1's output
+    ``h`` [rows, out_features] from the gradient ``dy`` [rows, in] of fc2's
+    output, ``weight_packed`` being ``pack_weight(fc2.weight, transpose=True)``.
+    ``column_sums``: an fp32 [out_features] tensor the result's column sums
+    (fc1's bias gradient) are ADDED into."""
+    dev, code, k, rows = _linear_checks(dy, weight_packed, out_features, None)
+    _require_device(dy, h)
+    if h.dtype != dy.dtype or tuple(h.shape) != (*dy.shape[:-1], out_features) or not h.is_contiguous():
+        raise ValueError(f"h must be a contiguous {dy.dtype} tensor of shape {(*dy.shape[:-1], out_features)}")
+    if column_sums is not None and (column_sums.dtype != torch.float32 or not column_sums.is_contiguous()
+                                    or tuple(column_sums.shape) != (out_features,) or column_sums.device != dev):
+        raise ValueError(f"column_sums must be a contiguous fp32 [{out_features}] tensor on {dev}")
+    dh = torch.empty_like(h)
+    if rows:
+        with torch.cuda.device(dev):
+            st = _lib.load().terra_swin_linear_gelu_bwd(_ptr(dy), _ptr(h), _ptr(dh), code, int(rows), int(k),
+                                                        int(out_features), _ptr(weight_packed), _ptr(column_sums),
+                                                        _stream(dev))
+        _lib.check(st, "terra_swin_linear_gelu_bwd")
+    return dh
 
 
 def gelu_backward_supported(h: torch.Tensor) -> bool:

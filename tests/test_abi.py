@@ -457,3 +457,27 @@ def test_linear_residual_rejects_bad_arguments():
     assert _lin_res_call(rows=5 * 64, geom=full) == -3 and "window tokens" in L.last_error()
     other_c = kernels.WindowGeometry(1, 16, 24, 768, 8).to_c()
     assert _lin_res_call(rows=6 * 64, geom=other_c) == -3 and "out_features" in L.last_error()
+
+
+def test_training_linear_entries_reject_bad_arguments():
+    lib = L.load()
+    p = lambda a: ctypes.c_void_p(a << 28)  # noqa: E731
+
+    def keep(x=p(1), h=p(2), y=p(3), dtype=L.DTYPE_BF16, rows=512, k=192, n=768, w=p(5)):
+        return lib.terra_swin_linear_gelu_keep(x, h, y, dtype, rows, k, n, w, None, None)
+
+    def bwd(dy=p(1), h=p(2), dh=p(3), dtype=L.DTYPE_BF16, rows=512, k=192, n=768, w=p(5), s=None):
+        return lib.terra_swin_linear_gelu_bwd(dy, h, dh, dtype, rows, k, n, w, s, None)
+
+    def pack(w=p(1), out=p(2), dtype=L.DTYPE_F32, n=768, k=192):
+        return lib.terra_swin_pack_weight(w, out, dtype, 1, n, k, None)
+
+    for call in (keep, bwd):
+        assert call(h=None) == -1 and call(w=None) == -1
+        assert call(dtype=L.DTYPE_F32) == -5 and call(k=96) == -3 and call(n=192) == -3 and call(rows=-1) == -3
+        assert call(h=ctypes.c_void_p((2 << 28) + 4)) == -4
+        assert call(rows=0) == 0
+    assert keep(h=p(3)) == -3 and keep(y=p(1)) == -3 and "overlap" in L.last_error()
+    assert bwd(dh=p(2)) == -3 and bwd(dh=p(1)) == -3 and bwd(s=ctypes.c_void_p((6 << 28) + 2)) == -4
+    assert pack(w=None) == -1 and pack(dtype=L.DTYPE_F16) == -5 and pack(n=24) == -3 and pack(k=48) == -3
+    assert pack(out=ctypes.c_void_p((2 << 28) + 8)) == -4 and pack(out=p(1)) == -3

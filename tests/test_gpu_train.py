@@ -466,3 +466,104 @@ def test_block_autocast_training_sums_biases_in_kernels(dev):
     bound = dqkv.shape[0] * 2.0 ** -24 * dqkv.double().abs().sum(0).cpu() + 1e-30
     got = torch.cat([blk.attn.q_linear.bias.grad, blk.attn.k_linear.bias.grad, blk.attn.v_linear.bias.grad])
     assert ((got.double().cpu() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("transpose", [False, True])
+def test_pack_weight_equals_cast_transpose_and_pack(dev, dtype, transpose):
+    for n, k in ((16, 32), (192, 768), (768, 96)):
+        w = workloads.activations((k, n) if transpose else (n, k), 580).to(dtype).to(dev)
+        p = (w.t() if transpose else w).to(torch.bfloat16).contiguous()
+        assert torch.equal(kernels.pack_weight(w, transpose), kernels.pack_linear(p))
+
+
+LINEAR_GELU_SHAPES = [(1, 64, 256), (257, 128, 512), (700, 192, 768), (256 * 260 + 5, 64, 768), (300, 1024, 4096)]
+
+
+@pytest.mark.parametrize("rows,k,n", LINEAR_GELU_SHAPES)
+def test_linear_gelu_keep(dev, rows, k, n):
+    """h is the plain linear kernel's output and y the GELU kernel's, bit for
+    bit (edges of the 256-row tiles, several tiles per workgroup)."""
+    x = torch.randn(rows, k, device=dev, generator=torch.Generator(dev).manual_seed(581)).bfloat16()
+    w = workloads.activations((n, k), 582).to(dev) * k ** -0.5
+    b = workloads.activations((n,), 583).to(dev) * 0.1
+    pk = kernels.pack_weight(w)
+    h, y = kernels.linear_gelu_keep(x, pk, n, b)
+    assert torch.equal(h, kernels.linear(x, pk, n, b))
+    assert torch.equal(y, kernels.linear(x, pk, n, b, gelu=True))
+
+
+@pytest.mark.parametrize("rows,k,n", LINEAR_GELU_SHAPES)
+def test_linear_gelu_backward(dev, rows, k, n):
+    """bf16((dy W2) * slope(h)) against float64: one fp32 sum of k products
+    (k u relative to the sum of their magnitudes), one fp32 slope and one bf16
+    rounding; tiny, large, infinite and NaN h; the column sums against those
+    of the values written, within the fp32 summation bound."""
+    g = torch.Generator(dev).manual_seed(584)
+    dy = torch.randn(rows, k, device=dev, generator=g).bfloat16()
+    h = (torch.randn(rows, n, device=dev, generator=g) * 2).bfloat16()
+    special = torch.tensor([0.0, -0.0, 2.0 ** -13, -(2.0 ** -13), 2.0 ** -14, -(2.0 ** -20), 1e-30, 7.96875, -7.96875,
+                            8.0, -8.0, 31.0, -31.0, 300.0, -300.0], device=dev).bfloat16()
+    h.view(-1)[:special.numel()] = special
+    w2 = workloads.activations((k, n), 585).to(dev) * n ** -0.5
+    sums = torch.ones(n, device=dev)
+    pk = kernels.pack_weight(w2, transpose=True)
+    got = kernels.linear_gelu_backward(dy, pk, n, h, column_sums=sums)
+    wd, hd = w2.bfloat16().double(), h.double()
+    slope = 0.5 * (1 + torch.special.erf(hd / 2 ** 0.5)) + hd * torch.exp(-hd * hd / 2) / (2 * torch.pi) ** 0.5
+    want = (dy.double() @ wd) * slope
+    mag = dy.double().abs() @ wd.abs()  # what the fp32 sum's rounding scales with
+    # the slope in fp32: 2^-22 absolute (erff, expf and their sum); bf16: 2^-8 of the value
+    bound = want.abs() * 2.0 ** -8 + mag * (k * 2.0 ** -24 * slope.abs() + 2.0 ** -22) + 1e-30
+    assert ((got.double() - want).abs() <= bound).all()
+    vals = got.double()
+    assert ((sums.double() - 1 - vals.sum(0)).abs() <= (rows + 8) * 2.0 ** -24 * (vals.abs().sum(0) + 1)).all()
+    assert torch.equal(got, kernels.linear_gelu_backward(dy, pk, n, h))
+    h[0, :3] = torch.tensor([float("inf"), float("-inf"), float("nan")], device=dev).bfloat16()
+    bad = kernels.linear_gelu_backward(dy, pk, n, h)
+    assert bad[0, :3].isnan().all() and not bad[1:].isnan().any() and not bad[0, 3:].isnan().any()
+
+
+@pytest.mark.parametrize("x_dtype,C,tokens", [(torch.float32, 192, 21999), (torch.bfloat16, 1024, 16500)])
+def test_mlp_training_on_linear_kernels(dev, x_dtype, C, tokens):
+    """Rows that fill the chip run fc1 + GELU and the GELU backward on the
+    linear kernels; outputs and gradients against float64 autograd of the
+    bf16-rounded weights, 1e-2 normwise (the products' bf16 operands)."""
+    m = _mlp_case(C, 590)
+    x = workloads.activations((tokens, C), 591).to(x_dtype)
+    gy = workloads.activations((tokens, C), 592).to(x_dtype)
+    md = copy.deepcopy(m).to(dev)
+    calls = {"keep": 0, "bwd": 0}
+    k0, b0 = kernels.linear_gelu_keep, kernels.linear_gelu_backward
+
+    def ck(*a, **k):
+        calls["keep"] += 1
+        return k0(*a, **k)
+
+    def cb(*a, **k):
+        calls["bwd"] += 1
+        return b0(*a, **k)
+
+    kernels.linear_gelu_keep, kernels.linear_gelu_backward = ck, cb
+    try:
+        xd = x.to(dev).requires_grad_(True)
+        with torch.amp.autocast(device_type="cuda", dtype=torch.bfloat16):
+            y = md(xd)
+        y.backward(gy.to(dev))
+    finally:
+        kernels.linear_gelu_keep, kernels.linear_gelu_backward = k0, b0
+    assert calls == {"keep": 1, "bwd": 1} and y.dtype == x_dtype
+    mref = copy.deepcopy(m).to(dev)
+    yr, xg, pg = _oracle_mlp_grads(mref, x.to(dev), gy.to(dev), torch.float64, bf16_weights=True)
+    assert _normwise(y.detach(), yr) <= 1e-2
+    assert _normwise(xd.grad, xg) <= 1e-2
+    for n, p in md.named_parameters():
+        assert _normwise(p.grad, pg[n]) <= 1e-2, n
+
+
+def test_mlp_training_refuses_mixed_dtypes_outside_autocast(dev):
+    """bf16 rows with fp32 parameters and no autocast are refused, as F.linear refuses them, at any size."""
+    m = _mlp_case(192, 595).to(dev)
+    x = workloads.activations((30000, 192), 596).to(torch.bfloat16).to(dev).requires_grad_(True)
+    with pytest.raises(RuntimeError):
+        m(x)
