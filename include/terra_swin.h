@@ -499,6 +499,20 @@ int terra_swin_linear_gelu_bwd(const void* dy, const void* h, void* dh, int dtyp
                                int in_features, int out_features,
                                const void* weight_packed, float* column_sums, void* stream);
 
+/* Weight gradient of a linear layer over token rows (the autograd backward of
+ * an nn.Linear's weight, models/attention.py:223-228, 281, models/mlp.py:162-168):
+ *   dw[o][i] = sum_m dy[m][o] x[m][i]
+ * dy [rows, out_features], x [rows, in_features] contiguous bf16; dw fp32
+ * [out_features, in_features], written (not added to); fp32 sums, in an order
+ * fixed by the sizes.  Feature counts are multiples of 16; rows > 0.
+ * terra_swin_weight_grad_slices gives the number of token slices s (a negative
+ * value is a status); workspace holds s * out_features * in_features fp32
+ * values, overwritten (may be NULL for s = 1).
+ */
+int terra_swin_weight_grad_slices(int64_t rows, int out_features, int in_features);
+int terra_swin_weight_grad(const void* dy, const void* x, float* dw, int dtype, int64_t rows,
+                           int out_features, int in_features, void* workspace, void* stream);
+
 /* Backward of the MLP half's activation in the training step
  * (core/runtime/run_model.py:362-617): for rows x features tensors
  *   dh = dout * (Phi(h) + h phi(h)),

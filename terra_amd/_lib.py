@@ -65,6 +65,8 @@ EXPORTED_SYMBOLS = (
     "terra_swin_linear_gelu_keep",
     "terra_swin_linear_gelu_bwd",
     "terra_swin_pack_weight",
+    "terra_swin_weight_grad",
+    "terra_swin_weight_grad_slices",
 )
 
 
@@ -246,6 +248,10 @@ def load() -> ctypes.CDLL:
         lib.terra_swin_linear_gelu_bwd.restype = ctypes.c_int
         lib.terra_swin_linear_gelu_bwd.argtypes = [vp, vp, vp, ctypes.c_int, i64, ctypes.c_int, ctypes.c_int, vp, vp,
                                                    vp]
+        lib.terra_swin_weight_grad_slices.restype = ctypes.c_int
+        lib.terra_swin_weight_grad_slices.argtypes = [i64, ctypes.c_int, ctypes.c_int]
+        lib.terra_swin_weight_grad.restype = ctypes.c_int
+        lib.terra_swin_weight_grad.argtypes = [vp, vp, vp, ctypes.c_int, i64, ctypes.c_int, ctypes.c_int, vp, vp]
         version = lib.terra_abi_version()
         if version != ABI_VERSION:
             raise RuntimeError(f"terra_amd: {LIB_PATH} has ABI version {version}, expected {ABI_VERSION}; rebuild it")

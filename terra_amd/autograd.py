@@ -150,15 +150,22 @@ def partition_ln(x: torch.Tensor, geom: WindowGeometry, weight: Optional[torch.T
 
 def weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """dy^T x for dy [T, out] and x [T, in] (a Linear's weight gradient, the
-    contraction over all T tokens), in fp32.  For large T the tokens are
-    split into k slices contracted as one batched GEMM with an fp32 output and
-    then summed: hipBLASLt takes no split-K tiles for a contraction this long
-    and runs the plain product 3.5-7.7x slower (c3: 524288 tokens, 1.0-1.6 ms
-    against 0.10-0.25 ms per weight gradient).  Slices of at least 2048
-    tokens, at most 128 of them: at c3, 128 slices of 4096 measured 97-250 us
-    per weight gradient against 115-350 us with 64 and 241-266 us with 256."""
+    contraction over all T tokens), in fp32.  bf16 rows run on the HIP
+    weight-gradient kernel, which cuts the tokens into as many slices as give
+    each compute unit one (output tile, slice) pair and adds them in order
+    (us, against the library's batched product over token slices and its sum:
+    524288 x 768 x 192 213-247 / 251-300, 524288 x 576 x 192 165 / 242,
+    156672 x 4096 x 1024 1097 / 1530, 50176 x 512 x 128 25 / 33; equal at 524288
+    x 192 x 192 and 32768 x 768 x 768).  Other dtypes (and feature counts that
+    are no multiple of 16) take the library: for large T in fp16 k slices
+    contracted as one batched GEMM with an fp32 output and then summed, since
+    hipBLASLt takes no split-K tiles for a contraction this long."""
     T, o = dy.shape
     i = x.shape[1]
+    if dy.dtype == torch.bfloat16:
+        dy, x = dy.contiguous(), x.contiguous()
+        if kernels.weight_grad_supported(dy, x):
+            return kernels.weight_grad(dy, x)
     k = next((k for k in (128, 64, 32, 16, 8) if T % k == 0 and T // k >= 2048), 1)
     if k == 1 or dy.dtype not in (torch.bfloat16, torch.float16):
         return (dy.t() @ x).float()

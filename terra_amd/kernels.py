@@ -933,6 +933,36 @@ def linear_gelu_backward(dy: torch.Tensor, weight_packed: torch.Tensor, out_feat
     return dh
 
 
+def weight_grad_supported(dy: torch.Tensor, x: torch.Tensor) -> bool:
+    """Whether :func:`weight_grad` serves dy [T, out] and x [T, in]: contiguous
+    16-byte aligned bf16 device rows (1 <= T < 2^31), feature counts multiples
+    of 16 up to 2^20."""
+    return (dy.device.type == "cuda" and dy.dtype == x.dtype == torch.bfloat16 and dy.dim() == x.dim() == 2
+            and 0 < dy.shape[0] == x.shape[0] < 2 ** 31 and dy.is_contiguous() and x.is_contiguous()
+            and all(0 < n <= 2 ** 20 and n % 16 == 0 for n in (dy.shape[1], x.shape[1]))
+            and dy.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0)
+
+
+def weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """``dy^T x`` for dy [T, out] and x [T, in] (bf16) in fp32: a Linear's
+    weight gradient over every token row (terra_swin_weight_grad)."""
+    dev = _require_device(dy, x)
+    code = _dtype_code(dy, (torch.bfloat16,))
+    if not weight_grad_supported(dy, x):
+        raise ValueError("weight_grad takes contiguous 16-byte aligned bf16 dy [T, out] and x [T, in] with T > 0 and "
+                         f"feature counts multiples of 16 (got {tuple(dy.shape)} {dy.dtype}, {tuple(x.shape)} {x.dtype})")
+    rows, o, i = dy.shape[0], dy.shape[1], x.shape[1]
+    lib = _lib.load()
+    out = torch.empty((o, i), dtype=torch.float32, device=dev)
+    slices = lib.terra_swin_weight_grad_slices(rows, o, i)
+    work = torch.empty((slices, o, i), dtype=torch.float32, device=dev) if slices > 1 else None
+    with torch.cuda.device(dev):
+        st = lib.terra_swin_weight_grad(_ptr(dy), _ptr(x), _ptr(out), code, int(rows), int(o), int(i), _ptr(work),
+                                        _stream(dev))
+    _lib.check(st, "terra_swin_weight_grad")
+    return out
+
+
 def gelu_backward_supported(h: torch.Tensor) -> bool:
     """Whether :func:`gelu_backward` serves a pre-activation like ``h``
     (a bf16 or fp32 device tensor whose rows are whole 16-byte chunks of at

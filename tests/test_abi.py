@@ -481,3 +481,20 @@ def test_training_linear_entries_reject_bad_arguments():
     assert bwd(dh=p(2)) == -3 and bwd(dh=p(1)) == -3 and bwd(s=ctypes.c_void_p((6 << 28) + 2)) == -4
     assert pack(w=None) == -1 and pack(dtype=L.DTYPE_F16) == -5 and pack(n=24) == -3 and pack(k=48) == -3
     assert pack(out=ctypes.c_void_p((2 << 28) + 8)) == -4 and pack(out=p(1)) == -3
+
+
+def test_weight_grad_rejects_bad_arguments():
+    lib = L.load()
+    p = lambda a: ctypes.c_void_p(a << 28)  # noqa: E731
+
+    def call(dy=p(1), x=p(2), dw=p(3), dtype=L.DTYPE_BF16, rows=4096, o=768, i=192, work=p(4)):
+        return lib.terra_swin_weight_grad(dy, x, dw, dtype, rows, o, i, work, None)
+
+    assert call(dy=None) == -1 and call(x=None) == -1 and call(dw=None) == -1
+    assert call(dtype=L.DTYPE_F32) == -5 and call(dtype=9) == -2
+    assert call(rows=-1) == -3 and call(rows=0) == -3 and call(o=24) == -3 and call(i=0) == -3
+    assert call(x=ctypes.c_void_p((2 << 28) + 8)) == -4
+    assert call(work=None) == -1 and "workspace" in L.last_error()
+    assert lib.terra_swin_weight_grad_slices(4096, 768, 192) == 8
+    assert lib.terra_swin_weight_grad_slices(100, 768, 192) == 1
+    assert lib.terra_swin_weight_grad_slices(4096, 24, 192) < 0

@@ -567,3 +567,37 @@ def test_mlp_training_refuses_mixed_dtypes_outside_autocast(dev):
     x = workloads.activations((30000, 192), 596).to(torch.bfloat16).to(dev).requires_grad_(True)
     with pytest.raises(RuntimeError):
         m(x)
+
+
+# (T, out, in): one token, tails of a 32-token stage, widths that fill and do
+# not fill the 256 / 192 / 128 tiles, fewer and more stages than LDS buffers,
+# slices with a short last one, more tiles than compute units.
+WEIGHT_GRAD_SHAPES = [(1, 16, 16), (31, 32, 48), (100, 256, 256), (161, 128, 512), (513, 192, 768), (4099, 400, 336),
+                      (20000, 576, 192), (70001, 768, 192), (33, 4096, 4352)]
+
+
+@pytest.mark.parametrize("T,o,i", WEIGHT_GRAD_SHAPES)
+def test_weight_grad(dev, T, o, i):
+    """dy^T x against float64: fp32 sums of exact bf16 products, so each entry
+    is within T u of the sum of their magnitudes; the same bits twice; the
+    tokens past the end (neighbouring memory full of NaN) are not read."""
+    g = torch.Generator(dev).manual_seed(600)
+    buf_dy = torch.full((T * o + 40 * o,), float("nan"), device=dev, dtype=torch.bfloat16)
+    buf_x = torch.full((T * i + 40 * i,), float("nan"), device=dev, dtype=torch.bfloat16)
+    dy, x = buf_dy[:T * o].view(T, o), buf_x[:T * i].view(T, i)
+    dy.copy_(torch.randn(T, o, device=dev, generator=g))
+    x.copy_(torch.randn(T, i, device=dev, generator=g))
+    got = kernels.weight_grad(dy, x)
+    want = dy.double().t() @ x.double()
+    mag = dy.double().abs().t() @ x.double().abs()
+    assert got.dtype == torch.float32 and tuple(got.shape) == (o, i)
+    assert ((got.double() - want).abs() <= (T + 1) * 2.0 ** -24 * mag).all()
+    assert torch.equal(got, kernels.weight_grad(dy, x))
+
+
+def test_weight_grad_refuses_other_operands(dev):
+    dy = torch.zeros(64, 32, device=dev, dtype=torch.bfloat16)
+    for bad_dy, bad_x in ((dy.float(), dy.float()), (dy, dy[:32]), (dy.t(), dy.t()), (dy[:0], dy[:0]),
+                          (dy[:, :8].contiguous(), dy)):
+        with pytest.raises((ValueError, TypeError)):
+            kernels.weight_grad(bad_dy, bad_x)
