@@ -499,6 +499,24 @@ int terra_swin_linear_gelu_bwd(const void* dy, const void* h, void* dh, int dtyp
                                int in_features, int out_features,
                                const void* weight_packed, float* column_sums, void* stream);
 
+/* Epilogues of terra_swin_linear_short. */
+enum terra_short_epilogue {
+  TERRA_SHORT_STORE = 0,     /* y = bf16(x W^T + b)                     */
+  TERRA_SHORT_GELU_KEEP = 1  /* keep = bf16(x W^T + b), y = GELU(keep)  */
+};
+
+/* Token-row linear layer of 128 or 192 input features (bf16, contiguous rows),
+ * the training step's narrow layers: out_features a multiple of 128 or 192 up
+ * to 4096, weight_packed as terra_swin_pack_weight, bias fp32 or NULL, keep
+ * non-NULL with its epilogue only.  All tensors 16-byte aligned, outputs
+ * overlapping nothing.
+ * Replaces  the nn.Linear calls of models/attention.py:223-228, 281 and
+ *           models/mlp.py:162-165, and their backward
+ */
+int terra_swin_linear_short(const void* x, void* y, void* keep, int dtype, int64_t rows,
+                            int in_features, int out_features, const void* weight_packed,
+                            const float* bias, int epilogue, void* stream);
+
 /* Weight gradient of a linear layer over token rows (the autograd backward of
  * an nn.Linear's weight, models/attention.py:223-228, 281, models/mlp.py:162-168):
  *   dw[o][i] = sum_m dy[m][o] x[m][i]

@@ -174,29 +174,71 @@ def weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
                      out_dtype=torch.float32).sum(0)
 
 
+def _bf16_linears(x: torch.Tensor, *params: Optional[torch.Tensor]) -> bool:
+    """Whether F.linear of bf16 rows like x with these parameters is a bf16
+    product: under bf16 autocast, or with bf16 parameters and no autocast."""
+    if torch.is_autocast_enabled(x.device.type):
+        return kernels.autocast_bf16(x)
+    return all(p is None or p.dtype == torch.bfloat16 for p in params)
+
+
+def _short_kernel(x: torch.Tensor, out_features: int) -> bool:
+    """The short-row linear kernels serve and fill the chip with rows like x
+    (524288 rows, us, against the library's product: 192 -> 576 130 / 300,
+    192 -> 192 60 / 113; 50176 rows of 128 -> 384 12 / 28)."""
+    return (kernels.linear_short_supported(x, x.shape[-1], out_features)
+            and kernels.linear_short_fills(x.numel() // x.shape[-1], out_features))
+
+
+def _linear_kernel(x: torch.Tensor, out_features: int) -> bool:
+    """The token-row linear kernels serve and fill the chip with rows like x."""
+    return (x.is_contiguous() and kernels.linear_supported(x, x.shape[-1], out_features)
+            and kernels.linear_fills(x.numel() // x.shape[-1], out_features))
+
+
+def _input_grad(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """dy @ weight for dy [T, out] in the GEMMs' dtype and a Linear's weight
+    [out, in] of any dtype: on the linear kernels where they serve the shape
+    (156672 rows, 4096 -> 1024: 980-1060 us against 1130-1240 for the
+    library's product with an untransposed weight)."""
+    if dy.dtype != torch.bfloat16:
+        return dy @ weight.to(dy.dtype)
+    if _short_kernel(dy, weight.shape[1]):
+        return kernels.linear_short(dy, kernels.pack_weight(weight, transpose=True), weight.shape[1])
+    if _linear_kernel(dy, weight.shape[1]):
+        return kernels.linear(dy, kernels.pack_weight(weight, transpose=True), weight.shape[1])
+    return dy @ weight.to(dy.dtype)
+
+
 class _Linear(torch.autograd.Function):
     """F.linear for training, in the dtype bf16 autocast gives it (x, weight
     and bias cast to bf16 inside an autocast region, as F.linear's autocast
-    rule does), with the weight gradient from :func:`weight_grad`.  The bias
-    gradient comes from a :class:`ColumnSumLink` when the output gradient's
-    producer summed it (in the order of its own kernel), else from a sum."""
+    rule does; on the HIP linear kernels the bias stays fp32), with the weight
+    gradient from :func:`weight_grad`.  The bias gradient comes from a
+    :class:`ColumnSumLink` when the output gradient's producer summed it (in
+    the order of its own kernel), else from a sum."""
 
     @staticmethod
     def forward(ctx, x, weight, bias, bias_sums):
         dt = torch.bfloat16 if (torch.is_autocast_enabled(x.device.type)
                                 and torch.get_autocast_dtype(x.device.type) == torch.bfloat16) else x.dtype
         xc, wc = x.to(dt), weight.to(dt)
-        bc = None if bias is None else bias.to(dt)
         ctx.save_for_backward(xc, wc)
         ctx.dtypes = (x.dtype, weight.dtype, None if bias is None else bias.dtype)
         ctx.bias_sums = bias_sums
+        o = weight.shape[0]
+        if (dt == torch.bfloat16 and weight.dim() == 2 and weight.shape[1] == x.shape[-1]
+                and (bias is None or bias.numel() == o) and _bf16_linears(xc, weight, bias) and _short_kernel(xc, o)):
+            return kernels.linear_short(xc, kernels.pack_weight(wc), o, None if bias is None else bias.float())
+        bc = None if bias is None else bias.to(dt)
         return torch.nn.functional.linear(xc, wc, bc)
 
     @staticmethod
     def backward(ctx, dy: torch.Tensor):
         xc, wc = ctx.saved_tensors
         xd, wd, bd = ctx.dtypes
-        dy2 = dy.reshape(-1, dy.shape[-1]).to(wc.dtype)
+        dt = xc.dtype  # the product's dtype
+        dy2 = dy.reshape(-1, dy.shape[-1]).to(dt)
         dx = dw = db = None
         if ctx.needs_input_grad[0]:
             dx = _input_grad(dy2, wc).view(xc.shape).to(xd)
@@ -206,7 +248,7 @@ class _Linear(torch.autograd.Function):
         if ctx.bias_sums is not None:
             sums, ctx.bias_sums.sums = ctx.bias_sums.sums, None
         if bd is not None and ctx.needs_input_grad[2]:
-            db = (sums if sums is not None and dy.dtype == wc.dtype else dy2.sum(0, dtype=torch.float32)).to(bd)
+            db = (sums if sums is not None and dy.dtype == dt else dy2.sum(0, dtype=torch.float32)).to(bd)
         return dx, dw, db, None
 
 
@@ -220,30 +262,6 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
     return torch.nn.functional.linear(x, weight, bias)
 
 
-def _bf16_linears(x: torch.Tensor, *params: torch.Tensor) -> bool:
-    """Whether F.linear of bf16 rows like x with these parameters is a bf16
-    product: under bf16 autocast, or with bf16 parameters and no autocast."""
-    if torch.is_autocast_enabled(x.device.type):
-        return kernels.autocast_bf16(x)
-    return all(p.dtype == torch.bfloat16 for p in params)
-
-
-def _linear_kernel(x: torch.Tensor, out_features: int) -> bool:
-    """The token-row linear kernels serve and fill the chip with rows like x."""
-    return (x.is_contiguous() and kernels.linear_supported(x, x.shape[-1], out_features)
-            and kernels.linear_fills(x.numel() // x.shape[-1], out_features))
-
-
-def _input_grad(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """dy @ weight for dy [T, out] in the GEMMs' dtype and a Linear's weight
-    [out, in] of any dtype: on the linear kernel where it serves the shape
-    (156672 rows, 4096 -> 1024: 980-1060 us against 1130-1240 for the
-    library's product with an untransposed weight)."""
-    if _linear_kernel(dy, weight.shape[1]):
-        return kernels.linear(dy, kernels.pack_weight(weight, transpose=True), weight.shape[1])
-    return dy @ weight.to(dy.dtype)
-
-
 class _Mlp(torch.autograd.Function):
     """SequentialMlp.forward (models/mlp.py:152-172) for training:
     y = x + fc2(GELU(fc1(LayerNorm(x)))).  The LayerNorm forward and its
@@ -251,7 +269,7 @@ class _Mlp(torch.autograd.Function):
     terra_swin_partition_ln / _bwd over the token rows.  With bf16 GEMMs that
     fill the chip, fc1 and the GELU are one linear kernel that keeps fc1's
     output (156672 rows, C = 1024: 1576 us against 1673 for the library's
-    product and torch's GELU; 524288 rows, C = 192: 503 against 631), a bf16
+    product and torch's GELU; 524288 rows, C = 192: 330 against 631), a bf16
     residual is added in fc2's, and in the backward the product with fc2's
     weight, the GELU derivative and fc1's bias gradient are one
     (1446 against 1972 us; 451 against 778).  Smaller or other shapes run the
@@ -271,7 +289,10 @@ class _Mlp(torch.autograd.Function):
         xn = kernels.swin_partition_ln(rows.view(1, -1, 1, C), geom, ln_w, ln_b, eps,
                                        out_dtype=linear_input_dtype(rows)).view(-1, C)
         y = None
-        if _bf16_linears(xn, w1, b1, w2, b2) and _linear_kernel(xn, w1.shape[0]):
+        bf16 = xn.dtype == torch.bfloat16 and _bf16_linears(xn, w1, b1, w2, b2)
+        if bf16 and _short_kernel(xn, w1.shape[0]):
+            h1, a = kernels.linear_short(xn, kernels.pack_weight(w1), w1.shape[0], b1.float(), gelu_keep=True)
+        elif bf16 and _linear_kernel(xn, w1.shape[0]):
             h1, a = kernels.linear_gelu_keep(xn, kernels.pack_weight(w1), w1.shape[0], b1.float())
             if rows.dtype == torch.bfloat16 and w2.shape[0] == C and _linear_kernel(a, C):
                 y = kernels.linear_residual(a, kernels.pack_weight(w2), C, rows, b2.float())

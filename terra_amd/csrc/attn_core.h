@@ -526,6 +526,12 @@ __device__ __forceinline__ void dma_to_lds16_at(const void* sbase, uint32_t voff
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(sbase), "{m0}"(lds_base) : "memory");
 }
 
+// The load through a wave-uniform buffer descriptor: lanes whose byte offset
+// lies outside it write zeros.
+__device__ __forceinline__ void dma_buffer_to_lds16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t lds_base) {
+  asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(voff), "s"(r), "{m0}"(lds_base) : "memory");
+}
+
 // One 4-byte global -> LDS load per lane from a wave-uniform base plus a
 // 32-bit lane offset: lane l writes LDS bytes [lds_base + 4 l, + 4).
 __device__ __forceinline__ void dma_to_lds4_at(const void* sbase, uint32_t voff, uint32_t lds_base) {

@@ -82,6 +82,12 @@ __device__ __forceinline__ float group8_sum(float v) {
   return v + dpp_move<0x141>(v);
 }
 
+// Sum over the 16 aligned lanes of a row (every lane ends with it).
+__device__ __forceinline__ float row16_sum(float v) {
+  v = group8_sum(v);
+  return v + dpp_move<0x128>(v);  // row_ror:8
+}
+
 // ---- streaming stores ------------------------------------------------------
 // Output streams are written through buffer stores carrying the sc1 cache-
 // policy bit.  Measured on MI355X (201 MB arrays, 16-byte accesses):

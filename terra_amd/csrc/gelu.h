@@ -71,5 +71,83 @@ __device__ __forceinline__ float gelu_slope(float h) {
   return cdf + h * pdf;
 }
 
+// The GELU's slope Phi(h) + h phi(h) of a bf16 h: an fp32 table for 2^-13 <=
+// |h| < 8 filled with gelu_slope; from 8 on the last entries (1, and -8e-14 for
+// negative h) stand for the limits 1 and 0 to fp32 rounding; below 2^-13 the
+// slope is 1/2 + 2 phi(0) h to fp32 rounding (the next term is below 2^-40).
+// +-inf and NaN give NaN (inf * 0).  16 KB.
+constexpr uint32_t kSlopeTabLo = 0x3900;  // bf16 bits of 2^-13
+constexpr uint32_t kSlopeTabHi = 0x4100;  // bf16 bits of 8
+constexpr int kSlopeTabSpan = (int)(kSlopeTabHi - kSlopeTabLo);
+constexpr int kSlopeTabBytes = 2 * kSlopeTabSpan * 4;
+
+typedef uint32_t gelu_u32x4 __attribute__((ext_vector_type(4)));
+
+// Slope of any bf16 value (bits b): the table or the closed forms.
+__device__ __forceinline__ float slope_any(uint32_t b, const uint8_t* table) {
+  const uint32_t mag = b & 0x7fffu, sign = b >> 15;
+  const uint32_t d = mag - kSlopeTabLo;  // wraps below kSlopeTabLo
+  const uint32_t idx = (d < (uint32_t)kSlopeTabSpan ? d : (uint32_t)kSlopeTabSpan - 1u) + sign * (uint32_t)kSlopeTabSpan;
+  const float tab = *reinterpret_cast<const float*>(table + 4u * idx);
+  const float small = fmaf(0.79788456080286536f, __uint_as_float(b << 16), 0.5f);
+  return mag >= 0x7f80u ? __uint_as_float(0x7fc00000u) : (mag < kSlopeTabLo ? small : tab);
+}
+
+__device__ __forceinline__ void slope_table_fill(float* table, int tid, int nthreads) {
+  for (int e = tid; e < 2 * kSlopeTabSpan; e += nthreads) {
+    const uint32_t bits = e < kSlopeTabSpan ? kSlopeTabLo + e : 0x8000u + kSlopeTabLo + (e - kSlopeTabSpan);
+    table[e] = gelu_slope(__uint_as_float(bits << 16));
+  }
+}
+
+// Slopes of the two bf16 values of `p` by table; `dmax`
+// collects mag - kSlopeTabLo per half (wrapping below it): from kSlopeRare on
+// a value is tiny, infinite or NaN and its lookup is wrong.
+constexpr uint32_t kSlopeRare = 0x7f80u - kSlopeTabLo;
+__device__ __forceinline__ void slope_pair(uint32_t p, const uint8_t* table, u16x2& dmax, float& lo, float& hi) {
+  const u16x2 v = __builtin_bit_cast(u16x2, p);
+  const u16x2 d = (v & (u16x2)0x7fff) - (u16x2)(uint16_t)kSlopeTabLo;
+  dmax = __builtin_elementwise_max(dmax, d);
+  const u16x2 off = (__builtin_elementwise_min(d, (u16x2)(uint16_t)(kSlopeTabSpan - 1)) +
+                     (v >> 15) * (u16x2)(uint16_t)kSlopeTabSpan) << 2;  // < 2^14
+  lo = *reinterpret_cast<const float*>(table + off.x);
+  hi = *reinterpret_cast<const float*>(table + off.y);
+}
+
+// Slopes of the eight bf16 values of a 16-byte chunk.  A wave holding a value
+// whose lookup is wrong redoes the chunk with the closed forms.
+__device__ __forceinline__ void slope_chunk(gelu_u32x4 h, const uint8_t* table, float (&sl)[8]) {
+  u16x2 dmax = {0, 0};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) slope_pair(h[e], table, dmax, sl[2 * e], sl[2 * e + 1]);
+  const uint32_t dm = dmax.x > dmax.y ? dmax.x : dmax.y;
+  if (__builtin_amdgcn_ballot_w64(dm >= kSlopeRare) != 0) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      sl[2 * e] = slope_any(h[e] & 0xffffu, table);
+      sl[2 * e + 1] = slope_any(h[e] >> 16, table);
+    }
+  }
+}
+
+// GELU of four packed bf16 pairs in place: table lookups; a wave holding a
+// value outside the table (|x| < 2^-22 or >= 32) redoes the chunk exactly.
+__device__ __forceinline__ void gelu_chunk(uint32_t (&v)[4], const uint16_t* table) {
+  u16x2 dmax = {0, 0};
+  uint32_t r[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    asm volatile("" : "+v"(v[e]));
+    r[e] = gelu_pair_table(v[e], table, dmax);
+  }
+  const uint32_t dm = dmax.x > dmax.y ? dmax.x : dmax.y;
+  if (__builtin_amdgcn_ballot_w64(dm >= (uint32_t)kGeluSpan) != 0) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = gelu_bf16(v[e] & 0xffffu, table) | (gelu_bf16(v[e] >> 16, table) << 16);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = r[e];
+}
+
 }  // namespace
 }  // namespace terra

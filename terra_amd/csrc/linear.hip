@@ -82,16 +82,6 @@ static_assert(kLinGeluOff + kGeluBytes <= 160 * 1024, "LDS");
 // then the GELU or slope table.
 enum { kEpiStore = 0, kEpiGelu = 1, kEpiResidual = 2, kEpiScatter = 3, kEpiGeluKeep = 4, kEpiGeluBwd = 5 };
 
-// The GELU's slope Phi(h) + h phi(h) of a bf16 h: an fp32 table for 2^-13 <=
-// |h| < 8 filled with gelu_slope; from 8 on the last entries (1, and -8e-14 for
-// negative h) stand for the limits 1 and 0 to fp32 rounding; below 2^-13 the
-// slope is 1/2 + 2 phi(0) h to fp32 rounding (the next term is below 2^-40).
-// +-inf and NaN give NaN (inf * 0).  16 KB: with the stages and the column
-// sums exactly the 160 KB of a CU.
-constexpr uint32_t kSlopeTabLo = 0x3900;  // bf16 bits of 2^-13
-constexpr uint32_t kSlopeTabHi = 0x4100;  // bf16 bits of 8
-constexpr int kSlopeTabSpan = (int)(kSlopeTabHi - kSlopeTabLo);
-constexpr int kSlopeTabBytes = 2 * kSlopeTabSpan * 4;
 static_assert(kLinGeluOff + kSlopeTabBytes <= 160 * 1024, "LDS");
 
 template <int kEpi>
@@ -99,33 +89,6 @@ constexpr int lin_lds_bytes() {
   return kLinGeluOff + (kEpi == kEpiGeluBwd ? kSlopeTabBytes : (kEpi == kEpiGelu || kEpi == kEpiGeluKeep) ? kGeluBytes : 0);
 }
 
-__device__ __forceinline__ float slope_exact(uint32_t b) {
-  const uint32_t mag = b & 0x7fffu;
-  const float h = __uint_as_float(b << 16);
-  if (mag >= 0x7f80u) return __uint_as_float(0x7fc00000u);
-  if (mag < kSlopeTabLo) return fmaf(0.79788456080286536f, h, 0.5f);
-  return mag >= kSlopeTabHi ? (b >> 15 ? 0.f : 1.f) : gelu_slope(h);
-}
-
-// Byte offsets into the slope table of the two bf16 values of `p`; `dmax`
-// collects mag - kSlopeTabLo per half (wrapping below it): from kSlopeRare on
-// a value is tiny, infinite or NaN and its lookup is wrong.
-constexpr uint32_t kSlopeRare = 0x7f80u - kSlopeTabLo;
-__device__ __forceinline__ void slope_pair(uint32_t p, const uint8_t* table, u16x2& dmax, float& lo, float& hi) {
-  const u16x2 v = __builtin_bit_cast(u16x2, p);
-  const u16x2 d = (v & (u16x2)0x7fff) - (u16x2)(uint16_t)kSlopeTabLo;
-  dmax = __builtin_elementwise_max(dmax, d);
-  const u16x2 off = (__builtin_elementwise_min(d, (u16x2)(uint16_t)(kSlopeTabSpan - 1)) +
-                     (v >> 15) * (u16x2)(uint16_t)kSlopeTabSpan) << 2;  // < 2^14
-  lo = *reinterpret_cast<const float*>(table + off.x);
-  hi = *reinterpret_cast<const float*>(table + off.y);
-}
-
-// Sum over the 16 aligned lanes of a row (every lane ends with it).
-__device__ __forceinline__ float row16_sum(float v) {
-  v = group8_sum(v);
-  return v + dpp_move<0x128>(v);  // row_ror:8
-}
 
 struct LinParams {
   const uint8_t* x;       // [M rows] x K bf16, row stride x_ld bytes
@@ -203,13 +166,8 @@ void linear_kernel(const LinParams p) {
   for (int e = tid; e < p.N; e += kLinThreads) s_bias[e] = p.bias != nullptr ? p.bias[e] : 0.f;
   if constexpr (kEpi == kEpiGelu || kEpi == kEpiGeluKeep)
     gelu_table_fill(reinterpret_cast<uint16_t*>(smem + kLinGeluOff), tid, kLinThreads);
-  if constexpr (kEpi == kEpiGeluBwd) {  // s_bias holds the column sums
-    float* table = reinterpret_cast<float*>(smem + kLinGeluOff);
-    for (int e = tid; e < 2 * kSlopeTabSpan; e += kLinThreads) {
-      const uint32_t bits = e < kSlopeTabSpan ? kSlopeTabLo + e : 0x8000u + kSlopeTabLo + (e - kSlopeTabSpan);
-      table[e] = gelu_slope(__uint_as_float(bits << 16));
-    }
-  }
+  if constexpr (kEpi == kEpiGeluBwd)  // s_bias holds the column sums
+    slope_table_fill(reinterpret_cast<float*>(smem + kLinGeluOff), tid, kLinThreads);
   __syncthreads();
   const int xcd = (int)blockIdx.x & 7;
   const int nx = ((int)gridDim.x - xcd + 7) >> 3;  // workgroups with this blockIdx % 8
@@ -504,17 +462,7 @@ void linear_kernel(const LinParams p) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             float sl[8];
-            u16x2 dmax = {0, 0};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) slope_pair(h[q][j][e], s_slope, dmax, sl[2 * e], sl[2 * e + 1]);
-            const uint32_t dm = dmax.x > dmax.y ? dmax.x : dmax.y;
-            if (__builtin_amdgcn_ballot_w64(dm >= kSlopeRare) != 0) {
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                sl[2 * e] = slope_exact(h[q][j][e] & 0xffffu);
-                sl[2 * e + 1] = slope_exact(h[q][j][e] >> 16);
-              }
-            }
+            slope_chunk(h[q][j], s_slope, sl);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               const f32x4& c = acc[2 * (qb + q) + (e >> 1)][j];
@@ -554,29 +502,11 @@ void linear_kernel(const LinParams p) {
       }
       if constexpr (kEpi == kEpiGelu || kEpi == kEpiGeluKeep) {
 #pragma unroll
-        for (int ah = 0; ah < 2; ++ah) {
-          // Table lookups; a wave holding a value outside the table (|x| < 2^-22
-          // or >= 32) redoes the values exactly.
-          u16x2 dmax = {0, 0};
-          uint2 gv[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            uint2& v = o[j][4 * ah + i];
-            asm volatile("" : "+v"(v.x), "+v"(v.y));
-            gv[i].x = gelu_pair_table(v.x, s_gelu, dmax);
-            gv[i].y = gelu_pair_table(v.y, s_gelu, dmax);
-          }
-          const uint32_t dm = dmax.x > dmax.y ? dmax.x : dmax.y;
-          if (__builtin_amdgcn_ballot_w64(dm >= (uint32_t)kGeluSpan) != 0) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const uint2 v = o[j][4 * ah + i];
-              gv[i].x = gelu_bf16(v.x & 0xffffu, s_gelu) | (gelu_bf16(v.x >> 16, s_gelu) << 16);
-              gv[i].y = gelu_bf16(v.y & 0xffffu, s_gelu) | (gelu_bf16(v.y >> 16, s_gelu) << 16);
-            }
-          }
-#pragma unroll
-          for (int i = 0; i < 4; ++i) o[j][4 * ah + i] = gv[i];
+        for (int q = 0; q < 4; ++q) {
+          uint32_t v[4] = {o[j][2 * q].x, o[j][2 * q].y, o[j][2 * q + 1].x, o[j][2 * q + 1].y};
+          gelu_chunk(v, s_gelu);
+          o[j][2 * q] = make_uint2(v[0], v[1]);
+          o[j][2 * q + 1] = make_uint2(v[2], v[3]);
         }
       }
 #pragma unroll

@@ -60,10 +60,6 @@ __device__ __forceinline__ int wg_swz(int r) {
   return W % 128 == 0 ? 2 * (r & 7) : 2 * ((r >> 1) & 3);
 }
 
-__device__ __forceinline__ void dma_buffer_to_lds16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t lds_base) {
-  asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(voff), "s"(r), "{m0}"(lds_base) : "memory");
-}
-
 template <int WA, int WB>
 __global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void weight_grad_kernel(const WgParams p) {

@@ -933,6 +933,54 @@ def linear_gelu_backward(dy: torch.Tensor, weight_packed: torch.Tensor, out_feat
     return dh
 
 
+def linear_short_supported(x: torch.Tensor, in_features: int, out_features: int) -> bool:
+    """Whether :func:`linear_short` serves this layer: contiguous 16-byte
+    aligned bf16 device rows of 128 or 192 features, out_features a multiple of
+    128 or 192 up to 4096."""
+    return (x.device.type == "cuda" and x.dtype == torch.bfloat16 and in_features in (128, 192)
+            and 0 < out_features <= LINEAR_MAX_OUT and (out_features % 128 == 0 or out_features % 192 == 0)
+            and x.is_contiguous() and x.data_ptr() % 16 == 0 and x.numel() // in_features < 2 ** 31 - 64)
+
+
+def linear_short_fills(rows: int, out_features: int) -> bool:
+    """Whether a :func:`linear_short` launch has a 64-row tile of a feature
+    block for each of the 256 compute units; below that a training step's small
+    products stay with the library."""
+    width = 192 if out_features % 192 == 0 else 128
+    return -(-rows // 64) * (out_features // width) >= 256
+
+
+def linear_short(x: torch.Tensor, weight_packed: torch.Tensor, out_features: int,
+                 bias: Optional[torch.Tensor] = None, gelu_keep: bool = False):
+    """A linear layer of 128 or 192 input features over token rows
+    (terra_swin_linear_short): ``bf16(x W^T + b)``, or with ``gelu_keep`` the
+    pair (h, GELU(h)) of :func:`linear_gelu_keep`."""
+    dev = _require_device(x, weight_packed)
+    code = _dtype_code(x, (torch.bfloat16,))
+    k = x.shape[-1]
+    if not linear_short_supported(x, k, out_features):
+        raise ValueError("linear_short takes contiguous bf16 rows of 128 or 192 features and out_features % 128 == 0 or "
+                         f"% 192 == 0, <= 4096 (got {x.dtype}, {k} -> {out_features})")
+    if weight_packed.dtype != x.dtype or weight_packed.numel() != out_features * k or not weight_packed.is_contiguous():
+        raise ValueError(f"weight_packed must be a contiguous packed {x.dtype} tensor of {out_features * k} elements")
+    if bias is not None:
+        _require_device(x, bias)
+        if bias.dtype != torch.float32 or bias.numel() != out_features or not bias.is_contiguous():
+            raise ValueError(f"bias must be a contiguous fp32 tensor of {out_features} elements")
+        if bias.data_ptr() % 16:
+            bias = bias.clone()
+    shape = (*x.shape[:-1], out_features)
+    y = torch.empty(shape, dtype=x.dtype, device=dev)
+    keep = torch.empty(shape, dtype=x.dtype, device=dev) if gelu_keep else None
+    if x.numel():
+        with torch.cuda.device(dev):
+            st = _lib.load().terra_swin_linear_short(_ptr(x), _ptr(y), _ptr(keep), code, x.numel() // k, int(k),
+                                                     int(out_features), _ptr(weight_packed), _ptr(bias),
+                                                     1 if gelu_keep else 0, _stream(dev))
+        _lib.check(st, "terra_swin_linear_short")
+    return (keep, y) if gelu_keep else y
+
+
 def weight_grad_supported(dy: torch.Tensor, x: torch.Tensor) -> bool:
     """Whether :func:`weight_grad` serves dy [T, out] and x [T, in]: contiguous
     16-byte aligned bf16 device rows (1 <= T < 2^31), feature counts multiples

@@ -498,3 +498,18 @@ def test_weight_grad_rejects_bad_arguments():
     assert lib.terra_swin_weight_grad_slices(4096, 768, 192) == 8
     assert lib.terra_swin_weight_grad_slices(100, 768, 192) == 1
     assert lib.terra_swin_weight_grad_slices(4096, 24, 192) < 0
+
+
+def test_linear_short_rejects_bad_arguments():
+    p = lambda a: ctypes.c_void_p(a << 28)  # noqa: E731
+
+    def call(x=p(1), y=p(2), keep=None, dtype=L.DTYPE_BF16, rows=512, k=192, n=576, w=p(4), b=None, epi=0):
+        return L.load().terra_swin_linear_short(x, y, keep, dtype, rows, k, n, w, b, epi, None)
+
+    assert call(x=None) == -1 and call(w=None) == -1 and call(y=None) == -1
+    assert call(keep=p(3)) == -1 and call(epi=1) == -1 and call(epi=2) == -3
+    assert call(dtype=L.DTYPE_F32) == -5 and call(dtype=9) == -2
+    assert call(k=64) == -3 and call(n=320) == -3 and call(n=4224) == -3 and call(rows=-1) == -3
+    assert call(x=ctypes.c_void_p((1 << 28) + 8)) == -4 and call(b=ctypes.c_void_p((1 << 28) + 4)) == -4
+    assert call(y=p(1)) == -3 and call(keep=p(2), epi=1) == -3 and "overlap" in L.last_error()
+    assert call(rows=0) == 0

@@ -223,3 +223,31 @@ def test_linear_empty_rows(dev):
     w = kernels.pack_linear(torch.zeros(256, 256, dtype=torch.bfloat16, device=dev))
     assert kernels.linear(x, w, 256).shape == (0, 256)
     assert kernels.linear_residual(x, w, 256, torch.empty(0, 256, dtype=torch.bfloat16, device=dev)).shape == (0, 256)
+
+
+# (rows, in, out): one row, a tail row, whole tiles, feature blocks of 192 and
+# 128, one and several blocks, more tiles than resident workgroups.
+SHORT_SHAPES = [(1, 192, 192), (64, 128, 128), (65, 192, 128), (300, 128, 192), (500, 128, 512), (777, 192, 1024),
+                (70001, 192, 576), (120000, 128, 384), (90000, 192, 768)]
+
+
+@pytest.mark.parametrize("rows,k,n", SHORT_SHAPES)
+def test_linear_short(dev, rows, k, n):
+    """The short-row linear kernel against float64 (one fp32 sum of k products
+    and its bf16 rounding), with and without bias, and its GELU pair: h the
+    same bits, y torch's GELU of h; memory past the outputs untouched."""
+    x = torch.randn(rows, k, device=dev, generator=torch.Generator(dev).manual_seed(40)).bfloat16()
+    w, b = _weights(n, k, 41, scale=k ** -0.5)
+    pk, bd = kernels.pack_linear(w.to(dev)), b.to(dev)
+    y = kernels.linear_short(x, pk, n, bd)
+    ref = x.double() @ w.to(dev).double().t()
+    mag = x.double().abs() @ w.to(dev).double().abs().t() + bd.double().abs()
+    assert ((y.double() - ref - bd.double()).abs() <= (ref + bd.double()).abs() * 2.0 ** -8 + mag * k * 2.0 ** -24).all()
+    assert ((kernels.linear_short(x, pk, n).double() - ref).abs() <= ref.abs() * 2.0 ** -8 + mag * k * 2.0 ** -24).all()
+    h, a = kernels.linear_short(x, pk, n, bd, gelu_keep=True)
+    assert torch.equal(h, y) and torch.equal(a, torch.nn.functional.gelu(h))
+    guard = torch.full((rows * n + 4096,), 7.0, device=dev, dtype=torch.bfloat16)
+    st = L.load().terra_swin_linear_short(x.data_ptr(), guard.data_ptr(), None, L.DTYPE_BF16, rows, k, n, pk.data_ptr(),
+                                          bd.data_ptr(), 0, None)
+    torch.cuda.synchronize()
+    assert st == 0 and torch.equal(guard[:rows * n].view(rows, n), y) and bool((guard[rows * n:] == 7.0).all())

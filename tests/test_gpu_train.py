@@ -534,24 +534,28 @@ def test_mlp_training_on_linear_kernels(dev, x_dtype, C, tokens):
     gy = workloads.activations((tokens, C), 592).to(x_dtype)
     md = copy.deepcopy(m).to(dev)
     calls = {"keep": 0, "bwd": 0}
-    k0, b0 = kernels.linear_gelu_keep, kernels.linear_gelu_backward
+    k0, s0, b0 = kernels.linear_gelu_keep, kernels.linear_short, kernels.linear_gelu_backward
 
     def ck(*a, **k):
         calls["keep"] += 1
         return k0(*a, **k)
 
+    def cs(*a, **k):
+        calls["keep"] += bool(k.get("gelu_keep"))
+        return s0(*a, **k)
+
     def cb(*a, **k):
         calls["bwd"] += 1
         return b0(*a, **k)
 
-    kernels.linear_gelu_keep, kernels.linear_gelu_backward = ck, cb
+    kernels.linear_gelu_keep, kernels.linear_short, kernels.linear_gelu_backward = ck, cs, cb
     try:
         xd = x.to(dev).requires_grad_(True)
         with torch.amp.autocast(device_type="cuda", dtype=torch.bfloat16):
             y = md(xd)
         y.backward(gy.to(dev))
     finally:
-        kernels.linear_gelu_keep, kernels.linear_gelu_backward = k0, b0
+        kernels.linear_gelu_keep, kernels.linear_short, kernels.linear_gelu_backward = k0, s0, b0
     assert calls == {"keep": 1, "bwd": 1} and y.dtype == x_dtype
     mref = copy.deepcopy(m).to(dev)
     yr, xg, pg = _oracle_mlp_grads(mref, x.to(dev), gy.to(dev), torch.float64, bf16_weights=True)
