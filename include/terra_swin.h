@@ -393,6 +393,17 @@ int terra_swin_block_fwd(const void* x, void* y, int dtype,
 int terra_swin_pack_linear(const void* weight, void* packed, int dtype,
                            int out_features, int in_features, void* stream);
 
+/* terra_swin_block_fwd in fp32 for the small fp32 configuration: 7x7 windows, 96
+ * channels, 3 heads.  x, y and all parameters fp32; qkv_weight [288, 96] and
+ * proj_weight [96, 96] row-major (packed_weights must be 0); the rest as
+ * terra_swin_block_fwd, every product, statistic and sum in fp32.
+ */
+int terra_swin_block_f32_fwd(const float* x, float* y, const terra_swin_block_desc* desc,
+                             const float* ln_gamma, const float* ln_beta,
+                             const float* qkv_weight, const float* qkv_bias,
+                             const float* proj_weight, const float* proj_bias,
+                             const float* bias_table, const uint64_t* land_bits, void* stream);
+
 /* Fused MLP half-block (bf16 activations).
  * Replaces SequentialMlp.forward              models/mlp.py:152-172:
  *           x = self.norm2(x)                  models/mlp.py:159 (nn.LayerNorm)

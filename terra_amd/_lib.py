@@ -66,6 +66,7 @@ EXPORTED_SYMBOLS = (
     "terra_swin_linear_gelu_bwd",
     "terra_swin_pack_weight",
     "terra_swin_weight_grad",
+    "terra_swin_block_f32_fwd",
     "terra_swin_linear_short",
     "terra_swin_weight_grad_slices",
 )
@@ -251,6 +252,9 @@ def load() -> ctypes.CDLL:
                                                    vp]
         lib.terra_swin_weight_grad_slices.restype = ctypes.c_int
         lib.terra_swin_weight_grad_slices.argtypes = [i64, ctypes.c_int, ctypes.c_int]
+        lib.terra_swin_block_f32_fwd.restype = ctypes.c_int
+        lib.terra_swin_block_f32_fwd.argtypes = [vp, vp, ctypes.POINTER(SwinBlockDesc), vp, vp, vp, vp, vp, vp, vp, vp,
+                                                 vp]
         lib.terra_swin_linear_short.restype = ctypes.c_int
         lib.terra_swin_linear_short.argtypes = [vp, vp, vp, ctypes.c_int, i64, ctypes.c_int, ctypes.c_int, vp, vp,
                                                 ctypes.c_int, vp]

@@ -182,6 +182,14 @@ def _bf16_linears(x: torch.Tensor, *params: Optional[torch.Tensor]) -> bool:
     return all(p is None or p.dtype == torch.bfloat16 for p in params)
 
 
+def _bias32(bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """A bias as the linear kernels read it: contiguous 16-byte aligned fp32."""
+    if bias is None:
+        return None
+    b = bias.float().contiguous()
+    return b.clone() if b.data_ptr() % 16 else b
+
+
 def _short_kernel(x: torch.Tensor, out_features: int) -> bool:
     """The short-row linear kernels serve and fill the chip with rows like x
     (524288 rows, us, against the library's product: 192 -> 576 130 / 300,
@@ -192,7 +200,7 @@ def _short_kernel(x: torch.Tensor, out_features: int) -> bool:
 
 def _linear_kernel(x: torch.Tensor, out_features: int) -> bool:
     """The token-row linear kernels serve and fill the chip with rows like x."""
-    return (x.is_contiguous() and kernels.linear_supported(x, x.shape[-1], out_features)
+    return (x.is_contiguous() and x.data_ptr() % 16 == 0 and kernels.linear_supported(x, x.shape[-1], out_features)
             and kernels.linear_fills(x.numel() // x.shape[-1], out_features))
 
 
@@ -229,7 +237,7 @@ class _Linear(torch.autograd.Function):
         o = weight.shape[0]
         if (dt == torch.bfloat16 and weight.dim() == 2 and weight.shape[1] == x.shape[-1]
                 and (bias is None or bias.numel() == o) and _bf16_linears(xc, weight, bias) and _short_kernel(xc, o)):
-            return kernels.linear_short(xc, kernels.pack_weight(wc), o, None if bias is None else bias.float())
+            return kernels.linear_short(xc, kernels.pack_weight(wc), o, _bias32(bias))
         bc = None if bias is None else bias.to(dt)
         return torch.nn.functional.linear(xc, wc, bc)
 
@@ -291,11 +299,12 @@ class _Mlp(torch.autograd.Function):
         y = None
         bf16 = xn.dtype == torch.bfloat16 and _bf16_linears(xn, w1, b1, w2, b2)
         if bf16 and _short_kernel(xn, w1.shape[0]):
-            h1, a = kernels.linear_short(xn, kernels.pack_weight(w1), w1.shape[0], b1.float(), gelu_keep=True)
+            h1, a = kernels.linear_short(xn, kernels.pack_weight(w1), w1.shape[0], _bias32(b1), gelu_keep=True)
         elif bf16 and _linear_kernel(xn, w1.shape[0]):
-            h1, a = kernels.linear_gelu_keep(xn, kernels.pack_weight(w1), w1.shape[0], b1.float())
-            if rows.dtype == torch.bfloat16 and w2.shape[0] == C and _linear_kernel(a, C):
-                y = kernels.linear_residual(a, kernels.pack_weight(w2), C, rows, b2.float())
+            h1, a = kernels.linear_gelu_keep(xn, kernels.pack_weight(w1), w1.shape[0], _bias32(b1))
+            if rows.dtype == torch.bfloat16 and w2.shape[0] == C and rows.data_ptr() % 16 == 0 \
+                    and _linear_kernel(a, C):
+                y = kernels.linear_residual(a, kernels.pack_weight(w2), C, rows, _bias32(b2))
         else:
             h1 = torch.nn.functional.linear(xn, w1, b1)
             a = torch.nn.functional.gelu(h1)

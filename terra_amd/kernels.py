@@ -586,6 +586,17 @@ def swin_block_supported(x: torch.Tensor, geom: WindowGeometry, num_heads: int) 
             and (geom.window, num_heads, geom.channels) in BLOCK_SHAPES)
 
 
+# (window, heads, channels) of the fp32 half-block kernel.
+BLOCK_F32_SHAPES = ((7, 3, 96),)
+
+
+def swin_block_f32_supported(x: torch.Tensor, geom: WindowGeometry, num_heads: int) -> bool:
+    """Whether :func:`swin_block_f32` serves this call (fp32 device tensor,
+    (window, heads, channels) in BLOCK_F32_SHAPES)."""
+    return (x.device.type == "cuda" and x.dtype == torch.float32
+            and (geom.window, num_heads, geom.channels) in BLOCK_F32_SHAPES)
+
+
 def pack_linear(weight: torch.Tensor) -> torch.Tensor:
     """MFMA fragment order of a bf16 nn.Linear weight [out, in] (out % 16 == 0,
     in % 32 == 0) for :func:`swin_block` with ``packed_weights=True``; returns
@@ -629,12 +640,35 @@ def swin_block(x: torch.Tensor, geom: WindowGeometry, num_heads: int, scale: flo
         if out.shape != x.shape or out.dtype != x.dtype or out.device != x.device:
             raise ValueError("out must be a contiguous tensor like x")
         return out
+    _dtype_code(x, (torch.bfloat16,))
     given = (qkv_weight, qkv_bias, proj_weight, proj_bias, ln_weight, ln_bias, bias_table, land_bits)
     key = ("block", tuple(map(id, given)), geom, num_heads, float(scale), float(ln_eps), bool(layernorm),
            bool(shift_mask), float(mask_value), bool(packed_weights), x.shape, x.dtype, x.device)
     return _prepared(key, given, lambda: _BlockLaunch(
         x, geom, num_heads, scale, qkv_weight, qkv_bias, proj_weight, proj_bias, ln_weight, ln_bias, ln_eps,
         layernorm, bias_table, shift_mask, land_bits, mask_value, packed_weights))(x, out)
+
+
+def swin_block_f32(x: torch.Tensor, geom: WindowGeometry, num_heads: int, scale: float,
+                   qkv_weight: torch.Tensor, qkv_bias: Optional[torch.Tensor],
+                   proj_weight: torch.Tensor, proj_bias: Optional[torch.Tensor],
+                   ln_weight: Optional[torch.Tensor] = None, ln_bias: Optional[torch.Tensor] = None,
+                   ln_eps: float = 1e-5, layernorm: bool = True,
+                   bias_table: Optional[torch.Tensor] = None, shift_mask: bool = False,
+                   land_bits: Optional[torch.Tensor] = None, mask_value: float = MASK_VALUE,
+                   out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """:func:`swin_block` in fp32 (terra_swin_block_f32_fwd) for the shapes of
+    BLOCK_F32_SHAPES: fp32 ``x`` [B, H, W, C] and parameters, row-major
+    ``qkv_weight`` [3C, C] and ``proj_weight`` [C, C]."""
+    if geom.batch == 0 and x.numel() == 0:
+        _require_device(x)
+        return torch.empty_like(x) if out is None else out
+    given = (qkv_weight, qkv_bias, proj_weight, proj_bias, ln_weight, ln_bias, bias_table, land_bits)
+    key = ("block_f32", tuple(map(id, given)), geom, num_heads, float(scale), float(ln_eps), bool(layernorm),
+           bool(shift_mask), float(mask_value), x.shape, x.dtype, x.device)
+    return _prepared(key, given, lambda: _BlockLaunch(
+        x, geom, num_heads, scale, qkv_weight, qkv_bias, proj_weight, proj_bias, ln_weight, ln_bias, ln_eps,
+        layernorm, bias_table, shift_mask, land_bits, mask_value, False))(x, out)
 
 
 # Prepared launches, keyed by the ids of the parameter tensors, the call's
@@ -692,7 +726,8 @@ class _Launch:
         elif out.shape != x.shape or out.dtype != x.dtype or not out.is_contiguous() or out.device != self.device:
             raise ValueError("out must be a contiguous tensor like x")
         dev = self.device
-        args = (x.data_ptr(), out.data_ptr(), self.code, ctypes.byref(self.desc)) + self.ptrs
+        code = () if self.code is None else (self.code,)
+        args = (x.data_ptr(), out.data_ptr(), *code, ctypes.byref(self.desc)) + self.ptrs
         if dev.index is not None and dev.index != torch.cuda.current_device():
             with torch.cuda.device(dev):
                 st = self.fn(*args, _stream(dev))
@@ -703,12 +738,17 @@ class _Launch:
 
 
 class _BlockLaunch(_Launch):
-    """terra_swin_block_fwd with its checks (see :func:`swin_block`)."""
+    """terra_swin_block_fwd, or for fp32 x terra_swin_block_f32_fwd, with its
+    checks (see :func:`swin_block`, :func:`swin_block_f32`)."""
 
     def __init__(self, x, geom, num_heads, scale, qkv_weight, qkv_bias, proj_weight, proj_bias, ln_weight, ln_bias,
                  ln_eps, layernorm, bias_table, shift_mask, land_bits, mask_value, packed_weights):
         dev = _require_device(x, qkv_weight, proj_weight)
-        code = _dtype_code(x, (torch.bfloat16,))
+        f32_block = x.dtype == torch.float32
+        if f32_block and not swin_block_f32_supported(x, geom, num_heads):
+            raise ValueError(f"the fp32 half-block serves (window, heads, channels) in {BLOCK_F32_SHAPES} (got "
+                             f"{(geom.window, num_heads, geom.channels)})")
+        code = _dtype_code(x, (torch.bfloat16, torch.float32) if f32_block else (torch.bfloat16,))
         C = geom.channels
         if tuple(x.shape) != (geom.batch, geom.height, geom.width, C) or not x.is_contiguous():
             raise ValueError(f"x must be a contiguous [{geom.batch}, {geom.height}, {geom.width}, {C}] tensor")
@@ -766,7 +806,10 @@ class _BlockLaunch(_Launch):
         self.keep = tuple(copies) or None  # converted copies live as long as this (uncached) launch
         self.ptrs = (_ptr(params[0]), _ptr(params[1]), _ptr(qkv_weight), _ptr(params[2]), _ptr(proj_weight),
                      _ptr(params[3]), _ptr(table), _ptr(land_bits))
-        self.fn, self.name = _lib.load().terra_swin_block_fwd, "terra_swin_block_fwd"
+        if f32_block:  # no dtype argument
+            self.fn, self.name, self.code = _lib.load().terra_swin_block_f32_fwd, "terra_swin_block_f32_fwd", None
+        else:
+            self.fn, self.name = _lib.load().terra_swin_block_fwd, "terra_swin_block_fwd"
 
 
 MLP_CHANNELS = (128, 192, 384, 768)
@@ -882,6 +925,8 @@ def pack_weight(weight: torch.Tensor, transpose: bool = False) -> torch.Tensor:
     if weight.dim() != 2:
         raise ValueError("weight must be a 2-D tensor")
     weight = weight.detach().contiguous()
+    if weight.data_ptr() % 16:  # a view into a flat parameter buffer
+        weight = weight.clone()
     n, k = (weight.shape[1], weight.shape[0]) if transpose else weight.shape
     out = torch.empty(n * k, dtype=torch.bfloat16, device=dev)
     with torch.cuda.device(dev):
@@ -967,8 +1012,6 @@ def linear_short(x: torch.Tensor, weight_packed: torch.Tensor, out_features: int
         _require_device(x, bias)
         if bias.dtype != torch.float32 or bias.numel() != out_features or not bias.is_contiguous():
             raise ValueError(f"bias must be a contiguous fp32 tensor of {out_features} elements")
-        if bias.data_ptr() % 16:
-            bias = bias.clone()
     shape = (*x.shape[:-1], out_features)
     y = torch.empty(shape, dtype=x.dtype, device=dev)
     keep = torch.empty(shape, dtype=x.dtype, device=dev) if gelu_keep else None

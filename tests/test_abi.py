@@ -513,3 +513,21 @@ def test_linear_short_rejects_bad_arguments():
     assert call(x=ctypes.c_void_p((1 << 28) + 8)) == -4 and call(b=ctypes.c_void_p((1 << 28) + 4)) == -4
     assert call(y=p(1)) == -3 and call(keep=p(2), epi=1) == -3 and "overlap" in L.last_error()
     assert call(rows=0) == 0
+
+
+def test_block_f32_rejects_bad_arguments():
+    p = lambda a: ctypes.c_void_p(a << 28)  # noqa: E731
+
+    def call(x=p(1), y=p(2), w=p(3), wp=p(4), land=None, packed=0, heads=3, eps=1e-5, **geom):
+        d = L.SwinBlockDesc()
+        d.geom = _geom(**dict(dict(height=14, width=21, channels=96, window=7), **geom))
+        d.heads, d.scale, d.ln_eps, d.layernorm, d.packed_weights = heads, 0.1, eps, 1, packed
+        d.land_windows = 4
+        return L.load().terra_swin_block_f32_fwd(x, y, ctypes.byref(d), None, None, w, None, wp, None, None, land, None)
+
+    assert call(x=None) == -1 and call(w=None) == -1
+    assert call(window=8, height=16, width=16) == -5 and call(channels=128) == -5 and call(heads=4) == -5
+    assert call(packed=1) == -5 and call(eps=-1.0) == -3 and call(height=15) == -3
+    assert call(y=ctypes.c_void_p((2 << 28) + 4)) == -4 and call(y=ctypes.c_void_p((1 << 28) + 64)) == -3
+    assert call(land=p(5)) == -3 and "land_windows" in L.last_error()
+    assert L.load().terra_swin_block_f32_fwd(p(1), p(2), None, None, None, p(3), None, p(4), None, None, None, None) == -1

@@ -1,0 +1,89 @@
+"""GPU parity of the fp32 half-block kernel (terra_swin_block_f32_fwd: 7x7
+windows, 96 channels, 3 heads) against the float64 oracle (1e-5, the fp32
+contract; measured 1e-7 to 1e-6) and against the staged path, over every frame
+form."""
+import pytest
+import torch
+
+from helpers import assert_block_matches, gain_block, params_of, rel_norm
+from oracle import swin_oracle as so
+from terra_amd import config, kernels, workloads
+from terra_amd.transformer import SequentialSwinTransformer
+
+pytestmark = pytest.mark.gpu
+
+# (B, H, W, layer, pad, win_row_begin, win_rows, valid, land, mask, bias)
+CASES = [
+    (1, 7, 7, 0, (0, 0, 0, 0), 0, None, None, False, True, True),        # one window
+    (1, 56, 56, 0, (0, 0, 0, 0), 0, None, None, False, True, True),
+    (2, 28, 42, 1, (0, 0, 0, 0), 0, None, None, False, True, True),      # shifted, masked
+    (1, 28, 28, 1, (0, 0, 0, 0), 0, None, None, True, False, True),      # land keys, no shift mask
+    (3, 21, 35, 1, (0, 0, 0, 0), 0, None, None, True, True, False),      # land and shift, no bias table
+    (2, 25, 31, 1, (2, 1, 1, 3), 0, None, None, True, True, True),       # frame padding on every side
+    (2, 21, 28, 1, (0, 7, 0, 0), 0, 3, (2, 9), True, True, True),        # slab: rows not emitted, pad windows
+    (1, 140, 161, 1, (0, 0, 0, 0), 0, None, None, True, True, True),     # 460 windows: two per workgroup
+]
+
+
+def _block(dev, case):
+    B, H, W, layer, pad, r0, rows, valid, land, mask, bias = case
+    lm = workloads.land_mask(H, W, seed=71) if land else None
+    blk = SequentialSwinTransformer(layer_idx=layer, height=H, width=W, embedding_dim=96, window_size=7, num_heads=3,
+                                    use_attn_mask=mask, use_relative_position_bias=bias, land_mask=lm, pad=pad,
+                                    win_row_begin=r0, win_rows=rows, valid_windows=valid)
+    workloads.init_block_params(blk, layer)
+    return gain_block(blk).to(dev), lm, workloads.activations((B, H * W, 96), 72)
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_block_f32_matches_oracle_and_staged_path(dev, case, monkeypatch):
+    B, H, W, layer, pad, r0, rows, valid, land, mask, bias = case
+    blk, lm, x = _block(dev, case)
+    calls = []
+    orig = kernels.swin_block_f32
+    monkeypatch.setattr(kernels, "swin_block_f32", lambda *a, **k: calls.append(1) or orig(*a, **k))
+    xd = x.to(dev)
+    with torch.no_grad():
+        y = blk(xd)
+        blk.use_fused_block = False
+        staged = blk(xd)
+    assert calls == [1]
+    ref = so.swin_block_attention(x, H, W, 7, blk.shift_size, 3, params_of(blk), land=lm, use_attn_mask=mask, pad=pad,
+                                  win_row_begin=r0, win_rows=rows, valid=valid, compute_dtype=torch.float64)
+    assert_block_matches(y, ref, x, 1e-5, 1e-5)
+    assert rel_norm(y - xd, staged - xd) <= 1e-5
+
+
+def test_block_f32_in_place_without_layernorm_and_routes(dev, monkeypatch):
+    """out = x gives the same bits; LayerNorm off; autocast, gradients and
+    bf16 parameters keep their own paths; parameter updates are seen."""
+    blk, _, x = _block(dev, CASES[2])
+    xd = x.to(dev)
+    geom = blk.geometry(2)
+    grid = xd.view(2, 28, 42, 96)
+    with torch.no_grad():
+        want = blk(xd).view_as(grid)
+        buf = grid.clone()
+        got = kernels.swin_block_f32(buf, geom, 3, blk.attn.scale, shift_mask=True, out=buf,
+                                     **blk._block_f32_args(grid, geom))
+        assert got.data_ptr() == buf.data_ptr() and torch.equal(got, want)
+        blk.attn.proj.weight.mul_(0.5)
+        blk.attn.k_linear.bias.add_(1.0)
+        changed = blk(xd).view_as(grid)
+        assert not torch.equal(changed, want)
+        blk.use_fused_block = False
+        assert rel_norm(changed - grid, blk(xd).view_as(grid) - grid) <= 1e-5
+        blk.use_fused_block = True
+        with torch.amp.autocast("cuda", dtype=torch.bfloat16):
+            assert blk._block_f32_args(grid, geom) is None
+    assert blk._block_f32_args(grid, geom) is None  # parameters need gradients
+    with torch.no_grad(), pytest.raises((TypeError, ValueError)):
+        kernels.swin_block(grid, geom, 3, 1.0, torch.zeros(288, 96, device=dev), None, torch.zeros(96, 96, device=dev), None)
+    monkeypatch.setattr(config, "use_layernorm", False)
+    plain = SequentialSwinTransformer(layer_idx=1, height=28, width=42, embedding_dim=96, window_size=7, num_heads=3)
+    workloads.init_block_params(plain, 1)
+    plain = plain.to(dev)
+    with torch.no_grad():
+        y = plain(xd)
+        plain.use_fused_block = False
+        assert rel_norm(y - xd, plain(xd) - xd) <= 1e-5

@@ -605,3 +605,30 @@ def test_weight_grad_refuses_other_operands(dev):
                           (dy[:, :8].contiguous(), dy)):
         with pytest.raises((ValueError, TypeError)):
             kernels.weight_grad(bad_dy, bad_x)
+
+
+def test_training_accepts_parameters_at_any_offset(dev):
+    """Parameters that are views into one flat buffer (4-byte offsets): the same
+    gradients as aligned ones."""
+    torch.manual_seed(7)
+    m = _mlp_case(192, 610).to(dev)
+    x = workloads.activations((9000, 192), 611).to(dev)
+    gy = workloads.activations((9000, 192), 612).to(dev)
+
+    def grads(shift):
+        md = copy.deepcopy(m)
+        params = list(md.parameters())
+        flat = torch.empty(sum(p.numel() + shift for p in params) + shift, device=dev)
+        at = shift
+        for p in params:
+            flat[at:at + p.numel()].copy_(p.detach().reshape(-1))
+            p.data = flat[at:at + p.numel()].view(p.shape)
+            at += p.numel() + shift
+        xs = x.clone().requires_grad_(True)
+        with torch.amp.autocast("cuda", dtype=torch.bfloat16):
+            y = md(xs)
+        y.backward(gy)
+        return [y.detach(), xs.grad] + [p.grad for p in params]
+
+    for a, b in zip(grads(0), grads(1)):
+        assert _normwise(a, b) <= 1e-6
