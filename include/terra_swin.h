@@ -404,6 +404,18 @@ int terra_swin_block_f32_fwd(const float* x, float* y, const terra_swin_block_de
                              const float* proj_weight, const float* proj_bias,
                              const float* bias_table, const uint64_t* land_bits, void* stream);
 
+/* The same that also writes what the training step's backward reads: the
+ * LayerNorm windows [B * nW, 49, 96], q | k | v [B * nW, 49, 288] and the
+ * attention output [B * nW, 49, 96] of every emitted window (no valid-window
+ * range).
+ */
+int terra_swin_block_f32_train(const float* x, float* y, float* windows, float* qkv, float* o,
+                               const terra_swin_block_desc* desc,
+                               const float* ln_gamma, const float* ln_beta,
+                               const float* qkv_weight, const float* qkv_bias,
+                               const float* proj_weight, const float* proj_bias,
+                               const float* bias_table, const uint64_t* land_bits, void* stream);
+
 /* Fused MLP half-block (bf16 activations).
  * Replaces SequentialMlp.forward              models/mlp.py:152-172:
  *           x = self.norm2(x)                  models/mlp.py:159 (nn.LayerNorm)

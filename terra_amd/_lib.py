@@ -67,6 +67,7 @@ EXPORTED_SYMBOLS = (
     "terra_swin_pack_weight",
     "terra_swin_weight_grad",
     "terra_swin_block_f32_fwd",
+    "terra_swin_block_f32_train",
     "terra_swin_linear_short",
     "terra_swin_weight_grad_slices",
 )
@@ -255,6 +256,9 @@ def load() -> ctypes.CDLL:
         lib.terra_swin_block_f32_fwd.restype = ctypes.c_int
         lib.terra_swin_block_f32_fwd.argtypes = [vp, vp, ctypes.POINTER(SwinBlockDesc), vp, vp, vp, vp, vp, vp, vp, vp,
                                                  vp]
+        lib.terra_swin_block_f32_train.restype = ctypes.c_int
+        lib.terra_swin_block_f32_train.argtypes = [vp, vp, vp, vp, vp, ctypes.POINTER(SwinBlockDesc), vp, vp, vp, vp,
+                                                   vp, vp, vp, vp, vp]
         lib.terra_swin_linear_short.restype = ctypes.c_int
         lib.terra_swin_linear_short.argtypes = [vp, vp, vp, ctypes.c_int, i64, ctypes.c_int, ctypes.c_int, vp, vp,
                                                 ctypes.c_int, vp]

@@ -218,6 +218,19 @@ def _input_grad(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return dy @ weight.to(dy.dtype)
 
 
+def _linear_forward(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]):
+    """F.linear in the dtype bf16 autocast gives it; returns the result and x
+    and weight in that dtype (for the backward)."""
+    dt = torch.bfloat16 if (torch.is_autocast_enabled(x.device.type)
+                            and torch.get_autocast_dtype(x.device.type) == torch.bfloat16) else x.dtype
+    xc, wc = x.to(dt), weight.to(dt)
+    o = weight.shape[0]
+    if (dt == torch.bfloat16 and weight.dim() == 2 and weight.shape[1] == x.shape[-1]
+            and (bias is None or bias.numel() == o) and _bf16_linears(xc, weight, bias) and _short_kernel(xc, o)):
+        return kernels.linear_short(xc, kernels.pack_weight(wc), o, _bias32(bias)), xc, wc
+    return torch.nn.functional.linear(xc, wc, None if bias is None else bias.to(dt)), xc, wc
+
+
 class _Linear(torch.autograd.Function):
     """F.linear for training, in the dtype bf16 autocast gives it (x, weight
     and bias cast to bf16 inside an autocast region, as F.linear's autocast
@@ -228,18 +241,11 @@ class _Linear(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, weight, bias, bias_sums):
-        dt = torch.bfloat16 if (torch.is_autocast_enabled(x.device.type)
-                                and torch.get_autocast_dtype(x.device.type) == torch.bfloat16) else x.dtype
-        xc, wc = x.to(dt), weight.to(dt)
+        y, xc, wc = _linear_forward(x, weight, bias)
         ctx.save_for_backward(xc, wc)
         ctx.dtypes = (x.dtype, weight.dtype, None if bias is None else bias.dtype)
         ctx.bias_sums = bias_sums
-        o = weight.shape[0]
-        if (dt == torch.bfloat16 and weight.dim() == 2 and weight.shape[1] == x.shape[-1]
-                and (bias is None or bias.numel() == o) and _bf16_linears(xc, weight, bias) and _short_kernel(xc, o)):
-            return kernels.linear_short(xc, kernels.pack_weight(wc), o, _bias32(bias))
-        bc = None if bias is None else bias.to(dt)
-        return torch.nn.functional.linear(xc, wc, bc)
+        return y
 
     @staticmethod
     def backward(ctx, dy: torch.Tensor):
@@ -509,3 +515,117 @@ def window_attention_qkv(qkv: torch.Tensor, num_heads: int, window_size: Tuple[i
                                    bias_sums)
     return kernels.window_attention(qkv[..., :C], qkv[..., C:2 * C], qkv[..., 2 * C:], num_heads, window_size,
                                     scale, bias_table=bias_table, mask=mask, n_real=n_real, mask_value=mask_value)
+
+
+class _AttentionHalf(torch.autograd.Function):
+    """SequentialSwinTransformer.forward (models/transformer.py:142-300) for
+    training as one function:
+
+        y = x + reverse(proj(attention(qkv(partition(LayerNorm(x))))))
+
+    through the kernels of partition_ln, linear, window_attention_qkv and
+    reverse above, in the dtypes bf16 autocast gives each.  One function
+    instead of a chain of them: a small block's step is bound by the host
+    (fp32, 56x56 tokens, C = 96: 757 us for 230 us of GPU work with separate
+    functions, concatenation nodes and a fill per accumulator, 525-690 us so;
+    408-577 us with the fp32 kernel that serves that shape's whole forward in
+    one launch and keeps what the backward reads)."""
+
+    @staticmethod
+    def forward(ctx, x, ln_w, ln_b, qw, kw, vw, qb, kb, vb, pw, pb, table, geom, eps, num_heads, scale, mask):
+        C = geom.channels
+        w, b = torch.cat((qw, kw, vw), 0), None if qb is None else torch.cat((qb, kb, vb), 0)
+        ctx.cfg = (geom, eps, num_heads, scale, mask)
+        if x.dtype == torch.float32 and not torch.is_autocast_enabled(x.device.type):
+            # The small fp32 configuration: the whole forward in one launch.
+            done = kernels.swin_block_f32_train(x, geom, num_heads, scale, w, b, pw, pb, ln_w, ln_b, eps, table, mask)
+            if done is not None:
+                y, windows, qkv, o = done
+                ctx.dtypes = (x.dtype, x.dtype, qw.dtype, None if qb is None else qb.dtype, pw.dtype, pb.dtype)
+                ctx.save_for_backward(x, ln_w, ln_b, windows, w, qkv, table, o, pw)
+                return y
+        windows = kernels.swin_partition_ln(x, geom, ln_w, ln_b, eps, out_dtype=linear_input_dtype(x))
+        qkv, xw, wc = _linear_forward(windows, w, b)
+        ws = (geom.window, geom.window)
+        o = kernels.window_attention(qkv[..., :C], qkv[..., C:2 * C], qkv[..., 2 * C:], num_heads, ws, scale,
+                                     bias_table=table, mask=mask)
+        p, oc, pwc = _linear_forward(o, pw, pb)
+        out_dtype = torch.promote_types(p.dtype, x.dtype)
+        if out_dtype != p.dtype and not (p.dtype == torch.bfloat16 and out_dtype == torch.float32):
+            p = p.to(out_dtype)
+        y = kernels.swin_reverse(p.contiguous(), geom, residual=x.to(out_dtype), out_dtype=out_dtype)
+        ctx.dtypes = (windows.dtype, p.dtype, qw.dtype, None if qb is None else qb.dtype, pw.dtype, pb.dtype)
+        ctx.save_for_backward(x, ln_w, ln_b, xw, wc, qkv, table, oc, pwc)
+        return y
+
+    @staticmethod
+    def backward(ctx, dy: torch.Tensor):
+        x, ln_w, ln_b, xw, wc, qkv, table, oc, pwc = ctx.saved_tensors
+        geom, eps, num_heads, scale, mask = ctx.cfg
+        win_dtype, p_dtype, w_dtype, b_dtype, pw_dtype, pb_dtype = ctx.dtypes
+        need = ctx.needs_input_grad
+        C, dev = geom.channels, x.device
+        # Accumulators the kernels add into, in one zeroed buffer.
+        sums_p = p_dtype != dy.dtype and need[10]
+        sums_qkv = b_dtype is not None and any(need[6:9]) and kernels.attention_backward_sums_supported(
+            qkv[..., :C], num_heads, (geom.window, geom.window), None)
+        sizes = [C if sums_p else 0, 3 * C if sums_qkv else 0, table.numel() if table is not None and need[11] else 0,
+                 C if ln_w is not None and need[1] else 0, C if ln_b is not None and need[2] else 0]
+        sizes = [-(-n // 4) * 4 for n in sizes]  # each part 16-byte aligned
+        parts = torch.zeros(sum(sizes), dtype=torch.float32, device=dev).split(sizes)
+        dpb, dqkvb, dtable, dln_w, dln_b = (t if n else None for t, n in zip(parts, sizes))
+        if dpb is not None:
+            dpb = dpb[:C]
+        if dqkvb is not None:
+            dqkvb = dqkvb[:3 * C]
+        if dtable is not None:
+            dtable = dtable[:table.numel()].view(table.shape)
+        if dln_w is not None:
+            dln_w = dln_w[:C]
+        if dln_b is not None:
+            dln_b = dln_b[:C]
+        grad = dy.contiguous().view(geom.batch, geom.height, geom.width, C)
+        if p_dtype != grad.dtype:  # bf16 windows, fp32 output
+            dp = kernels.swin_partition(grad, geom, out_dtype=p_dtype, column_sums=dpb)
+        else:
+            dp = kernels.swin_partition(grad, geom)
+        dp2 = dp.view(-1, C).to(pwc.dtype)
+        if need[10] and (dpb is None or dp.dtype != pwc.dtype):
+            dpb = dp2.sum(0, dtype=torch.float32)
+        dpw = weight_grad(dp2, oc.reshape(-1, C)).to(pw_dtype) if need[9] else None
+        dq = dk = dv = dqb = dkb = dvb = dx = None
+        if any(need[:9]) or need[11]:
+            _check_backward(qkv[..., :C], num_heads, (geom.window, geom.window), None)
+            do = _input_grad(dp2, pwc).view(oc.shape).to(qkv.dtype)
+            dqkv = torch.empty_like(qkv)
+            kernels.window_attention_backward(
+                qkv[..., :C], qkv[..., C:2 * C], qkv[..., 2 * C:], do.contiguous(), num_heads,
+                (geom.window, geom.window), scale, bias_table=table, mask=mask, dq=dqkv[..., :C],
+                dk=dqkv[..., C:2 * C], dv=dqkv[..., 2 * C:], dbias=dtable, column_sums=dqkvb)
+            dqkv2 = dqkv.view(-1, 3 * C)
+            if any(need[3:6]):
+                dw = weight_grad(dqkv2, xw.reshape(-1, C)).to(w_dtype)
+                dq, dk, dv = (dw[i * C:(i + 1) * C] if need[3 + i] else None for i in range(3))
+            if b_dtype is not None and any(need[6:9]):
+                db = (dqkvb if dqkvb is not None else dqkv2.sum(0, dtype=torch.float32)).to(b_dtype)
+                dqb, dkb, dvb = (db[i * C:(i + 1) * C] if need[6 + i] else None for i in range(3))
+            if any(need[:3]):
+                dxw = _input_grad(dqkv2, wc).view(xw.shape).to(win_dtype)
+                # The residual's gradient is added in the LayerNorm backward's kernel.
+                dx = kernels.swin_partition_ln_backward(
+                    dxw.contiguous(), x, geom, ln_w, eps, dresidual=grad.to(x.dtype) if need[0] else None,
+                    dweight=dln_w, dbias=dln_b)
+        cast = lambda g, t: None if g is None else g.to(t)  # noqa: E731
+        return (dx if need[0] else None, None if dln_w is None else dln_w.to(ln_w.dtype),
+                None if dln_b is None else dln_b.to(ln_b.dtype), dq, dk, dv, dqb, dkb, dvb, dpw, cast(dpb, pb_dtype),
+                None if dtable is None else dtable.to(table.dtype), None, None, None, None, None)
+
+
+def attention_half(x: torch.Tensor, geom: WindowGeometry, norm: torch.nn.LayerNorm, attn: torch.nn.Module,
+                   mask: MaskArg) -> torch.Tensor:
+    """The attention half-block on x [B, H, W, C] with gradients (see
+    :class:`_AttentionHalf`); ``attn``: a WindowAttention of plain Linears with
+    a biased proj."""
+    q, k, v, proj = attn.q_linear, attn.k_linear, attn.v_linear, attn.proj
+    return _AttentionHalf.apply(x, norm.weight, norm.bias, q.weight, k.weight, v.weight, q.bias, k.bias, v.bias,
+                                proj.weight, proj.bias, attn._table(), geom, norm.eps, attn.num_heads, attn.scale, mask)

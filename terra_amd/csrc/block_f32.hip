@@ -44,6 +44,9 @@ struct BlockF32Params {
   const float* b_proj;       // [96] or NULL
   const float* bias_table;   // [169][3] or NULL
   const uint64_t* land_bits; // [land_windows] or NULL
+  float* keep_xn;            // kKeep: window tokens [B * nWe, 49, 96], q | k | v
+  float* keep_qkv;           // [B * nWe, 49, 288] and attention output [B * nWe, 49,
+  float* keep_o;             // 96] for the backward
   int32_t land_windows;
   int32_t layernorm, shift_mask;
   float eps, scale_l2e, mask_l2e;
@@ -92,6 +95,7 @@ __device__ __forceinline__ void rows_product(const f32x4 (&w)[6], const float* r
   }
 }
 
+template <bool kKeep>
 __global__ __launch_bounds__(kFThreads) __attribute__((amdgpu_waves_per_eu(3, 3)))
 void block_f32_kernel(const BlockF32Params p) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -154,6 +158,7 @@ void block_f32_kernel(const BlockF32Params p) {
     const bool use_shift = p.shift_mask && (((int)wr + 2) * kFWs > p.Hp || ((int)wc + 2) * kFWs > p.Wp);
     const uint64_t land =
         p.land_bits != nullptr ? p.land_bits[((int64_t)b * p.nWe + wl) % p.land_windows] : 0ull;
+    const int64_t row0 = ((int64_t)b * p.nWe + wl) * kFN;  // kKeep: the window's first token row
     if (t < 64) {  // waves 0 .. 7
       float sum = 0.f;
 #pragma unroll
@@ -181,6 +186,7 @@ void block_f32_kernel(const BlockF32Params p) {
           for (int e = 0; e < 4; ++e) o[e] = (v[c][e] - mean) * rstd * gm[e] + bt[e];
         }
         if (gtok < 0) o = f32x4{0.f, 0.f, 0.f, 0.f};  // frame padding and rows 49 .. 63
+        if (kKeep && t < kFN) *reinterpret_cast<f32x4*>(p.keep_xn + (row0 + t) * kFC + c0) = o;
         *reinterpret_cast<f32x4*>(s.xn + t * kFPitch + c0) = o;
       }
       if (sub == 0) {
@@ -205,6 +211,8 @@ void block_f32_kernel(const BlockF32Params p) {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const int tok = 16 * (2 * tp + j) + c16;
+        if (kKeep && tok < kFN)
+          *reinterpret_cast<f32x4*>(p.keep_qkv + (row0 + tok) * (3 * kFC) + 16 * ft + 4 * g) = acc[j];
         if (part == 2) {  // uniform
 #pragma unroll
           for (int r = 0; r < 4; ++r) s.vt[(f + r) * kFVPitch + tok] = acc[j][r];
@@ -291,8 +299,11 @@ void block_f32_kernel(const BlockF32Params p) {
             o[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[ct][e], st[jt][e], o[ct], 0, 0, 0);
       }
 #pragma unroll
-      for (int ct = 0; ct < 2; ++ct)
-        *reinterpret_cast<f32x4*>(s.xn + i * kFPitch + 32 * h + 16 * ct + 4 * g) = o[ct] * inv;
+      for (int ct = 0; ct < 2; ++ct) {
+        const f32x4 v = o[ct] * inv;
+        *reinterpret_cast<f32x4*>(s.xn + i * kFPitch + 32 * h + 16 * ct + 4 * g) = v;
+        if (kKeep && i < kFN) *reinterpret_cast<f32x4*>(p.keep_o + (row0 + i) * kFC + 32 * h + 16 * ct + 4 * g) = v;
+      }
     }
     __syncthreads();
     // ---- proj + residual ------------------------------------------------------
@@ -314,16 +325,25 @@ void block_f32_kernel(const BlockF32Params p) {
   }
 }
 
-}  // namespace
-}  // namespace terra
+template <bool kKeep>
+int launch_block_f32(const BlockF32Params& p, hipStream_t s) {
+  constexpr int lds = (int)sizeof(BlockF32Lds);
+  static_assert(lds <= 160 * 1024, "LDS");
+  auto kern = block_f32_kernel<kKeep>;
+  static const hipError_t attr =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (attr != hipSuccess) return fail(TERRA_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(attr));
+  constexpr int kCus = 256;  // one workgroup per CU
+  kern<<<p.units < kCus ? p.units : kCus, kFThreads, lds, s>>>(p);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(TERRA_ERR_LAUNCH, "fp32 block kernel launch failed: %s", hipGetErrorString(e));
+  return TERRA_OK;
+}
 
-using namespace terra;
-
-extern "C" int terra_swin_block_f32_fwd(const float* x, float* y, const terra_swin_block_desc* desc,
-                                        const float* ln_gamma, const float* ln_beta, const float* qkv_weight,
-                                        const float* qkv_bias, const float* proj_weight, const float* proj_bias,
-                                        const float* bias_table, const uint64_t* land_bits, void* stream) {
-  clear_error();
+// keep: the training entry's three outputs, or NULL.
+int block_f32(const float* x, float* y, float* const* keep, const terra_swin_block_desc* desc, const float* ln_gamma,
+              const float* ln_beta, const float* qkv_weight, const float* qkv_bias, const float* proj_weight,
+              const float* proj_bias, const float* bias_table, const uint64_t* land_bits, void* stream) {
   if (desc == nullptr) return fail(TERRA_ERR_NULL, "desc is NULL");
   if (x == nullptr || y == nullptr || qkv_weight == nullptr || proj_weight == nullptr)
     return fail(TERRA_ERR_NULL, "x, y, qkv_weight and proj_weight must be non-NULL");
@@ -389,14 +409,41 @@ extern "C" int terra_swin_block_f32_fwd(const float* x, float* y, const terra_sw
   p.units = (int32_t)units;
   p.fd_frame = FastDiv((uint32_t)frame_windows);
   p.fd_nWw = FastDiv((uint32_t)dims.nWw);
-  constexpr int lds = (int)sizeof(BlockF32Lds);
-  static_assert(lds <= 160 * 1024, "LDS");
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(block_f32_kernel),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  if (attr != hipSuccess) return fail(TERRA_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(attr));
-  constexpr int kCus = 256;  // one workgroup per CU
-  block_f32_kernel<<<p.units < kCus ? p.units : kCus, kFThreads, lds, static_cast<hipStream_t>(stream)>>>(p);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail(TERRA_ERR_LAUNCH, "fp32 block kernel launch failed: %s", hipGetErrorString(e));
-  return TERRA_OK;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (keep == nullptr) return launch_block_f32<false>(p, s);
+  // A pad window's rows belong to the kept tensors but are not computed here.
+  if (p.valid_end > 0) return fail(TERRA_ERR_UNSUPPORTED, "the training form needs every emitted window valid");
+  for (int i = 0; i < 3; ++i) {
+    if (keep[i] == nullptr) return fail(TERRA_ERR_NULL, "the kept tensors must be non-NULL");
+    if (((uintptr_t)keep[i] & 15u) != 0) return fail(TERRA_ERR_ALIGN, "tensors must be 16-byte aligned");
+  }
+  p.keep_xn = keep[0];
+  p.keep_qkv = keep[1];
+  p.keep_o = keep[2];
+  return launch_block_f32<true>(p, s);
+}
+
+}  // namespace
+}  // namespace terra
+
+using namespace terra;
+
+extern "C" int terra_swin_block_f32_fwd(const float* x, float* y, const terra_swin_block_desc* desc,
+                                        const float* ln_gamma, const float* ln_beta, const float* qkv_weight,
+                                        const float* qkv_bias, const float* proj_weight, const float* proj_bias,
+                                        const float* bias_table, const uint64_t* land_bits, void* stream) {
+  clear_error();
+  return block_f32(x, y, nullptr, desc, ln_gamma, ln_beta, qkv_weight, qkv_bias, proj_weight, proj_bias, bias_table,
+                   land_bits, stream);
+}
+
+extern "C" int terra_swin_block_f32_train(const float* x, float* y, float* windows, float* qkv, float* o,
+                                          const terra_swin_block_desc* desc, const float* ln_gamma,
+                                          const float* ln_beta, const float* qkv_weight, const float* qkv_bias,
+                                          const float* proj_weight, const float* proj_bias, const float* bias_table,
+                                          const uint64_t* land_bits, void* stream) {
+  clear_error();
+  float* const keep[3] = {windows, qkv, o};
+  return block_f32(x, y, keep, desc, ln_gamma, ln_beta, qkv_weight, qkv_bias, proj_weight, proj_bias, bias_table,
+                   land_bits, stream);
 }

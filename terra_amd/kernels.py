@@ -671,6 +671,36 @@ def swin_block_f32(x: torch.Tensor, geom: WindowGeometry, num_heads: int, scale:
         layernorm, bias_table, shift_mask, land_bits, mask_value, False))(x, out)
 
 
+def swin_block_f32_train(x: torch.Tensor, geom: WindowGeometry, num_heads: int, scale: float,
+                         qkv_weight: torch.Tensor, qkv_bias: Optional[torch.Tensor], proj_weight: torch.Tensor,
+                         proj_bias: Optional[torch.Tensor], ln_weight: Optional[torch.Tensor],
+                         ln_bias: Optional[torch.Tensor], ln_eps: float, bias_table: Optional[torch.Tensor],
+                         mask: Optional[WindowMask]):
+    """:func:`swin_block_f32` that also returns what the backward reads:
+    (y, LayerNorm windows, q | k | v, attention output), the last three over
+    the emitted windows [B_, 49, .] (terra_swin_block_f32_train).  None where
+    it does not serve the call: other shapes, dtypes or alignments, a
+    valid-window range, an explicit mask."""
+    shift = mask.shift if mask is not None else None
+    land = mask.land_bits if mask is not None else None
+    tensors = (x, qkv_weight, proj_weight, qkv_bias, proj_bias, ln_weight, ln_bias, bias_table)
+    if not swin_block_f32_supported(x, geom, num_heads) or geom.valid is not None or geom.batch == 0 \
+            or isinstance(shift, torch.Tensor) or any(
+                t is not None and (t.dtype != torch.float32 or not t.is_contiguous() or t.data_ptr() % 16)
+                for t in tensors):
+        return None
+    y, n = torch.empty_like(x), geom.num_windows
+    kept = tuple(torch.empty((n, 49, c), dtype=x.dtype, device=x.device) for c in (96, 288, 96))
+    given = (qkv_weight, qkv_bias, proj_weight, proj_bias, ln_weight, ln_bias, bias_table, land)
+    launch = _BlockLaunch(x, geom, num_heads, scale, *given[:6], ln_eps, True, bias_table, shift is not None, land,
+                          MASK_VALUE, False)
+    with torch.cuda.device(x.device):
+        st = _lib.load().terra_swin_block_f32_train(_ptr(x), _ptr(y), *map(_ptr, kept), ctypes.byref(launch.desc),
+                                                    *launch.ptrs, _stream(x.device))
+    _lib.check(st, "terra_swin_block_f32_train")
+    return (y, *kept)
+
+
 # Prepared launches, keyed by the ids of the parameter tensors, the call's
 # scalars and the activation shape.  An entry holds weak references to those
 # tensors with their data pointers and sizes, and serves a call only while

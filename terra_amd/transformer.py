@@ -160,6 +160,24 @@ class SequentialSwinTransformer(torch.nn.Module):
             kernels.autocast_bf16(x) and all(l.weight.dtype == torch.float32 for l in lins))
         return w_ok and attn.q_linear.bias is not None
 
+    def _one_function(self, x: torch.Tensor) -> bool:
+        """A training call runs as one autograd function: the fused LayerNorm
+        gather, q/k/v and proj plain Linears of one dtype each, proj biased,
+        a gradient needed upstream of the attention core.  Anything else keeps
+        the chain of functions, and so do calls large enough to be bound by
+        the GPU, since the chain frees its saved tensors one by one in the
+        backward (autocast step, C = 192, chain / one function: 2^20.6
+        elements 770 / 696 us and 24 / 39 MB at the peak, 2^23.6 738 / 668
+        and 192 / 312, 2^25.6 1007 / 1021 and 768 / 1248)."""
+        attn = self.attn
+        lins = (attn.q_linear, attn.k_linear, attn.v_linear, attn.proj)
+        return (config.use_layernorm and self._fusable_norm(x.dtype) and x.numel() <= 1 << 24
+                and type(attn) is WindowAttention
+                and autograd._needs_grad(x, self.norm1.weight, self.norm1.bias, *(l.weight for l in lins[:3]))
+                and all(type(l) is torch.nn.Linear for l in lins) and attn.proj.bias is not None
+                and len({l.weight.dtype for l in lins[:3]}) == 1
+                and len({None if l.bias is None else l.bias.dtype for l in lins[:3]}) == 1)
+
     def _block_f32_args(self, x: torch.Tensor, geom: WindowGeometry) -> Optional[dict]:
         """Arguments of kernels.swin_block_f32 where the whole half-block runs
         as one fp32 kernel, else None: fp32 activations and parameters outside
@@ -251,6 +269,8 @@ class SequentialSwinTransformer(torch.nn.Module):
         # Training: the partition / reverse permutations and the LayerNorm
         # with their HIP backward kernels.
         training = torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in self.parameters()))
+        if training and self._one_function(grid):
+            return autograd.attention_half(grid, geom, self.norm1, self.attn, self.window_mask(geom)).view(B, H * W, C)
         link = None
         if config.use_layernorm and not training and self._fusable_norm(grid.dtype):
             n = self.norm1

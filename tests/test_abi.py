@@ -531,3 +531,18 @@ def test_block_f32_rejects_bad_arguments():
     assert call(y=ctypes.c_void_p((2 << 28) + 4)) == -4 and call(y=ctypes.c_void_p((1 << 28) + 64)) == -3
     assert call(land=p(5)) == -3 and "land_windows" in L.last_error()
     assert L.load().terra_swin_block_f32_fwd(p(1), p(2), None, None, None, p(3), None, p(4), None, None, None, None) == -1
+
+
+def test_block_f32_train_rejects_bad_kept_tensors():
+    p = lambda a: ctypes.c_void_p(a << 28)  # noqa: E731
+
+    def call(xn=p(5), qkv=p(6), o=p(7), **geom):
+        d = L.SwinBlockDesc()
+        d.geom = _geom(**dict(dict(height=14, width=21, channels=96, window=7), **geom))
+        d.heads, d.scale, d.ln_eps, d.layernorm = 3, 0.1, 1e-5, 1
+        return L.load().terra_swin_block_f32_train(p(1), p(2), xn, qkv, o, ctypes.byref(d), None, None, p(3), None,
+                                                   p(4), None, None, None, None)
+
+    assert call(xn=None) == -1 and call(qkv=None) == -1 and call(o=None) == -1
+    assert call(o=ctypes.c_void_p((7 << 28) + 8)) == -4
+    assert call(valid_begin=1, valid_end=4) == -5

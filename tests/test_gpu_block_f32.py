@@ -21,6 +21,7 @@ CASES = [
     (3, 21, 35, 1, (0, 0, 0, 0), 0, None, None, True, True, False),      # land and shift, no bias table
     (2, 25, 31, 1, (2, 1, 1, 3), 0, None, None, True, True, True),       # frame padding on every side
     (2, 21, 28, 1, (0, 7, 0, 0), 0, 3, (2, 9), True, True, True),        # slab: rows not emitted, pad windows
+    (2, 21, 28, 1, (0, 7, 0, 0), 1, 2, None, False, True, True),         # slab without pad windows
     (1, 140, 161, 1, (0, 0, 0, 0), 0, None, None, True, True, True),     # 460 windows: two per workgroup
 ]
 
@@ -87,3 +88,37 @@ def test_block_f32_in_place_without_layernorm_and_routes(dev, monkeypatch):
         y = plain(xd)
         plain.use_fused_block = False
         assert rel_norm(y - xd, plain(xd) - xd) <= 1e-5
+
+
+@pytest.mark.parametrize("case", [c for c in CASES if c[7] is None])
+def test_block_f32_train_outputs(dev, case):
+    """terra_swin_block_f32_train: the result bits of the inference kernel, and
+    the LayerNorm windows, q | k | v and attention output of the staged kernels
+    over every emitted window."""
+    blk, _, x = _block(dev, case)
+    B, H, W = case[:3]
+    geom, xd, attn = blk.geometry(B), x.to(dev).view(B, H, W, 96), blk.attn
+    n, lins, mask = blk.norm1, (attn.q_linear, attn.k_linear, attn.v_linear), blk.window_mask(geom)
+    with torch.no_grad():
+        w, b = torch.cat([l.weight for l in lins]), torch.cat([l.bias for l in lins])
+        y, xn, qkv, o = kernels.swin_block_f32_train(xd, geom, 3, attn.scale, w, b, attn.proj.weight, attn.proj.bias,
+                                                     n.weight, n.bias, n.eps, attn._table(), mask)
+        assert torch.equal(y.view(B, H * W, 96), blk(xd.view(B, H * W, 96)))
+        xs = kernels.swin_partition_ln(xd, geom, n.weight, n.bias, n.eps)
+        qs = torch.nn.functional.linear(xs, w, b)
+        os = kernels.window_attention(qs[..., :96], qs[..., 96:192], qs[..., 192:], 3, (7, 7), attn.scale,
+                                      bias_table=attn._table(), mask=mask)
+    for got, want in ((xn, xs), (qkv, qs), (o, os)):
+        assert got.shape == want.shape and rel_norm(got, want) <= 1e-5
+
+
+def test_block_f32_train_serves_only_its_calls(dev):
+    blk, _, x = _block(dev, CASES[6])  # a valid-window range
+    n, attn, xd = blk.norm1, blk.attn, x.to(dev).view(2, 21, 28, 96)
+    w, geom = torch.zeros(288, 96, device=dev), blk.geometry(2)
+    args = (w, None, attn.proj.weight, None, n.weight, n.bias, n.eps, None, None)
+    assert kernels.swin_block_f32_train(xd, geom, 3, 1.0, *args) is None
+    whole = kernels.WindowGeometry(batch=2, height=21, width=28, channels=96, window=7)
+    assert kernels.swin_block_f32_train(xd.half(), whole, 3, 1.0, *args) is None
+    assert kernels.swin_block_f32_train(xd, whole, 3, 1.0, w.t().contiguous().t(), *args[1:]) is None
+    assert kernels.swin_block_f32_train(xd, whole, 4, 1.0, *args) is None

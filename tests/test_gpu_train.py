@@ -18,8 +18,9 @@ import torch
 
 from helpers import gain_block, params_of
 from oracle import swin_oracle as so
-from terra_amd import kernels, workloads
+from terra_amd import autograd, kernels, workloads
 from terra_amd.kernels import WindowGeometry
+from terra_amd.transformer import SequentialSwinTransformer
 
 pytestmark = pytest.mark.gpu
 
@@ -632,3 +633,80 @@ def test_training_accepts_parameters_at_any_offset(dev):
 
     for a, b in zip(grads(0), grads(1)):
         assert _normwise(a, b) <= 1e-6
+
+
+# (dtype, autocast, window, C, heads, frozen parameters, x needs a gradient, bias table, q/k/v bias)
+HALF_CASES = [
+    (torch.float32, False, 7, 96, 3, (), True, True, True),
+    (torch.float32, False, 7, 96, 3, ("q_linear.weight", "k_linear.bias", "norm1.bias", "proj.bias"), False, False, True),
+    (torch.float32, False, 8, 192, 6, ("proj.weight", "relative_position_bias_table"), True, True, False),
+    (torch.float32, True, 8, 192, 6, ("norm1.weight",), True, True, True),
+    (torch.bfloat16, False, 8, 128, 4, (), True, True, True),
+    (torch.float32, True, 7, 96, 3, ("q_linear", "k_linear", "v_linear", "norm1", "table"), True, False, True),
+]
+
+
+@pytest.mark.parametrize("case", HALF_CASES)
+def test_attention_half_matches_the_chain_of_functions(dev, case, monkeypatch):
+    """The attention half-block's training step as one function against the
+    chain of partition, Linear, core, Linear and reverse it replaces (masked,
+    shifted, padded frame): outputs and gradients agree to the rounding of the
+    compute dtype, and the same tensors get one."""
+    dtype, amp, ws, C, heads, frozen, xgrad, table, qkv_bias = case
+    blk = SequentialSwinTransformer(layer_idx=1, height=3 * ws - 2, width=4 * ws, embedding_dim=C, window_size=ws,
+                                    num_heads=heads, use_relative_position_bias=table, pad=(1, 1, 0, 0),
+                                    land_mask=workloads.land_mask(3 * ws - 2, 4 * ws, seed=81))
+    workloads.init_block_params(blk, 1)
+    blk = gain_block(blk)
+    if not qkv_bias:
+        for lin in (blk.attn.q_linear, blk.attn.k_linear, blk.attn.v_linear):
+            lin.bias = None
+    blk = blk.to(dev, dtype)
+    for n, p in blk.named_parameters():
+        p.requires_grad_(not any(f in n for f in frozen))
+    x0 = workloads.activations((2, (3 * ws - 2) * 4 * ws, C), 620).to(dev, dtype)
+    gy = workloads.activations(tuple(x0.shape), 621).to(dev, dtype)
+    calls = []
+    orig = autograd.attention_half
+    monkeypatch.setattr(autograd, "attention_half", lambda *a: calls.append(1) or orig(*a))
+
+    def step():
+        x = x0.clone().requires_grad_(xgrad)
+        blk.zero_grad(set_to_none=True)
+        with torch.amp.autocast("cuda", dtype=torch.bfloat16, enabled=amp):
+            y = blk(x)
+        y.backward(gy)
+        return {"y": y.detach(), "x": x.grad, **{n: p.grad for n, p in blk.named_parameters()}}
+
+    got = step()
+    assert calls == [1]
+    monkeypatch.setattr(blk, "_one_function", lambda x: False, raising=False)
+    want = step()
+    assert calls == [1]
+    # One rounding of the compute dtype and its sums' order on either side.
+    tol = 2.0 ** -8 if amp or dtype == torch.bfloat16 else 1e-5
+    for name, b in want.items():
+        a = got[name]
+        assert (a is None) == (b is None)
+        if b is not None:
+            assert a.dtype == b.dtype and a.shape == b.shape
+            # k's bias shifts a query's logits alike, so its exact gradient is
+            # zero: what is left is rounding, on the scale of q's and v's.
+            scale = want["attn.v_linear.bias"] if name == "attn.k_linear.bias" else b
+            assert (a.double() - b.double()).norm() <= tol * scale.double().norm(), name
+
+
+def test_attention_half_keeps_the_chain_for_other_calls(dev, monkeypatch):
+    """A subclassed projection, and a call with only proj trainable, stay on
+    the chain."""
+    monkeypatch.setattr(autograd, "attention_half", None)
+    for change in ("subclass", "frozen"):
+        blk = SequentialSwinTransformer(layer_idx=0, height=14, width=14, embedding_dim=96, window_size=7, num_heads=3)
+        if change == "subclass":
+            blk.attn.q_linear.__class__ = type("L", (torch.nn.Linear,), {})
+        else:
+            blk.requires_grad_(False)
+            blk.attn.proj.requires_grad_(True)
+        blk = blk.to(dev)
+        blk(torch.randn(1, 196, 96, device=dev)).sum().backward()
+        assert blk.attn.proj.weight.grad is not None
