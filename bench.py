@@ -300,9 +300,11 @@ def main():
 
     # Events around the fused kernel on its launch stream (torch's current
     # stream, which the C ABI receives as its hipStream_t).
-    events = {"swin_block": [], "partition": [], "window_attention": [], "reverse": [], "proj_scatter": []}
-    names = ("swin_block", "swin_partition_ln", "window_attention", "swin_reverse", "linear_residual")
-    keys = ("swin_block", "partition", "window_attention", "reverse", "proj_scatter")
+    events = {"swin_block": [], "partition": [], "window_attention": [], "reverse": [], "proj_scatter": [],
+              "block_f32": []}
+    names = ("swin_block", "swin_partition_ln", "window_attention", "swin_reverse", "linear_residual",
+             "linear_scatter", "swin_block_f32")
+    keys = ("swin_block", "partition", "window_attention", "reverse", "proj_scatter", "proj_scatter", "block_f32")
     orig = {n: getattr(kernels, n) for n in names}
     recording = {"on": False}
     last_call = {}
@@ -406,7 +408,8 @@ def main():
         fused = bool(events["swin_block"])
         if args.config == "c3" and not fused:
             raise RuntimeError("the fused block kernel did not serve the benchmark step")
-        if fused:
+        fused_f32 = bool(events["block_f32"])  # c1
+        if fused or fused_f32:
             blk.use_fused_block = False  # the five-stage path, for comparison
             ms_five = run(max(5, args.steps // 2), 10)
             blk.use_fused_block = True
@@ -464,7 +467,7 @@ def main():
             iso["mlp"] = isolated_us("mlp")
         with torch.no_grad():
             mlp_gemm = (not mlp_fused) and mlp._gemm_path(y_blk)
-        if mlp_gemm:  # C = 1024: HIP LayerNorm, fc1 + GELU on the linear kernel, fc2 + x on hipBLASLt
+        if mlp_gemm:  # C = 1024: HIP LayerNorm, fc1 + GELU and fc2 + x on the linear kernel
             last_call["mlp_gemm"] = (mlp, (y_blk,), {})
             iso["mlp_gemm"] = isolated_us("mlp_gemm")
         mlp.use_fused_mlp = False
@@ -477,9 +480,9 @@ def main():
         # synthetic output gradient (no optimizer update).  The LayerNorms and
         # their backward, partition / reverse and the attention core with its
         # backward run on the HIP kernels (the Linear bias gradients summed
-        # inside the kernels that write the gradients); the projection, fc1 and
-        # fc2 GEMMs and their backward on hipBLASLt through torch.  Median of
-        # 10 steps after 3 warm-up steps (a step is 5-6 ms at c3).
+        # inside the kernels that write the gradients); the GEMMs on the linear
+        # and weight-gradient kernels where they serve the shape, else on
+        # hipBLASLt through torch.  Median of 10 steps after 3 warm-up steps.
         train = training_step_us(cfg, dev, warmup=3, reps=10) if has_bwd else None
     finally:
         for n in names:
@@ -592,7 +595,7 @@ def main():
                             f"{'/land' if cfg.land else ''} mask" if cfg.rel_bias or cfg.attn_mask else
                             " without relative-position bias or mask")
                          + ", proj, reverse+roll, "
-                         f"residual) {'as one fused kernel' if fused else 'through the five-stage path'}, "
+                         f"residual) {'as one fused kernel' if fused or fused_f32 else 'through the five-stage path'}, "
                          f"B={cfg.batch}, {cfg.height}x{cfg.width} tokens, C={C}, "
                          f"{cfg.heads} heads, window {cfg.window}, shift {cfg.shift}"
                          + (", ~30% land mask" if cfg.land else "")),
@@ -686,7 +689,7 @@ def main():
         t_mlp = iso["mlp"]
     elif mlp_gemm:
         res["mlp_half"] = {
-            "kernel": "HIP LayerNorm over the token rows + linear_kernel (fc1 + exact GELU epilogue) + hipBLASLt fc2 + x",
+            "kernel": "HIP LayerNorm over the token rows + linear_kernel (fc1 + exact GELU epilogue; fc2 + x epilogue)",
             "us": iso["mlp_gemm"],
             "TFLOP_s": mlp_flops / (iso["mlp_gemm"] * 1e-6) / 1e12,
             "mfma_frac": mlp_flops / (iso["mlp_gemm"] * 1e-6) / 1e12 / MFMA_BF16_PEAK_TFLOPS,

@@ -488,6 +488,15 @@ int terra_swin_linear_residual(const void* x, const void* residual, void* y,
                                const void* weight_packed, const float* bias,
                                const terra_swin_geom* geom, void* stream);
 
+/* terra_swin_linear_residual with a geometry (non-NULL) of any window size:
+ * rows = B * nW * window^2.
+ */
+int terra_swin_linear_scatter(const void* x, const void* residual, void* y,
+                              int dtype, int64_t rows,
+                              int in_features, int out_features,
+                              const void* weight_packed, const float* bias,
+                              const terra_swin_geom* geom, void* stream);
+
 /* terra_swin_pack_linear of a weight that still has to be cast or transposed
  * (the training step's linear layers): packs P [out_features, in_features]
  * (multiples of 16 and 32), P = weight (row-major [out, in]) or, transposed

@@ -62,6 +62,7 @@ EXPORTED_SYMBOLS = (
     "terra_swin_gelu_bwd",
     "terra_swin_linear",
     "terra_swin_linear_residual",
+    "terra_swin_linear_scatter",
     "terra_swin_linear_gelu_keep",
     "terra_swin_linear_gelu_bwd",
     "terra_swin_pack_weight",
@@ -242,6 +243,9 @@ def load() -> ctypes.CDLL:
                                           ctypes.c_int, vp]
         lib.terra_swin_linear_residual.restype = ctypes.c_int
         lib.terra_swin_linear_residual.argtypes = [vp, vp, vp, ctypes.c_int, i64, ctypes.c_int, ctypes.c_int, vp, vp,
+                                                   ctypes.POINTER(SwinGeom), vp]
+        lib.terra_swin_linear_scatter.restype = ctypes.c_int
+        lib.terra_swin_linear_scatter.argtypes = [vp, vp, vp, ctypes.c_int, i64, ctypes.c_int, ctypes.c_int, vp, vp,
                                                    ctypes.POINTER(SwinGeom), vp]
         lib.terra_swin_pack_weight.restype = ctypes.c_int
         lib.terra_swin_pack_weight.argtypes = [vp, vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp]

@@ -80,7 +80,7 @@ static_assert(kLinGeluOff + kGeluBytes <= 160 * 1024, "LDS");
 
 // LDS of each epilogue past the stages: bias (or, gelu-bwd, the column sums),
 // then the GELU or slope table.
-enum { kEpiStore = 0, kEpiGelu = 1, kEpiResidual = 2, kEpiScatter = 3, kEpiGeluKeep = 4, kEpiGeluBwd = 5 };
+enum { kEpiStore = 0, kEpiGelu = 1, kEpiResidual = 2, kEpiScatter = 3, kEpiGeluKeep = 4, kEpiGeluBwd = 5, kEpiScatterAny = 6 };
 
 static_assert(kLinGeluOff + kSlopeTabBytes <= 160 * 1024, "LDS");
 
@@ -105,6 +105,8 @@ struct LinParams {
   // kEpiScatter: window-order rows of 8x8 windows -> grid tokens
   int32_t H, W, Hp, Wp, shift_h, shift_w, pad_top, pad_left;
   FastDiv fd_nWe, fd_nWw;  // emitted windows per image, windows per frame row
+  FastDiv fd_wn, fd_ws;    // kEpiScatterAny: tokens per window, window width
+  int32_t ws;
 };
 
 // This lane's index in its wave, computed where it is used (a volatile asm
@@ -122,16 +124,25 @@ __device__ __forceinline__ int lin_lane() {
 __device__ __forceinline__ int lin_swz(int row) { return (row ^ ((row >> 3) & 1)) & 7; }
 __device__ __forceinline__ int lin_slot(int row, int c) { return row * 8 + (c ^ lin_swz(row)); }
 
-// Grid token of window-order row m (window m / 64, token m % 64 of an 8x8
-// window), or -1 for a frame-padding token: the position the partition read
-// the row from (pad, then a cyclic shift by (shift_h, shift_w)).
+// Rows of other windows go through kEpiScatterAny (window 32, 156672 x 1024: the
+// block 2042 -> 1971 us against the library's product and the reverse kernel).
+// Grid token of window-order row m (8x8 windows: window m / 64, token m % 64;
+// kAny: windows of any size), or -1 for a frame-padding token: the position the
+// partition read the row from (pad, then a cyclic shift by (shift_h, shift_w)).
+template <bool kAny>
 __device__ __forceinline__ int64_t lin_grid_row(const LinParams& p, int m) {
-  const uint32_t w = (uint32_t)m >> 6, s = (uint32_t)m & 63u;
+  uint32_t w = (uint32_t)m >> 6, s = (uint32_t)m & 63u;
+  uint32_t sr = s >> 3, sc = s & 7u, ws = 8u;
+  if constexpr (kAny) {
+    ws = (uint32_t)p.ws;
+    p.fd_wn.divmod((uint32_t)m, w, s);
+    p.fd_ws.divmod(s, sr, sc);
+  }
   uint32_t b, wl, wr, wc;
   p.fd_nWe.divmod(w, b, wl);
   p.fd_nWw.divmod(wl, wr, wc);
-  int ph = (int)(wr * 8u + (s >> 3)) + p.shift_h;
-  int pw = (int)(wc * 8u + (s & 7u)) + p.shift_w;
+  int ph = (int)(wr * ws + sr) + p.shift_h;
+  int pw = (int)(wc * ws + sc) + p.shift_w;
   if (ph >= p.Hp) ph -= p.Hp;
   if (pw >= p.Wp) pw -= p.Wp;
   const int sh = ph - p.pad_top, sw = pw - p.pad_left;
@@ -389,7 +400,7 @@ void linear_kernel(const LinParams p) {
           o[j][i] = make_uint2(pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3]));
       __builtin_amdgcn_sched_barrier(0);  // the fp32 accumulators end here
     }
-    constexpr bool kScatter = kEpi == kEpiScatter;
+    constexpr bool kScatter = kEpi == kEpiScatter || kEpi == kEpiScatterAny;
     constexpr bool kRes = kEpi == kEpiResidual || kScatter;
     const int64_t tile0 = kScatter ? 0 : (int64_t)m0 * p.y_ld;
     const int left = p.M - m0 < kLinT ? p.M - m0 : kLinT;
@@ -405,7 +416,7 @@ void linear_kernel(const LinParams p) {
       int64_t orow = row;
       ok[j] = row < left;
       if constexpr (kScatter) {
-        orow = ok[j] ? lin_grid_row(p, m0 + row) : -1;
+        orow = ok[j] ? lin_grid_row<kEpi == kEpiScatterAny>(p, m0 + row) : -1;
         ok[j] = orow >= 0;  // frame padding
       }
       const uint32_t col = (uint32_t)(f0 + 128 * wm + 8 * g) * 2u;
@@ -565,8 +576,8 @@ int launch_linear(const LinParams& p, hipStream_t s) {
 // MiB and more (the other epilogues' rows are contiguous, so never those).
 template <int kEpi>
 int dispatch_linear(const LinParams& p, hipStream_t s) {
-  if constexpr (kEpi == kEpiStore || kEpi == kEpiGelu || kEpi == kEpiScatter) {
-    const int64_t bytes = kEpi == kEpiScatter ? p.y_bytes : (int64_t)kLinT * p.y_ld;
+  if constexpr (kEpi == kEpiStore || kEpi == kEpiGelu || kEpi == kEpiScatter || kEpi == kEpiScatterAny) {
+    const int64_t bytes = kEpi == kEpiScatter || kEpi == kEpiScatterAny ? p.y_bytes : (int64_t)kLinT * p.y_ld;
     if (bytes >= (int64_t)kLinDrop) return launch_linear<kEpi, true>(p, s);
   }
   return launch_linear<kEpi, false>(p, s);
@@ -637,10 +648,10 @@ extern "C" int terra_swin_linear(const void* x, void* y, int dtype, int64_t rows
   return epilogue == TERRA_LINEAR_GELU ? dispatch_linear<kEpiGelu>(p, s) : dispatch_linear<kEpiStore>(p, s);
 }
 
-extern "C" int terra_swin_linear_residual(const void* x, const void* residual, void* y, int dtype, int64_t rows,
-                                          int in_features, int out_features, const void* weight_packed,
-                                          const float* bias, const terra_swin_geom* geom, void* stream) {
-  clear_error();
+// any_window: the entry takes windows of every size, else 8x8 ones.
+static int linear_residual(const void* x, const void* residual, void* y, int dtype, int64_t rows, int in_features,
+                           int out_features, const void* weight_packed, const float* bias,
+                           const terra_swin_geom* geom, bool any_window, void* stream) {
   LinParams p{};
   const int st = lin_validate(x, weight_packed, bias, y, dtype, rows, in_features, out_features, in_features,
                               out_features, &p);
@@ -654,7 +665,8 @@ extern "C" int terra_swin_linear_residual(const void* x, const void* residual, v
     const int gs = validate_geom(geom, &dims);
     if (gs != TERRA_OK) return gs;
     const terra_swin_geom& q = *geom;
-    if (q.window != 8) return fail(TERRA_ERR_UNSUPPORTED, "the scatter epilogue needs 8x8 windows (got %d)", q.window);
+    if (q.window != 8 && !any_window)
+      return fail(TERRA_ERR_UNSUPPORTED, "the scatter epilogue needs 8x8 windows (got %d)", q.window);
     if (q.channels != out_features)
       return fail(TERRA_ERR_SHAPE, "geom channels (%d) must equal out_features (%d)", q.channels, out_features);
     // Every grid token must come from exactly one emitted window, so that the
@@ -662,14 +674,18 @@ extern "C" int terra_swin_linear_residual(const void* x, const void* residual, v
     if (q.win_row_begin != 0 || dims.rows != dims.nWh || q.valid_end > 0)
       return fail(TERRA_ERR_UNSUPPORTED,
                   "the scatter epilogue needs every window of the frame emitted (no window-row or valid-window range)");
-    if (rows != (int64_t)q.batch * dims.nWe * 64)
+    const int64_t wn = (int64_t)q.window * q.window;
+    if (rows != (int64_t)q.batch * dims.nWe * wn)
       return fail(TERRA_ERR_SHAPE, "rows (%lld) must be the window tokens of the frame (%lld)", (long long)rows,
-                  (long long)((int64_t)q.batch * dims.nWe * 64));
+                  (long long)((int64_t)q.batch * dims.nWe * wn));
     out_rows = (int64_t)q.batch * q.height * q.width;
     p.H = q.height; p.W = q.width; p.Hp = (int32_t)dims.Hp; p.Wp = (int32_t)dims.Wp;
     p.shift_h = q.shift_h; p.shift_w = q.shift_w; p.pad_top = q.pad_top; p.pad_left = q.pad_left;
     p.fd_nWe = FastDiv((uint32_t)dims.nWe);
     p.fd_nWw = FastDiv((uint32_t)dims.nWw);
+    p.ws = q.window;
+    p.fd_wn = FastDiv((uint32_t)wn);
+    p.fd_ws = FastDiv((uint32_t)q.window);
   }
   const int64_t xb = rows * (int64_t)in_features * 2, yb = out_rows * (int64_t)out_features * 2;
   if (rows > 0 && lin_overlap(x, xb, y, yb)) return fail(TERRA_ERR_SHAPE, "y overlaps x");
@@ -678,7 +694,26 @@ extern "C" int terra_swin_linear_residual(const void* x, const void* residual, v
   if (rows == 0) return TERRA_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
   p.y_bytes = yb;
-  return geom != nullptr ? dispatch_linear<kEpiScatter>(p, s) : dispatch_linear<kEpiResidual>(p, s);
+  if (geom == nullptr) return dispatch_linear<kEpiResidual>(p, s);
+  // 8x8 windows split a row number by shifts, the others by two more divisions.
+  return p.ws == 8 ? dispatch_linear<kEpiScatter>(p, s) : dispatch_linear<kEpiScatterAny>(p, s);
+}
+
+extern "C" int terra_swin_linear_residual(const void* x, const void* residual, void* y, int dtype, int64_t rows,
+                                          int in_features, int out_features, const void* weight_packed,
+                                          const float* bias, const terra_swin_geom* geom, void* stream) {
+  clear_error();
+  return linear_residual(x, residual, y, dtype, rows, in_features, out_features, weight_packed, bias, geom, false,
+                         stream);
+}
+
+extern "C" int terra_swin_linear_scatter(const void* x, const void* residual, void* y, int dtype, int64_t rows,
+                                         int in_features, int out_features, const void* weight_packed,
+                                         const float* bias, const terra_swin_geom* geom, void* stream) {
+  clear_error();
+  if (geom == nullptr) return fail(TERRA_ERR_NULL, "geom must be non-NULL");
+  return linear_residual(x, residual, y, dtype, rows, in_features, out_features, weight_packed, bias, geom, true,
+                         stream);
 }
 
 extern "C" int terra_swin_linear_gelu_keep(const void* x, void* h, void* y, int dtype, int64_t rows, int in_features,

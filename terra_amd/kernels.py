@@ -918,6 +918,18 @@ def linear_residual(x: torch.Tensor, weight_packed: torch.Tensor, out_features: 
     proj + window_reverse + roll + shortcut (models/attention.py:281,
     models/utils.py:41-45, models/transformer.py:246, 296-298); ``residual`` /
     ``out`` are [B, H, W, C].  ``out`` may be ``residual``."""
+    return _linear_residual("terra_swin_linear_residual", x, weight_packed, out_features, residual, bias, geom, out)
+
+
+def linear_scatter(x: torch.Tensor, weight_packed: torch.Tensor, out_features: int, residual: torch.Tensor,
+                   geom: WindowGeometry, bias: Optional[torch.Tensor] = None,
+                   out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """:func:`linear_residual` with a geometry of any window size
+    (terra_swin_linear_scatter)."""
+    return _linear_residual("terra_swin_linear_scatter", x, weight_packed, out_features, residual, bias, geom, out)
+
+
+def _linear_residual(entry: str, x, weight_packed, out_features, residual, bias, geom, out) -> torch.Tensor:
     dev, code, k, rows = _linear_checks(x, weight_packed, out_features, bias)
     _require_device(x, residual)
     if geom is None:
@@ -939,10 +951,10 @@ def linear_residual(x: torch.Tensor, weight_packed: torch.Tensor, out_features: 
         return out.view(shape)
     c_geom = None if geom is None else geom.to_c()
     with torch.cuda.device(dev):
-        st = _lib.load().terra_swin_linear_residual(_ptr(x), _ptr(residual), _ptr(out), code, int(rows), int(k),
-                                                    int(out_features), _ptr(weight_packed), _ptr(bias),
-                                                    None if c_geom is None else ctypes.byref(c_geom), _stream(dev))
-    _lib.check(st, "terra_swin_linear_residual")
+        st = getattr(_lib.load(), entry)(_ptr(x), _ptr(residual), _ptr(out), code, int(rows), int(k),
+                                         int(out_features), _ptr(weight_packed), _ptr(bias),
+                                         None if c_geom is None else ctypes.byref(c_geom), _stream(dev))
+    _lib.check(st, entry)
     return out.view(shape)
 
 

@@ -4,13 +4,17 @@ The attention half of a Swin block on one GPU.  For bf16 activations and
 (window, heads, C) in kernels.BLOCK_SHAPES (8x8 windows with 6, 12 or 12 heads
 at C = 192, 384, 768; 7x7 windows with 4 heads at C = 128) the whole half-block is one HIP
 kernel (``kernels.swin_block``: gather + LayerNorm + q/k/v + attention + proj
-+ residual + scatter).  Otherwise:
++ residual + scatter), and for fp32 in kernels.BLOCK_F32_SHAPES (7x7 windows with
+3 heads at C = 96) too (``kernels.swin_block_f32``).  Otherwise:
 
     x -> [norm1 + roll(-s) + window partition]      one HIP gather
       -> q/k/v projection (one GEMM)                 hipBLASLt via torch
       -> fused window-attention core                 one HIP kernel
       -> proj                                        hipBLASLt via torch
       -> [window reverse + roll(+s) + residual add]  one HIP scatter
+
+with proj and the scatter in one linear-kernel launch where that serves the
+shape, and training through autograd (narrow projections on HIP kernels).
 
 Module construction, parameter and buffer names (``norm1``, ``attn.*``,
 ``attn_mask``) follow the reference so its checkpoints load.  The shift mask
@@ -125,14 +129,18 @@ class SequentialSwinTransformer(torch.nn.Module):
     def _proj_scatter(self, x_windows: torch.Tensor, shortcut: torch.Tensor, geom: WindowGeometry) -> bool:
         """Whether the output projection, the window reverse and the residual
         add can run as one linear-kernel launch: bf16 windows and shortcut,
-        8x8 windows, C a multiple of 256 (the kernel's feature tile; C = 1024
+        8x8 windows (others where the rows fill the chip: window 32, C =
+        1024, 156672 tokens 2042 -> 1971 us for the block, 16384 tokens 238 ->
+        225; window 7, C = 256, 117600 tokens 269 -> 244), C a multiple of 256 (the kernel's feature tile; C = 1024
         for TERRA's pretrain blocks), every window of the frame emitted, a
         biased nn.Linear proj of the activation dtype (or fp32 under bf16
         autocast)."""
         C = geom.channels
-        if x_windows.dtype != torch.bfloat16 or shortcut.dtype != torch.bfloat16 or geom.window != 8:
+        if x_windows.dtype != torch.bfloat16 or shortcut.dtype != torch.bfloat16:
             return False
         if not kernels.linear_supported(x_windows, C, C):
+            return False
+        if geom.window != 8 and not kernels.linear_fills(x_windows.numel() // C, C):
             return False
         if geom.win_row_begin != 0 or geom.valid is not None or geom.rows != geom.frame_h // geom.window:
             return False
@@ -300,7 +308,11 @@ class SequentialSwinTransformer(torch.nn.Module):
             o = self.attn.attend(x_windows, mask=self.window_mask(geom))
             if o.dtype == torch.bfloat16:
                 w, b = self.attn.proj_packed()
-                y = kernels.linear_residual(o.contiguous(), w, C, shortcut.contiguous().view(B, H, W, C), b, geom=geom)
+                o, shortcut = o.contiguous(), shortcut.contiguous().view(B, H, W, C)
+                if geom.window == 8:
+                    y = kernels.linear_residual(o, w, C, shortcut, b, geom=geom)
+                else:
+                    y = kernels.linear_scatter(o, w, C, shortcut, geom=geom, bias=b)
                 return y.view(B, H * W, C)
             attn_windows = autograd.linear(o, self.attn.proj.weight, self.attn.proj.bias)
         else:

@@ -459,6 +459,19 @@ def test_linear_residual_rejects_bad_arguments():
     assert _lin_res_call(rows=6 * 64, geom=other_c) == -3 and "out_features" in L.last_error()
 
 
+def test_linear_scatter_rejects_bad_arguments():
+    def call(geom, rows):
+        return L.load().terra_swin_linear_scatter(FAKE, ctypes.c_void_p(1 << 31), ctypes.c_void_p(1 << 31), L.DTYPE_BF16,
+                                                  rows, 1024, 1024, FAKE, None,
+                                                  None if geom is None else ctypes.byref(geom), None)
+
+    assert call(None, 512) == -1
+    w7 = kernels.WindowGeometry(1, 14, 21, 1024, 7).to_c()
+    assert call(w7, 6 * 64) == -3 and "window tokens" in L.last_error()
+    slab = kernels.WindowGeometry(1, 14, 21, 1024, 7, 0, 0, (0, 0, 0, 0), 0, 1).to_c()
+    assert call(slab, 3 * 49) == -5 and "every window of the frame" in L.last_error()
+
+
 def test_training_linear_entries_reject_bad_arguments():
     lib = L.load()
     p = lambda a: ctypes.c_void_p(a << 28)  # noqa: E731

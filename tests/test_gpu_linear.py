@@ -146,6 +146,55 @@ def test_linear_scatter_bit_exact_with_identity_weight(dev, case):
     assert torch.equal(got, want)
 
 
+SCATTER_ANY_CASES = [  # (B, H, W, window, shift, pad)
+    (2, 64, 96, 32, 16, (0, 0, 0, 0)),
+    (3, 14, 21, 7, 3, (0, 0, 0, 0)),
+    (2, 13, 19, 7, 0, (1, 0, 0, 2)),
+    (1, 30, 50, 16, 5, (1, 1, 7, 7)),
+    (2, 5, 9, 1, 0, (0, 0, 0, 0)),
+    (1, 3, 3, 3, 1, (0, 0, 0, 0)),
+    (2, 16, 24, 8, 4, (0, 0, 0, 0)),
+]
+
+
+@pytest.mark.parametrize("case", SCATTER_ANY_CASES)
+def test_linear_scatter_any_window_bit_exact_with_identity_weight(dev, case):
+    """As above for windows of other sizes (terra_swin_linear_scatter)."""
+    B, H, W, ws, s, pad = case
+    C = 256
+    geom = WindowGeometry(B, H, W, C, ws, s, s, pad)
+    win = workloads.activations((geom.num_windows, ws * ws, C), 35).to(torch.bfloat16)
+    r = workloads.activations((B, H, W, C), 36).to(torch.bfloat16)
+    wd = kernels.pack_linear(torch.eye(C, dtype=torch.bfloat16).to(dev))
+    got = kernels.linear_scatter(win.to(dev), wd, C, r.to(dev), geom)
+    assert torch.equal(got.cpu(), so.reverse_frame(win, B, H, W, ws, s, s, pad, residual=r))
+    if ws != 8:  # the other entry keeps refusing these windows
+        with pytest.raises((ValueError, RuntimeError, NotImplementedError), match="8x8"):
+            kernels.linear_residual(win.to(dev), wd, C, r.to(dev), geom=geom)
+
+
+def test_block_window32_takes_the_scatter_launch(dev, monkeypatch):
+    """A window-32 block whose rows fill the chip projects, reverses and adds the
+    residual in one launch; the staged order gives the same to bf16 rounding."""
+    from terra_amd.transformer import SequentialSwinTransformer
+    blk = SequentialSwinTransformer(layer_idx=1, height=256, width=128, embedding_dim=512, window_size=32, num_heads=4,
+                                    use_attn_mask=False, use_relative_position_bias=False)
+    workloads.init_block_params(blk, 1)
+    blk = blk.to(dev, torch.bfloat16)
+    x = workloads.activations((1, 256 * 128, 512), 37).to(dev, torch.bfloat16)
+    calls = []
+    real = kernels.linear_scatter
+    monkeypatch.setattr(kernels, "linear_scatter", lambda *a, **k: calls.append(1) or real(*a, **k))
+    with torch.no_grad():
+        y = blk(x)
+        assert calls == [1]
+        monkeypatch.setattr(kernels, "linear_fills", lambda *a: False)
+        want = blk(x)
+        assert calls == [1]
+    # Two bf16 roundings (the product, the sum) on either side.
+    assert ((y - x).float() - (want - x).float()).norm() <= 2.0 ** -7 * (want - x).float().norm()
+
+
 @pytest.mark.parametrize("shape", [(1, 32, 48), (1, 288, 544)], ids=["small", "g1-grid"])
 def test_linear_scatter_matches_proj_then_reverse(dev, shape):
     """proj + reverse + residual in one kernel against the five-stage order
