@@ -11,11 +11,13 @@ parameter's data pointer or in-place version changes.
 Inference at other widths with C % 64 == 0 and 4C <= 4096 (C = 1024, the
 width of TERRA's pretrain blocks): the LayerNorm on the HIP LayerNorm kernel
 over the token rows, fc1 + exact GELU on the linear kernel's GELU epilogue,
-fc2 + residual on hipBLASLt.
+fc2 + residual on its residual epilogue (hipBLASLt where that does not serve
+the shape or the rows do not fill the chip).
 
 A call that needs a gradient runs autograd.mlp: the LayerNorm forward and
 backward (residual gradient included) on the HIP LayerNorm kernels over the
-token rows, the GEMMs on hipBLASLt.  Other shapes and dtypes run the
+token rows, the GEMMs on the linear and weight-gradient kernels where they
+serve the shapes, else on hipBLASLt.  Other shapes and dtypes run the
 reference's own sequence of torch modules on the device (norm2, fc1, act,
 fc2, residual).  Parameter names (``norm2``, ``fc1``, ``fc2``) and the seeded
 initialisation follow the reference so its checkpoints load.
@@ -81,8 +83,7 @@ class SequentialMlp(torch.nn.Module):
     def _trainable(self, x: torch.Tensor) -> bool:
         """A call that needs gradients through a plain LayerNorm over C <= 1024
         (rows of whole 16-byte chunks), the exact GELU and biased linears:
-        the LayerNorm and its backward run on the HIP kernels
-        (autograd.mlp), the GEMMs on hipBLASLt."""
+        autograd.mlp, the LayerNorm and its backward on the HIP kernels."""
         if not (torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in self.parameters()))):
             return False
         C = x.shape[-1]
@@ -102,8 +103,10 @@ class SequentialMlp(torch.nn.Module):
         hidden 4C, a plain LayerNorm, the exact GELU, biased bf16 linears (or
         fp32 ones under bf16 autocast), no gradient.  The LayerNorm runs on
         the HIP LayerNorm kernel over the token rows and fc1 + GELU on the
-        linear kernel with the GELU epilogue; fc2 + residual on hipBLASLt,
-        which is faster than the linear kernel for the 4C -> C product."""
+        linear kernel with the GELU epilogue, fc2 + residual on it too where C
+        is a multiple of 256 and the rows fill the chip (us for the
+        MLP, against hipBLASLt: 156672 x 1024 2409 / 2502, 16500 x 1024 342 /
+        397, 262144 x 256 406 / 461; equal at 65536 x 1024)."""
         if not self.use_fused_mlp or x.dim() < 1 or x.dtype != torch.bfloat16 or x.device.type != "cuda":
             return False
         C = x.shape[-1]
@@ -131,6 +134,8 @@ class SequentialMlp(torch.nn.Module):
         xn = kernels.swin_partition_ln(rows.view(1, n, 1, C), kernels.rows_geometry(n, C), a["ln_weight"],
                                        a["ln_bias"], a["ln_eps"]).view(n, C)
         h = kernels.linear(xn, a["fc1_weight"], 4 * C, a["fc1_bias"], gelu=True)
+        if kernels.linear_supported(h, 4 * C, C) and kernels.linear_fills(n, C):
+            return kernels.linear_residual(h, a["fc2_weight"], C, rows, a["fc2_bias"]).view(x.shape)
         w2, b2 = self._fc2_bf16()
         return (F.linear(h, w2, b2) + rows).view(x.shape)
 

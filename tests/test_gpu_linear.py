@@ -300,3 +300,24 @@ def test_linear_short(dev, rows, k, n):
                                           bd.data_ptr(), 0, None)
     torch.cuda.synchronize()
     assert st == 0 and torch.equal(guard[:rows * n].view(rows, n), y) and bool((guard[rows * n:] == 7.0).all())
+
+
+@pytest.mark.parametrize("C,tokens,amp", [(256, 65300, False), (1024, 16385, True), (256, 4097, False)])
+def test_mlp_inference_fc2_on_the_residual_epilogue(dev, C, tokens, amp, monkeypatch):
+    """SequentialMlp at widths the one-kernel MLP does not take: fc2 + residual
+    run on the linear kernel where the rows fill the chip, with the library's
+    result to the bf16 roundings of the product and of the sum."""
+    from terra_amd.mlp import SequentialMlp
+    torch.manual_seed(9)
+    m = SequentialMlp(C, 4 * C).to(dev, torch.float32 if amp else torch.bfloat16)
+    x = workloads.activations((1, tokens, C), 38).to(dev, torch.bfloat16)
+    calls = []
+    real, fills = kernels.linear_residual, kernels.linear_fills(tokens, C)
+    monkeypatch.setattr(kernels, "linear_residual", lambda *a, **k: calls.append(1) or real(*a, **k))
+    with torch.no_grad(), torch.amp.autocast("cuda", dtype=torch.bfloat16, enabled=amp):
+        y = m(x)
+        assert len(calls) == int(fills)
+        monkeypatch.setattr(kernels, "linear_fills", lambda *a: False)
+        want = m(x)
+    assert y.dtype == want.dtype
+    assert (y.float() - want.float()).norm() <= 2.0 ** -7 * want.float().norm()
