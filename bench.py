@@ -22,9 +22,9 @@ module through torch's ops, and `full_block` both halves together.
     python bench.py [--steps K] [--warmup W] [--no-cpu-baseline] [--config c1..c5|g1]
 
 The other configurations (default c3) run the same measurement: c5 through
-the 12-head fused kernel; c1, c2 and c4 (fp32, 7x7 windows, head dim 64)
-through the five-stage path, whose roofline is then the attention core's
-(HBM-bound), with the MLP half through torch's ops where no fused MLP kernel
+the 12-head fused kernel, c2 and c4 through theirs, c1 (fp32) through its
+one-kernel block; g1 and w32 run the staged path.  Where the step is not a
+bf16 fused kernel the roofline is the attention core's, with the MLP half through torch's ops where no fused MLP kernel
 serves the shape.
     python bench.py --mode kernels --steps 3     # the step's kernels only,
                                                  # plus a 192 MiB device copy
