@@ -146,9 +146,11 @@ class WindowAttention(torch.nn.Module):
 
     def proj_packed(self):
         """proj's weight in the fragment-packed layout of the linear kernels
-        (bf16; autocast's cast of an fp32 weight) and its bias as fp32,
-        cached until either changes; for calls without gradients."""
+        (bf16; autocast's cast of an fp32 weight), its bias as fp32, and that
+        bias rounded to bf16 first (as F.linear under autocast adds it), cached
+        until either changes; for calls without gradients."""
         w, b = self.proj.weight, self.proj.bias
+        f32 = lambda t: None if t is None else t.to(torch.float32).contiguous()  # noqa: E731
         return self._cached("proj_packed", [w, b], lambda: (
-            kernels.pack_linear(w.detach().to(torch.bfloat16).contiguous()),
-            None if b is None else b.detach().to(torch.float32).contiguous()))
+            kernels.pack_linear(w.detach().to(torch.bfloat16).contiguous()), f32(b),
+            f32(None if b is None else b.to(torch.bfloat16))))

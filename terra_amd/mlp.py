@@ -135,7 +135,7 @@ class SequentialMlp(torch.nn.Module):
                                        a["ln_bias"], a["ln_eps"]).view(n, C)
         h = kernels.linear(xn, a["fc1_weight"], 4 * C, a["fc1_bias"], gelu=True)
         if kernels.linear_supported(h, 4 * C, C) and kernels.linear_fills(n, C):
-            return kernels.linear_residual(h, a["fc2_weight"], C, rows, a["fc2_bias"]).view(x.shape)
+            return kernels.linear_residual(h, a["fc2_weight"], C, rows, self._fc2_bias()).view(x.shape)
         w2, b2 = self._fc2_bf16()
         return (F.linear(h, w2, b2) + rows).view(x.shape)
 
@@ -150,6 +150,18 @@ class SequentialMlp(torch.nn.Module):
             with torch.no_grad():
                 hit = (key, (w.detach().to(torch.bfloat16), b.detach().to(torch.bfloat16)))
             self._fc2_cache = hit
+        return hit[1]
+
+    def _fc2_bias(self) -> torch.Tensor:
+        """fc2's bias as F.linear adds it (under autocast rounded to bf16), in
+        fp32 for the residual epilogue, cached."""
+        b = self.fc2.bias
+        key = (b.data_ptr(), b._version, b.dtype, b.device)
+        hit = getattr(self, "_fc2_bias_cache", None)
+        if hit is None or hit[0] != key:
+            with torch.no_grad():
+                hit = (key, b.detach().to(torch.bfloat16).to(torch.float32).contiguous())
+            self._fc2_bias_cache = hit
         return hit[1]
 
     def _fused_args(self) -> dict:

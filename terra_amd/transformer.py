@@ -307,12 +307,12 @@ class SequentialSwinTransformer(torch.nn.Module):
             # proj + window reverse + inverse roll + residual in one kernel.
             o = self.attn.attend(x_windows, mask=self.window_mask(geom))
             if o.dtype == torch.bfloat16:
-                w, b = self.attn.proj_packed()
+                w, b, b_rounded = self.attn.proj_packed()
                 o, shortcut = o.contiguous(), shortcut.contiguous().view(B, H, W, C)
                 if geom.window == 8:
                     y = kernels.linear_residual(o, w, C, shortcut, b, geom=geom)
-                else:
-                    y = kernels.linear_scatter(o, w, C, shortcut, geom=geom, bias=b)
+                else:  # with the bias of the staged path's F.linear, which serves the calls that do not fill the chip
+                    y = kernels.linear_scatter(o, w, C, shortcut, geom=geom, bias=b_rounded)
                 return y.view(B, H * W, C)
             attn_windows = autograd.linear(o, self.attn.proj.weight, self.attn.proj.bias)
         else:

@@ -321,3 +321,40 @@ def test_mlp_inference_fc2_on_the_residual_epilogue(dev, C, tokens, amp, monkeyp
         want = m(x)
     assert y.dtype == want.dtype
     assert (y.float() - want.float()).norm() <= 2.0 ** -7 * want.float().norm()
+
+
+def test_window32_block_adds_the_bias_that_f_linear_adds(dev, monkeypatch):
+    """fp32 parameters under bf16 autocast: F.linear rounds proj's bias to bf16.
+    The scatter launch gives the staged path's result but for the order of the
+    fp32 sums, which moves a product of 512 terms across a bf16 rounding for
+    about one value in a thousand; an unrounded bias moves one in ten."""
+    from terra_amd.transformer import SequentialSwinTransformer
+    blk = SequentialSwinTransformer(layer_idx=1, height=256, width=128, embedding_dim=512, window_size=32, num_heads=4,
+                                    use_attn_mask=False, use_relative_position_bias=False)
+    workloads.init_block_params(blk, 1)
+    blk.attn.proj.bias.data.copy_(workloads.activations((512,), 39))
+    blk = blk.to(dev)
+    x = workloads.activations((1, 256 * 128, 512), 37).to(dev, torch.bfloat16)
+    calls = []
+    real = kernels.linear_scatter
+    monkeypatch.setattr(kernels, "linear_scatter", lambda *a, **k: calls.append(1) or real(*a, **k))
+    with torch.no_grad(), torch.amp.autocast("cuda", dtype=torch.bfloat16):
+        y = blk(x)
+        monkeypatch.setattr(kernels, "linear_fills", lambda *a: False)
+        want = blk(x)
+    assert calls == [1] and (y != want).float().mean() <= 0.01
+
+
+@pytest.mark.parametrize("C,tokens", [(256, 65300), (1024, 16385)])
+def test_mlp_fc2_adds_the_bias_that_f_linear_adds(dev, C, tokens, monkeypatch):
+    """As above for fc2 + residual in SequentialMlp."""
+    from terra_amd.mlp import SequentialMlp
+    torch.manual_seed(10)
+    m = SequentialMlp(C, 4 * C).to(dev)
+    m.fc2.bias.data.copy_(workloads.activations((C,), 39))
+    x = workloads.activations((1, tokens, C), 38).to(dev, torch.bfloat16)
+    with torch.no_grad(), torch.amp.autocast("cuda", dtype=torch.bfloat16):
+        y = m(x)
+        monkeypatch.setattr(kernels, "linear_fills", lambda *a: False)
+        want = m(x)
+    assert (y != want).float().mean() <= 0.01
