@@ -176,10 +176,21 @@ def weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
 
 def _bf16_linears(x: torch.Tensor, *params: Optional[torch.Tensor]) -> bool:
     """Whether F.linear of bf16 rows like x with these parameters is a bf16
-    product: under bf16 autocast, or with bf16 parameters and no autocast."""
+    product: under bf16 autocast, which casts fp32 and fp16 parameters (fp64
+    ones it leaves, and F.linear refuses), or with bf16 parameters and no
+    autocast."""
     if torch.is_autocast_enabled(x.device.type):
-        return kernels.autocast_bf16(x)
+        cast = (torch.bfloat16, torch.float32, torch.float16)
+        return kernels.autocast_bf16(x) and all(p is None or p.dtype in cast for p in params)
     return all(p is None or p.dtype == torch.bfloat16 for p in params)
+
+
+def _pack(weight: torch.Tensor, transpose: bool = False) -> torch.Tensor:
+    """:func:`kernels.pack_weight` of a weight of any dtype, which packs bf16
+    and fp32 ones; others are rounded to bf16 first, as autocast rounds them."""
+    if weight.dtype not in (torch.bfloat16, torch.float32):
+        weight = weight.to(torch.bfloat16)
+    return kernels.pack_weight(weight, transpose)
 
 
 def _bias32(bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
@@ -212,9 +223,9 @@ def _input_grad(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     if dy.dtype != torch.bfloat16:
         return dy @ weight.to(dy.dtype)
     if _short_kernel(dy, weight.shape[1]):
-        return kernels.linear_short(dy, kernels.pack_weight(weight, transpose=True), weight.shape[1])
+        return kernels.linear_short(dy, _pack(weight, transpose=True), weight.shape[1])
     if _linear_kernel(dy, weight.shape[1]):
-        return kernels.linear(dy, kernels.pack_weight(weight, transpose=True), weight.shape[1])
+        return kernels.linear(dy, _pack(weight, transpose=True), weight.shape[1])
     return dy @ weight.to(dy.dtype)
 
 
@@ -305,12 +316,12 @@ class _Mlp(torch.autograd.Function):
         y = None
         bf16 = xn.dtype == torch.bfloat16 and _bf16_linears(xn, w1, b1, w2, b2)
         if bf16 and _short_kernel(xn, w1.shape[0]):
-            h1, a = kernels.linear_short(xn, kernels.pack_weight(w1), w1.shape[0], _bias32(b1), gelu_keep=True)
+            h1, a = kernels.linear_short(xn, _pack(w1), w1.shape[0], _bias32(b1), gelu_keep=True)
         elif bf16 and _linear_kernel(xn, w1.shape[0]):
-            h1, a = kernels.linear_gelu_keep(xn, kernels.pack_weight(w1), w1.shape[0], _bias32(b1))
+            h1, a = kernels.linear_gelu_keep(xn, _pack(w1), w1.shape[0], _bias32(b1))
             if rows.dtype == torch.bfloat16 and w2.shape[0] == C and rows.data_ptr() % 16 == 0 \
                     and _linear_kernel(a, C):
-                y = kernels.linear_residual(a, kernels.pack_weight(w2), C, rows, _bias32(b2))
+                y = kernels.linear_residual(a, _pack(w2), C, rows, _bias32(b2))
         else:
             h1 = torch.nn.functional.linear(xn, w1, b1)
             a = torch.nn.functional.gelu(h1)
@@ -354,7 +365,7 @@ class _Mlp(torch.autograd.Function):
             # fc2's input gradient, the GELU derivative and fc1's bias gradient in one kernel.
             if ctx.needs_input_grad[4]:
                 db1 = torch.zeros(h1.shape[-1], dtype=torch.float32, device=h1.device)
-            dh1 = kernels.linear_gelu_backward(dh2, kernels.pack_weight(w2, transpose=True), h1.shape[-1], h1,
+            dh1 = kernels.linear_gelu_backward(dh2, _pack(w2, transpose=True), h1.shape[-1], h1,
                                                column_sums=db1)
         else:
             da = dh2 @ w2.to(gemm_dtype)

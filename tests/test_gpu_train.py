@@ -710,3 +710,32 @@ def test_attention_half_keeps_the_chain_for_other_calls(dev, monkeypatch):
         blk = blk.to(dev)
         blk(torch.randn(1, 196, 96, device=dev)).sum().backward()
         assert blk.attn.proj.weight.grad is not None
+
+
+@pytest.mark.parametrize("x_dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("C,tokens", [(192, 9000), (1024, 16500)])
+def test_mlp_training_casts_fp16_parameters_under_autocast(dev, C, tokens, x_dtype):
+    """fp16 parameters in a bf16 autocast region, which casts them, with rows
+    that fill the chip: the gradients of the fp16 values in float64, 1e-2
+    normwise (bf16 operands, weights rounded to bf16)."""
+    m = _mlp_case(C, 630).to(dev, torch.float16)
+    x = workloads.activations((tokens, C), 631).to(dev, x_dtype)
+    gy = workloads.activations((tokens, C), 632).to(dev)
+    xd = x.clone().requires_grad_(True)
+    with torch.amp.autocast("cuda", dtype=torch.bfloat16):
+        y = m(xd)
+    y.backward(gy.to(y.dtype))
+    yr, xg, pg = _oracle_mlp_grads(m, x, gy, torch.float64, bf16_weights=True)
+    assert _normwise(y.detach(), yr) <= 1e-2 and _normwise(xd.grad, xg) <= 1e-2
+    for n, p in m.named_parameters():
+        assert p.grad.dtype == torch.float16 and _normwise(p.grad, pg[n]) <= 1e-2, n
+
+
+def test_mlp_training_refuses_fp64_parameters_under_autocast(dev):
+    """Autocast leaves fp64 parameters as they are and F.linear refuses them, at any size."""
+    x = workloads.activations((9000, 192), 633).to(dev).requires_grad_(True)
+    for name in ("weight", "bias"):
+        m = _mlp_case(192, 634).to(dev)
+        setattr(m.fc1, name, torch.nn.Parameter(getattr(m.fc1, name).detach().double()))
+        with torch.amp.autocast("cuda", dtype=torch.bfloat16), pytest.raises(RuntimeError):
+            m(x)
