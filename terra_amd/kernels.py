@@ -704,8 +704,9 @@ def swin_block_f32_train(x: torch.Tensor, geom: WindowGeometry, num_heads: int, 
 # Prepared launches, keyed by the ids of the parameter tensors, the call's
 # scalars and the activation shape.  An entry holds weak references to those
 # tensors with their data pointers and sizes, and serves a call only while
-# each reference still names the tensor passed and its data pointer and size
-# are unchanged (so a reused id, a rebound ``.data`` or an in-place resize
+# each reference still names the tensor passed, its data pointer and size
+# are unchanged and it is contiguous (so a reused id, a ``.data`` rebound to
+# other memory or to a transposed view of the same, or an in-place resize
 # builds a new entry).  Entries are
 # made only when the kernel reads the caller's tensors themselves (no
 # conversion copies), so in-place updates of them are seen by later calls,
@@ -743,7 +744,7 @@ class _Launch:
             if t is None:
                 if ref is not None:
                     return False
-            elif ref is None or ref() is not t or t.data_ptr() != ptr or t.numel() != n:
+            elif ref is None or ref() is not t or t.data_ptr() != ptr or t.numel() != n or not t.is_contiguous():
                 return False
         return True
 

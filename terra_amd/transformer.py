@@ -210,9 +210,10 @@ class SequentialSwinTransformer(torch.nn.Module):
         ln_w, ln_b = (None, None) if n is None else (n.weight, n.bias)
         if parts[3] is None or any(t is not None and t.dtype != torch.float32 for t in (*parts, w, b, table, ln_w, ln_b)):
             return None
-        # The kernel reads 16 bytes at a time; views at other offsets (of a flat
-        # parameter buffer, say) stay on the staged path.
-        if any(t is not None and t.data_ptr() % 16 for t in (x, w, b, ln_w, ln_b)):
+        # The kernel reads 16 bytes at a time of a row-major weight; views at
+        # other offsets (of a flat parameter buffer, say) and a proj weight of
+        # other strides (a transposed or tied view) stay on the staged path.
+        if not w.is_contiguous() or any(t is not None and t.data_ptr() % 16 for t in (x, w, b, ln_w, ln_b)):
             return None
         qkv_w, qkv_b = attn._cached("qkv", parts, lambda: (torch.cat(parts[:3], 0), torch.cat(parts[3:], 0)))
         return dict(qkv_weight=qkv_w, qkv_bias=qkv_b, proj_weight=w, proj_bias=b, ln_weight=ln_w, ln_bias=ln_b,

@@ -122,3 +122,18 @@ def test_block_f32_train_serves_only_its_calls(dev):
     assert kernels.swin_block_f32_train(xd.half(), whole, 3, 1.0, *args) is None
     assert kernels.swin_block_f32_train(xd, whole, 3, 1.0, w.t().contiguous().t(), *args[1:]) is None
     assert kernels.swin_block_f32_train(xd, whole, 4, 1.0, *args) is None
+
+
+@pytest.mark.parametrize("warm", [False, True])
+def test_block_f32_leaves_a_transposed_proj_weight_to_the_staged_path(dev, warm):
+    """A proj weight that is a transposed view, from the start or rebound to one
+    of the same memory after a call, is served with its own values."""
+    blk, _, x = _block(dev, CASES[1])
+    xd, w = x.to(dev), blk.attn.proj.weight
+    with torch.no_grad():
+        if warm:
+            blk(xd)
+        w.data = w.data.t()
+        got = blk(xd)
+        blk.use_fused_block = False
+        assert rel_norm(got - xd, blk(xd) - xd) <= 1e-6

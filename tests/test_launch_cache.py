@@ -42,6 +42,13 @@ def test_rebound_data_and_resize_are_not_served():
     assert not e.serves((b,))
 
 
+def test_data_rebound_to_a_transposed_view_is_not_served():
+    a = torch.zeros(8, 8)
+    e = _entry(a)
+    a.data = a.data.t()  # same tensor object, memory and size, other strides
+    assert not e.serves((a,))
+
+
 def test_entry_keeps_nothing_alive():
     a = torch.zeros(16)
     ref_count = len(gc.get_referrers(a))
