@@ -543,11 +543,11 @@ class _AttentionHalf(torch.autograd.Function):
     one launch and keeps what the backward reads)."""
 
     @staticmethod
-    def forward(ctx, x, ln_w, ln_b, qw, kw, vw, qb, kb, vb, pw, pb, table, geom, eps, num_heads, scale, mask):
+    def forward(ctx, x, ln_w, ln_b, qw, kw, vw, qb, kb, vb, pw, pb, table, geom, eps, num_heads, scale, mask, fused):
         C = geom.channels
         w, b = torch.cat((qw, kw, vw), 0), None if qb is None else torch.cat((qb, kb, vb), 0)
         ctx.cfg = (geom, eps, num_heads, scale, mask)
-        if x.dtype == torch.float32 and not torch.is_autocast_enabled(x.device.type):
+        if fused and x.dtype == torch.float32 and not torch.is_autocast_enabled(x.device.type):
             # The small fp32 configuration: the whole forward in one launch.
             done = kernels.swin_block_f32_train(x, geom, num_heads, scale, w, b, pw, pb, ln_w, ln_b, eps, table, mask)
             if done is not None:
@@ -629,14 +629,14 @@ class _AttentionHalf(torch.autograd.Function):
         cast = lambda g, t: None if g is None else g.to(t)  # noqa: E731
         return (dx if need[0] else None, None if dln_w is None else dln_w.to(ln_w.dtype),
                 None if dln_b is None else dln_b.to(ln_b.dtype), dq, dk, dv, dqb, dkb, dvb, dpw, cast(dpb, pb_dtype),
-                None if dtable is None else dtable.to(table.dtype), None, None, None, None, None)
+                None if dtable is None else dtable.to(table.dtype), None, None, None, None, None, None)
 
 
 def attention_half(x: torch.Tensor, geom: WindowGeometry, norm: torch.nn.LayerNorm, attn: torch.nn.Module,
-                   mask: MaskArg) -> torch.Tensor:
+                   mask: MaskArg, fused: bool = True) -> torch.Tensor:
     """The attention half-block on x [B, H, W, C] with gradients (see
     :class:`_AttentionHalf`); ``attn``: a WindowAttention of plain Linears with
-    a biased proj."""
+    a biased proj.  ``fused`` False keeps the forward on the staged kernels."""
     q, k, v, proj = attn.q_linear, attn.k_linear, attn.v_linear, attn.proj
     return _AttentionHalf.apply(x, norm.weight, norm.bias, q.weight, k.weight, v.weight, q.bias, k.bias, v.bias,
-                                proj.weight, proj.bias, attn._table(), geom, norm.eps, attn.num_heads, attn.scale, mask)
+                                proj.weight, proj.bias, attn._table(), geom, norm.eps, attn.num_heads, attn.scale, mask, fused)

@@ -84,7 +84,8 @@ class SequentialSwinTransformer(torch.nn.Module):
         self._land_bits_cache = {}
         self._mask_cache = None
         # Run the whole half-block as one kernel where the shapes allow it
-        # (see _fusable_block); False forces the five-stage path.
+        # (see _fusable_block, _block_f32_args; fp32 training: the forward);
+        # False forces the five-stage path.
         self.use_fused_block = True
 
     def geometry(self, batch: int) -> WindowGeometry:
@@ -279,7 +280,8 @@ class SequentialSwinTransformer(torch.nn.Module):
         # with their HIP backward kernels.
         training = torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in self.parameters()))
         if training and self._one_function(grid):
-            return autograd.attention_half(grid, geom, self.norm1, self.attn, self.window_mask(geom)).view(B, H * W, C)
+            return autograd.attention_half(grid, geom, self.norm1, self.attn, self.window_mask(geom),
+                                           self.use_fused_block).view(B, H * W, C)
         link = None
         if config.use_layernorm and not training and self._fusable_norm(grid.dtype):
             n = self.norm1

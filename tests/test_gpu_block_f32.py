@@ -137,3 +137,24 @@ def test_block_f32_leaves_a_transposed_proj_weight_to_the_staged_path(dev, warm)
         got = blk(xd)
         blk.use_fused_block = False
         assert rel_norm(got - xd, blk(xd) - xd) <= 1e-6
+
+
+def test_block_f32_training_honours_use_fused_block(dev, monkeypatch):
+    """use_fused_block = False keeps a training forward on the staged kernels, with the same gradients to fp32 rounding."""
+    blk, _, x = _block(dev, CASES[2])
+    calls = []
+    orig = kernels.swin_block_f32_train
+    monkeypatch.setattr(kernels, "swin_block_f32_train", lambda *a, **k: calls.append(1) or orig(*a, **k))
+
+    def step():
+        xd = x.to(dev).requires_grad_(True)
+        blk.zero_grad(set_to_none=True)
+        y = blk(xd)
+        y.backward(torch.ones_like(y))
+        return y.detach() - xd.detach(), xd.grad, blk.attn.proj.weight.grad
+
+    want = step()
+    assert calls == [1]
+    blk.use_fused_block = False
+    got = step()
+    assert calls == [1] and all(rel_norm(a, b) <= 1e-5 for a, b in zip(got, want))
