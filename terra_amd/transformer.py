@@ -127,17 +127,25 @@ class SequentialSwinTransformer(torch.nn.Module):
                 and dtype in (torch.float32, torch.float16, torch.bfloat16)
                 and row_bytes % 16 == 0 and row_bytes <= 4096 and self.embedding_dim <= 1024)
 
+    def _plain_attn(self) -> bool:
+        """attn's forward may be passed by: a WindowAttention itself, with no
+        forward of its own and no forward hooks that would see the call."""
+        attn, hooks = self.attn, torch.nn.modules.module
+        return (type(attn) is WindowAttention and "forward" not in attn.__dict__
+                and not (attn._forward_hooks or attn._forward_pre_hooks)
+                and not (hooks._global_forward_hooks or hooks._global_forward_pre_hooks))
+
     def _proj_scatter(self, x_windows: torch.Tensor, shortcut: torch.Tensor, geom: WindowGeometry) -> bool:
         """Whether the output projection, the window reverse and the residual
         add can run as one linear-kernel launch: bf16 windows and shortcut,
         8x8 windows (others where the rows fill the chip: window 32, C =
         1024, 156672 tokens 2042 -> 1971 us for the block, 16384 tokens 238 ->
         225; window 7, C = 256, 117600 tokens 269 -> 244), C a multiple of 256 (the kernel's feature tile; C = 1024
-        for TERRA's pretrain blocks), every window of the frame emitted, a
-        biased nn.Linear proj of the activation dtype (or fp32 under bf16
+        for TERRA's pretrain blocks), every window of the frame emitted, attn's
+        forward free to be passed by, a biased nn.Linear proj of the activation dtype (or fp32 under bf16
         autocast)."""
         C = geom.channels
-        if x_windows.dtype != torch.bfloat16 or shortcut.dtype != torch.bfloat16:
+        if x_windows.dtype != torch.bfloat16 or shortcut.dtype != torch.bfloat16 or not self._plain_attn():
             return False
         if not kernels.linear_supported(x_windows, C, C):
             return False
@@ -190,7 +198,7 @@ class SequentialSwinTransformer(torch.nn.Module):
     def _block_f32_args(self, x: torch.Tensor, geom: WindowGeometry) -> Optional[dict]:
         """Arguments of kernels.swin_block_f32 where the whole half-block runs
         as one fp32 kernel, else None: fp32 activations and parameters outside
-        autocast, (window, heads, C) in kernels.BLOCK_F32_SHAPES, a plain
+        autocast, attn's forward free to be passed by, (window, heads, C) in kernels.BLOCK_F32_SHAPES, a plain
         LayerNorm (or none), biased q/k/v, and no gradient needed.  The q|k|v
         weights and biases are concatenated (cached until one changes).
         Faster than the staged path's five launches at every size (us per
@@ -198,6 +206,8 @@ class SequentialSwinTransformer(torch.nn.Module):
         440 -> 320."""
         attn = self.attn
         if not self.use_fused_block or not kernels.swin_block_f32_supported(x, geom, attn.num_heads):
+            return None
+        if not self._plain_attn():
             return None
         if torch.is_autocast_enabled(x.device.type) or (config.use_layernorm and not self._fusable_norm(x.dtype)):
             return None

@@ -16,6 +16,8 @@ import torch
 from helpers import assert_block_matches, gain_block, params_of
 from oracle import swin_oracle as so
 from terra_amd import kernels, workloads
+from terra_amd.attention import WindowAttention
+from terra_amd.transformer import SequentialSwinTransformer
 
 pytestmark = pytest.mark.gpu
 
@@ -265,3 +267,40 @@ def test_c4_stack_24_blocks_full_size(dev):
     growth = (torch.linalg.vector_norm(d_f - d_u) / torch.linalg.vector_norm(d_u)).item()
     print(f"24-block stack: |y - x| max {d_u.abs().max().item():.3f}, fused vs five-stage normwise {growth:.3e}")
     assert growth <= 5e-2, growth
+
+
+# (channels, heads, window, height, width, dtype): the fp32 kernel, the scatter launch of other windows and of 8x8 ones
+ONE_LAUNCH_BLOCKS = [(96, 3, 7, 28, 28, torch.float32), (512, 4, 32, 256, 128, torch.bfloat16),
+                     (256, 2, 8, 16, 16, torch.bfloat16)]
+
+
+@pytest.mark.parametrize("C,heads,ws,H,W,dtype", ONE_LAUNCH_BLOCKS)
+@pytest.mark.parametrize("how", ["hook", "pre-hook", "global hook", "subclass", "instance forward"])
+def test_one_launch_blocks_keep_the_call_of_attn(dev, C, heads, ws, H, W, dtype, how):
+    """Forward hooks on attn and a forward of its own are seen where proj or
+    the whole half-block would otherwise run in one launch."""
+    blk = SequentialSwinTransformer(layer_idx=0, height=H, width=W, embedding_dim=C, window_size=ws, num_heads=heads,
+                                    use_attn_mask=False, use_relative_position_bias=False)
+    blk = blk.to(dev, dtype)
+    x = workloads.activations((1, H * W, C), 90).to(dev, dtype)
+    calls = []
+    handle = None
+    orig = blk.attn.forward
+    if how == "hook":
+        blk.attn.register_forward_hook(lambda m, a, out: calls.append(1))
+    elif how == "pre-hook":
+        blk.attn.register_forward_pre_hook(lambda m, a: calls.append(1))
+    elif how == "global hook":
+        handle = torch.nn.modules.module.register_module_forward_hook(
+            lambda m, a, out: calls.append(1) if m is blk.attn else None)
+    elif how == "subclass":
+        blk.attn.__class__ = type("Own", (WindowAttention,), {"forward": lambda self, *a, **k: calls.append(1) or orig(*a, **k)})
+    else:
+        blk.attn.forward = lambda *a, **k: calls.append(1) or orig(*a, **k)
+    try:
+        with torch.no_grad():
+            blk(x)
+    finally:
+        if handle is not None:
+            handle.remove()
+    assert calls == [1]
