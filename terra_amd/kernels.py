@@ -660,9 +660,14 @@ def swin_block_f32(x: torch.Tensor, geom: WindowGeometry, num_heads: int, scale:
     """:func:`swin_block` in fp32 (terra_swin_block_f32_fwd) for the shapes of
     BLOCK_F32_SHAPES: fp32 ``x`` [B, H, W, C] and parameters, row-major
     ``qkv_weight`` [3C, C] and ``proj_weight`` [C, C]."""
-    if geom.batch == 0 and x.numel() == 0:
+    _dtype_code(x, (torch.float32,))
+    if geom.batch == 0 and x.numel() == 0:  # an empty batch: nothing to launch
         _require_device(x)
-        return torch.empty_like(x) if out is None else out
+        if out is None:
+            return torch.empty_like(x)
+        if out.shape != x.shape or out.dtype != x.dtype or out.device != x.device:
+            raise ValueError("out must be a contiguous tensor like x")
+        return out
     given = (qkv_weight, qkv_bias, proj_weight, proj_bias, ln_weight, ln_bias, bias_table, land_bits)
     key = ("block_f32", tuple(map(id, given)), geom, num_heads, float(scale), float(ln_eps), bool(layernorm),
            bool(shift_mask), float(mask_value), x.shape, x.dtype, x.device)

@@ -158,3 +158,18 @@ def test_block_f32_training_honours_use_fused_block(dev, monkeypatch):
     blk.use_fused_block = False
     got = step()
     assert calls == [1] and all(rel_norm(a, b) <= 1e-5 for a, b in zip(got, want))
+
+
+def test_block_f32_refuses_other_dtypes_and_outputs(dev):
+    """bf16 x of a shape the bf16 kernel serves, and an output unlike an empty x, are refused."""
+    bf = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=dev)  # noqa: E731
+    geom = kernels.WindowGeometry(batch=1, height=8, width=8, channels=192, window=8)
+    with pytest.raises(TypeError):
+        kernels.swin_block_f32(bf(1, 8, 8, 192), geom, 6, 1.0, bf(576, 192), None, bf(192, 192), None)
+    none = kernels.WindowGeometry(batch=0, height=7, width=7, channels=96, window=7)
+    f32 = lambda *s: torch.zeros(*s, device=dev)  # noqa: E731
+    args = (none, 3, 1.0, f32(288, 96), None, f32(96, 96), None)
+    assert kernels.swin_block_f32(f32(0, 7, 7, 96), *args).shape == (0, 7, 7, 96)
+    for out in (f32(1, 7, 7, 96), bf(0, 7, 7, 96)):
+        with pytest.raises(ValueError):
+            kernels.swin_block_f32(f32(0, 7, 7, 96), *args, out=out)
