@@ -304,3 +304,19 @@ def test_one_launch_blocks_keep_the_call_of_attn(dev, C, heads, ws, H, W, dtype,
         if handle is not None:
             handle.remove()
     assert calls == [1]
+
+
+@pytest.mark.parametrize("C,heads,ws,H,W", [(512, 4, 32, 256, 128), (256, 2, 8, 16, 16)])
+def test_bf16_block_takes_x_at_any_offset(dev, C, heads, ws, H, W):
+    """x two bytes off an 8-byte boundary, behind a norm that is not fused: the
+    residual the scatter launch does not read goes through the staged path, to
+    the bf16 roundings of the product and of the sum."""
+    blk = SequentialSwinTransformer(layer_idx=0, height=H, width=W, embedding_dim=C, window_size=ws, num_heads=heads,
+                                    use_attn_mask=False, use_relative_position_bias=False,
+                                    norm_layer=type("Norm", (torch.nn.LayerNorm,), {})).to(dev, torch.bfloat16)
+    buf = workloads.activations((H * W * C + 1,), 91).to(dev, torch.bfloat16)
+    x = buf[1:].view(1, H * W, C)
+    assert x.data_ptr() % 8 == 2
+    with torch.no_grad():
+        got, want = blk(x), blk(x.clone())
+    assert (got.float() - want.float()).norm() <= 2.0 ** -8 * want.float().norm()
