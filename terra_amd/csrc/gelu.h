@@ -71,13 +71,15 @@ __device__ __forceinline__ float gelu_slope(float h) {
   return cdf + h * pdf;
 }
 
-// The GELU's slope Phi(h) + h phi(h) of a bf16 h: an fp32 table for 2^-13 <=
-// |h| < 8 filled with gelu_slope; from 8 on the last entries (1, and -8e-14 for
-// negative h) stand for the limits 1 and 0 to fp32 rounding; below 2^-13 the
-// slope is 1/2 + 2 phi(0) h to fp32 rounding (the next term is below 2^-40).
-// +-inf and NaN give NaN (inf * 0).  16 KB.
-constexpr uint32_t kSlopeTabLo = 0x3900;  // bf16 bits of 2^-13
-constexpr uint32_t kSlopeTabHi = 0x4100;  // bf16 bits of 8
+// The GELU's slope Phi(h) + h phi(h) of a bf16 h: an fp32 table for 2^-12 <=
+// |h| < 16 filled with gelu_slope; from 16 on the last entries (1, and 0 for
+// negative h: exp(-127) is 0 in fp32) are the limits; below 2^-12 the slope is
+// 1/2 + 2 phi(0) h to fp32 rounding (the next term, -2/3 phi(0) h^3, is below
+// 2^-37).  The table ends where the slope does: with 2^-13 .. 8 in the same
+// 16 KB (all that the linear kernel's LDS leaves) every h <= -8 kept the slope
+// of -7.97, -5e-14.  +-inf and NaN give NaN (inf * 0).
+constexpr uint32_t kSlopeTabLo = 0x3980;  // bf16 bits of 2^-12
+constexpr uint32_t kSlopeTabHi = 0x4180;  // bf16 bits of 16
 constexpr int kSlopeTabSpan = (int)(kSlopeTabHi - kSlopeTabLo);
 constexpr int kSlopeTabBytes = 2 * kSlopeTabSpan * 4;
 

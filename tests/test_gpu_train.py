@@ -739,3 +739,17 @@ def test_mlp_training_refuses_fp64_parameters_under_autocast(dev):
         setattr(m.fc1, name, torch.nn.Parameter(getattr(m.fc1, name).detach().double()))
         with torch.amp.autocast("cuda", dtype=torch.bfloat16), pytest.raises(RuntimeError):
             m(x)
+
+
+def test_linear_gelu_backward_slope_of_every_bf16_value(dev):
+    """The slope in the linear kernel's epilogue against the GELU backward
+    kernel's, bit for bit, over all 2^16 values of h: a product of 2^60 shows
+    the tails, where the slope is far below fp32's resolution of 1."""
+    h = torch.arange(1 << 16, device=dev).to(torch.int32).to(torch.int16).view(torch.bfloat16).view(256, 256)
+    dy = torch.zeros(256, 64, device=dev, dtype=torch.bfloat16)
+    dy[:, 0] = 2.0 ** 60
+    w2 = torch.zeros(64, 256, device=dev)
+    w2[0] = 1.0
+    got = kernels.linear_gelu_backward(dy, kernels.pack_weight(w2, transpose=True), 256, h)
+    want = kernels.gelu_backward(torch.full_like(h, 2.0 ** 60), h)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(0.0), want.nan_to_num(0.0))
