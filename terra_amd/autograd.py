@@ -320,7 +320,7 @@ class _Mlp(torch.autograd.Function):
         elif bf16 and _linear_kernel(xn, w1.shape[0]):
             h1, a = kernels.linear_gelu_keep(xn, _pack(w1), w1.shape[0], _bias32(b1))
             if rows.dtype == torch.bfloat16 and w2.shape[0] == C and rows.data_ptr() % 16 == 0 \
-                    and _linear_kernel(a, C):
+                    and _linear_kernel(a, C) and kernels.linear_residual_pays(a.shape[0], a.shape[1], C):
                 y = kernels.linear_residual(a, _pack(w2), C, rows, _bias32(b2))
         else:
             h1 = torch.nn.functional.linear(xn, w1, b1)

@@ -866,8 +866,31 @@ def linear_supported(x: torch.Tensor, in_features: int, out_features: int) -> bo
 def linear_fills(rows: int, out_features: int) -> bool:
     """Whether a linear-kernel launch has a 256 x 256 tile for each of the 256
     compute units.  Below that the library's smaller tiles keep more of the
-    chip busy; at and above it the fused epilogues pay."""
-    return -(-rows // 256) * (out_features // LINEAR_OUT_MULTIPLE) >= 256
+    chip busy; at and above it the epilogues that replace a whole pass pay at
+    every row count (proj + scatter, 263 to 514 tiles: the block 1.00-1.07 of
+    the staged path's speed; the GELU backward 1.47 and more)."""
+    return linear_tiles(rows, out_features) >= 256
+
+
+def linear_tiles(rows: int, out_features: int) -> int:
+    """256 x 256 tiles of a linear-kernel launch."""
+    return -(-rows // 256) * (out_features // LINEAR_OUT_MULTIPLE)
+
+
+def linear_residual_pays(rows: int, in_features: int, out_features: int) -> bool:
+    """Whether fc2 + residual in one launch is as fast as the library's product
+    and an add.  The kernel's time goes by rounds of 256 tiles, the library's
+    smaller tiles fill a partial second round better, and the pass saved weighs
+    less the longer the contraction (us, library / kernel, for 256, 264, 288,
+    320, 352, 384, 480 tiles; 4096 -> 1024: 106 / 106, 150 / 183, 145 / 185, 156
+    / 189, 177 / 193, 183 / 197, 208 / 217, which in the whole MLP is 410 / 413
+    from 384 on; 2048 -> 512: 65 / 61, 83 / 104, 89 / 104, 96 / 104, 104 / 105,
+    111 / 106, 129 / 125; 1024 -> 256: 48 / 40, 67 / 64, 64 / 64, 70 / 66, 80 /
+    65, 82 / 68, 99 / 83).  65 row blocks of 4096 -> 1024 (260 tiles) are the
+    exception, the library taking 219 against 177."""
+    tiles = linear_tiles(rows, out_features)
+    least = 384 if in_features > 2048 else 340 if in_features > 1024 else 288
+    return linear_fills(rows, out_features) and (tiles <= (260 if in_features > 2048 else 256) or tiles >= least)
 
 
 def _linear_checks(x: torch.Tensor, weight_packed: torch.Tensor, out_features: int, bias: Optional[torch.Tensor]):

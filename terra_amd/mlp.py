@@ -12,7 +12,7 @@ Inference at other widths with C % 64 == 0 and 4C <= 4096 (C = 1024, the
 width of TERRA's pretrain blocks): the LayerNorm on the HIP LayerNorm kernel
 over the token rows, fc1 + exact GELU on the linear kernel's GELU epilogue,
 fc2 + residual on its residual epilogue (hipBLASLt where that does not serve
-the shape or the rows do not fill the chip).
+the shape or is slower).
 
 A call that needs a gradient runs autograd.mlp: the LayerNorm forward and
 backward (residual gradient included) on the HIP LayerNorm kernels over the
@@ -104,9 +104,10 @@ class SequentialMlp(torch.nn.Module):
         fp32 ones under bf16 autocast), no gradient.  The LayerNorm runs on
         the HIP LayerNorm kernel over the token rows and fc1 + GELU on the
         linear kernel with the GELU epilogue, fc2 + residual on it too where C
-        is a multiple of 256 and the rows fill the chip (us for the
-        MLP, against hipBLASLt: 156672 x 1024 2409 / 2502, 16500 x 1024 342 /
-        397, 262144 x 256 406 / 461; equal at 65536 x 1024)."""
+        is a multiple of 256 and kernels.linear_residual_pays (us for the MLP,
+        against fc2 on hipBLASLt: 156672 x 1024 2409 / 2502, 40000 x 1024 659 /
+        717, 16500 x 1024 347 / 390, 65536 x 512 308 / 324, 262144 x 256 406 /
+        461; equal at 24576 to 33000 and at 65536 x 1024)."""
         if not self.use_fused_mlp or x.dim() < 1 or x.dtype != torch.bfloat16 or x.device.type != "cuda":
             return False
         C = x.shape[-1]
@@ -134,7 +135,7 @@ class SequentialMlp(torch.nn.Module):
         xn = kernels.swin_partition_ln(rows.view(1, n, 1, C), kernels.rows_geometry(n, C), a["ln_weight"],
                                        a["ln_bias"], a["ln_eps"]).view(n, C)
         h = kernels.linear(xn, a["fc1_weight"], 4 * C, a["fc1_bias"], gelu=True)
-        if kernels.linear_supported(h, 4 * C, C) and kernels.linear_fills(n, C):
+        if kernels.linear_supported(h, 4 * C, C) and kernels.linear_residual_pays(n, 4 * C, C):
             return kernels.linear_residual(h, a["fc2_weight"], C, rows, self._fc2_bias()).view(x.shape)
         w2, b2 = self._fc2_bf16()
         return (F.linear(h, w2, b2) + rows).view(x.shape)

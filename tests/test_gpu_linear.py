@@ -358,3 +358,16 @@ def test_mlp_fc2_adds_the_bias_that_f_linear_adds(dev, C, tokens, monkeypatch):
         monkeypatch.setattr(kernels, "linear_fills", lambda *a: False)
         want = m(x)
     assert (y != want).float().mean() <= 0.01
+
+
+@pytest.mark.parametrize("C,tokens,launches", [(1024, 16896, 0), (1024, 24576, 1), (512, 33000, 0), (256, 66000, 0),
+                                               (256, 73728, 1)])
+def test_mlp_inference_takes_the_residual_launch_where_it_pays(dev, C, tokens, launches, monkeypatch):
+    from terra_amd.mlp import SequentialMlp
+    m = SequentialMlp(C, 4 * C).to(dev, torch.bfloat16)
+    calls = []
+    real = kernels.linear_residual
+    monkeypatch.setattr(kernels, "linear_residual", lambda *a, **k: calls.append(1) or real(*a, **k))
+    with torch.no_grad():
+        m(torch.randn(1, tokens, C, device=dev, dtype=torch.bfloat16))
+    assert len(calls) == launches

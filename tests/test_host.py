@@ -152,3 +152,15 @@ def test_window_mask_land_bits_follow_the_frame(monkeypatch):
     m1 = blk.window_mask(blk.geometry(1))
     assert m1.land_bits.tolist() == [1, 2]
     assert seen == [0, 1]
+
+
+@pytest.mark.parametrize("rows,k,n,pays", [
+    (16128, 4096, 1024, False), (16129, 4096, 1024, True), (16640, 4096, 1024, True), (16641, 4096, 1024, False),
+    (24320, 4096, 1024, False), (24321, 4096, 1024, True), (32768, 2048, 512, True), (32769, 2048, 512, False),
+    (43264, 2048, 512, False), (43265, 2048, 512, True), (65536, 1024, 256, True), (65537, 1024, 256, False),
+    (73472, 1024, 256, False), (73473, 1024, 256, True), (10 ** 6, 4096, 1024, True)])
+def test_linear_residual_pays_by_rounds(rows, k, n, pays):
+    """fc2 + residual takes its one launch on a whole round of tiles and again
+    from where the second round is filled enough, between which the library
+    is faster."""
+    assert kernels.linear_residual_pays(rows, k, n) is pays
