@@ -218,13 +218,13 @@ def _linear_kernel(x: torch.Tensor, out_features: int) -> bool:
 def _input_grad(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """dy @ weight for dy [T, out] in the GEMMs' dtype and a Linear's weight
     [out, in] of any dtype: on the linear kernels where they serve the shape
-    (156672 rows, 4096 -> 1024: 980-1060 us against 1130-1240 for the
+    and are as fast as the library (156672 rows, 4096 -> 1024: 980-1060 us against 1130-1240 for the
     library's product with an untransposed weight)."""
     if dy.dtype != torch.bfloat16:
         return dy @ weight.to(dy.dtype)
     if _short_kernel(dy, weight.shape[1]):
         return kernels.linear_short(dy, _pack(weight, transpose=True), weight.shape[1])
-    if _linear_kernel(dy, weight.shape[1]):
+    if _linear_kernel(dy, weight.shape[1]) and kernels.linear_product_pays(dy.shape[0], weight.shape[1]):
         return kernels.linear(dy, _pack(weight, transpose=True), weight.shape[1])
     return dy @ weight.to(dy.dtype)
 
@@ -317,7 +317,7 @@ class _Mlp(torch.autograd.Function):
         bf16 = xn.dtype == torch.bfloat16 and _bf16_linears(xn, w1, b1, w2, b2)
         if bf16 and _short_kernel(xn, w1.shape[0]):
             h1, a = kernels.linear_short(xn, _pack(w1), w1.shape[0], _bias32(b1), gelu_keep=True)
-        elif bf16 and _linear_kernel(xn, w1.shape[0]):
+        elif bf16 and _linear_kernel(xn, w1.shape[0]) and kernels.linear_gelu_keep_pays(xn.shape[0], C, w1.shape[0]):
             h1, a = kernels.linear_gelu_keep(xn, _pack(w1), w1.shape[0], _bias32(b1))
             if rows.dtype == torch.bfloat16 and w2.shape[0] == C and rows.data_ptr() % 16 == 0 \
                     and _linear_kernel(a, C) and kernels.linear_residual_pays(a.shape[0], a.shape[1], C):

@@ -893,6 +893,28 @@ def linear_residual_pays(rows: int, in_features: int, out_features: int) -> bool
     return linear_fills(rows, out_features) and (tiles <= (260 if in_features > 2048 else 256) or tiles >= least)
 
 
+def linear_product_pays(rows: int, out_features: int) -> bool:
+    """Whether a plain product of bf16 rows (an input gradient) on the linear
+    kernel is as fast as the library's.  Nothing rides on it, so the rounds
+    alone decide: from half a second round on, but for a third round less than
+    a third full (us, library / kernel, 3072 -> 1024, tiles: 264 108 / 138, 320
+    119 / 141, 384 132 / 150, 400 140 / 140, 480 153 / 148, 576 203 / 220, 640
+    262 / 218, 768 250 / 250, 1024 333 / 331, 1152 423 / 388)."""
+    tiles = linear_tiles(rows, out_features)
+    return tiles >= 388 and not 512 < tiles < 600
+
+
+def linear_gelu_keep_pays(rows: int, in_features: int, out_features: int) -> bool:
+    """Whether fc1 with the GELU and its input kept in one launch is as fast as
+    the library's product and torch's GELU.  Up to 512 input features from one
+    round on (1.1 to 1.9 times); above that the two stores of a tile weigh on a
+    short call and it takes four rounds (us, library / kernel, 1024 -> 4096,
+    tiles: 256 51 / 62, 384 79 / 91, 512 90 / 100, 768 129 / 134, 1024 171 / 168,
+    1152 207 / 194; 768 -> 3072: 264 68 / 73, 576 98 / 107, 768 114 / 112, 1032 179
+    / 158)."""
+    return linear_fills(rows, out_features) and (in_features <= 512 or linear_tiles(rows, out_features) >= 1024)
+
+
 def _linear_checks(x: torch.Tensor, weight_packed: torch.Tensor, out_features: int, bias: Optional[torch.Tensor]):
     dev = _require_device(x, weight_packed)
     code = _dtype_code(x, (torch.bfloat16,))

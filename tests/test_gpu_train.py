@@ -753,3 +753,25 @@ def test_linear_gelu_backward_slope_of_every_bf16_value(dev):
     got = kernels.linear_gelu_backward(dy, kernels.pack_weight(w2, transpose=True), 256, h)
     want = kernels.gelu_backward(torch.full_like(h, 2.0 ** 60), h)
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(0.0), want.nan_to_num(0.0))
+
+
+@pytest.mark.parametrize("tokens,launches", [(6001, (0, 1, 0)), (17000, (1, 1, 0)), (26000, (1, 1, 1))])
+def test_mlp_training_takes_the_linear_kernels_where_they_pay(dev, tokens, launches, monkeypatch):
+    """fc1 + GELU, the GELU backward and fc1's input gradient (1024 features)
+    against float64 on either side of each rule."""
+    m = _mlp_case(1024, 640).to(dev)
+    x, gy = (workloads.activations((tokens, 1024), s).to(dev, torch.bfloat16) for s in (641, 642))
+    calls = []
+    names = ("linear_gelu_keep", "linear_gelu_backward", "linear")
+    for name in names:
+        real = getattr(kernels, name)
+        monkeypatch.setattr(kernels, name, lambda *a, name=name, real=real, **k: calls.append(name) or real(*a, **k))
+    xd = x.clone().requires_grad_(True)
+    with torch.amp.autocast("cuda", dtype=torch.bfloat16):
+        y = m(xd)
+    y.backward(gy)
+    assert tuple(calls.count(n) for n in names) == launches
+    yr, xg, pg = _oracle_mlp_grads(m, x, gy, torch.float64, bf16_weights=True)
+    assert _normwise(y.detach(), yr) <= 1e-2 and _normwise(xd.grad, xg) <= 1e-2
+    for n, p in m.named_parameters():
+        assert _normwise(p.grad, pg[n]) <= 1e-2, n

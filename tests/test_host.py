@@ -164,3 +164,17 @@ def test_linear_residual_pays_by_rounds(rows, k, n, pays):
     from where the second round is filled enough, between which the library
     is faster."""
     assert kernels.linear_residual_pays(rows, k, n) is pays
+
+
+@pytest.mark.parametrize("rows,n,pays", [(16384, 1024, False), (24576, 1024, False), (24577, 1024, True), (32768, 1024, True),
+                                         (32769, 1024, False), (38144, 1024, False), (38145, 1024, True), (33024, 768, False),
+                                         (33025, 768, True), (10 ** 6, 256, True)])
+def test_linear_product_pays_by_rounds(rows, n, pays):
+    assert kernels.linear_product_pays(rows, n) is pays
+
+
+@pytest.mark.parametrize("rows,k,n,pays", [(4096, 1024, 4096, False), (16128, 1024, 4096, False), (16129, 1024, 4096, True),
+                                           (21760, 768, 3072, False), (21761, 768, 3072, True), (8192, 512, 2048, True),
+                                           (7936, 512, 2048, False), (10752, 384, 1536, False), (10753, 384, 1536, True)])
+def test_linear_gelu_keep_pays_by_rounds(rows, k, n, pays):
+    assert kernels.linear_gelu_keep_pays(rows, k, n) is pays
