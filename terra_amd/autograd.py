@@ -151,12 +151,14 @@ def partition_ln(x: torch.Tensor, geom: WindowGeometry, weight: Optional[torch.T
 def weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """dy^T x for dy [T, out] and x [T, in] (a Linear's weight gradient, the
     contraction over all T tokens), in fp32.  bf16 rows run on the HIP
-    weight-gradient kernel, which cuts the tokens into as many slices as give
-    each compute unit one (output tile, slice) pair and adds them in order
-    (us, against the library's batched product over token slices and its sum:
-    524288 x 768 x 192 213-247 / 251-300, 524288 x 576 x 192 165 / 242,
-    156672 x 4096 x 1024 1097 / 1530, 50176 x 512 x 128 25 / 33; equal at 524288
-    x 192 x 192 and 32768 x 768 x 768).  Other dtypes (and feature counts that
+    weight-gradient kernel, which cuts the tokens into as many slices as fill
+    the compute units with (output tile, slice) pairs, sums each in two levels
+    and adds them in a fixed order (us, against the library's batched product
+    over token slices and its sum, or for other token counts its plain product
+    rounded to bf16: 524288 x 768 x 192 204 / 255, 524288 x 576 x 192 176 / 246,
+    156672 x 4096 x 1024 1370 / 1562, 50176 x 512 x 128 25 / 31, 16385 x 1024 x 1024
+    49 / 140, 2001 x 1024 x 1024 25 / 22; equal at 524288 x 192 x 192 and 32768 x
+    768 x 768).  Other dtypes (and feature counts that
     are no multiple of 16) take the library: for large T in fp16 k slices
     contracted as one batched GEMM with an fp32 output and then summed, since
     hipBLASLt takes no split-K tiles for a contraction this long."""

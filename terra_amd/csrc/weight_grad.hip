@@ -11,17 +11,32 @@
 // Both operands are stored with the contracted dimension (tokens) outermost.  A
 // workgroup streams stages of 32 token rows of its two column ranges straight
 // into LDS (global->LDS loads by buffer descriptor: rows past the end read 0),
-// four buffers, and reads MFMA fragments by transposed LDS reads
+// wg_bufs buffers (6 to 8), and reads MFMA fragments by transposed LDS reads
 // (ds_read_b64_tr_b16: four tokens of one column per lane), so nothing is
 // transposed through memory.  x is the A operand, so a lane's four accumulator
 // rows are consecutive in dW; eight waves, 2 x 4, each WA / 2 x WB / 4 of the
 // tile.
 //
+// Sums are taken in two levels: the matrix cores add kWgFold stages (1024
+// tokens) to an accumulator, which is then added to a second one.  One chain
+// over a slice rounds the growing sum at every stage.  Normwise errors against
+// float64, 156672 x 4096 x 1024: 4 slices of one chain 1.3e-6, in two levels
+// 2.5e-7, the library's product over 64 slices 3.1e-7; 524288 x 768 x 192: 5.2e-7,
+// 2.1e-7, 4.0e-7.  Two accumulators per output leave room for tiles of 128 x 256
+// where one had 256 x 256 (1137 us); the same error by one chain in each of 64
+// slices costs 2 GB of partial results.
+// Times, us, library / here: 156672 x 4096 x 1024 1562 / 1370 (1520 in 64
+// slices), 156672 x 3072 x 1024 1183 / 1089, 524288 x 768 x 192 255 / 204,
+// 524288 x 576 x 192 246 / 176, 32768 x 768 x 768 54 / 53, 2001 x 1024 x 1024 22 / 25.
+//
 // What bounds it: for narrow layers (C = 192) HBM, every operand row being read
 // once (the output tiles of a slice share an XCD's L2); for wide ones (C =
-// 1024) the matrix cores and the power limit.  A stage's fragments are read
-// while the one before is multiplied, each right after its registers' last use,
-// in pinned order, and the loads run as many stages ahead as the LDS holds.
+// 1024) the matrix cores and the power limit, and 15 TB/s out of L2.  A stage's
+// fragments are read while the one before is multiplied, each right after its
+// registers' last use, in pinned order, and the loads run as many stages ahead
+// as the LDS holds.  An XCD's workgroups take a square of a slice's tiles (the
+// shorter side of their grid first), so that they share their rows (1024 x 4096:
+// 1405 -> 1380 us).
 #include "common.h"
 #include "attn_core.h"
 
@@ -30,7 +45,9 @@ namespace {
 
 constexpr int kWgThreads = 512;
 constexpr int kWgTok = 32;     // tokens per stage (one MFMA k-step)
+constexpr int kWgFold = 32;    // stages per accumulator chain
 constexpr int kWgCus = 256;    // one workgroup per CU
+constexpr int kWgLong = 4096;  // per slice, from which a second round pays
 constexpr int kWgMinTokens = 512;  // per slice: below this its fixed cost outweighs the split
 
 struct WgParams {
@@ -40,11 +57,11 @@ struct WgParams {
   int64_t rows;
   int64_t slice_rows; // a multiple of kWgTok
   int32_t na, nb;
-  int32_t tiles_b, tiles, slices;
+  int32_t tiles_a, tiles_b, tiles, slices;
   int32_t per_xcd;    // workgroups per XCD
 };
 
-// LDS buffers of a tile: as many stages as fit (5 for 256 x 256), at most 8.
+// LDS buffers of a tile: as many stages as fit (6 for 128 x 256), at most 8.
 constexpr int wg_bufs(int wa, int wb) {
   const int n = 160 * 1024 / (kWgTok * (wa + wb) * 2);
   return n < 8 ? n : 8;
@@ -79,7 +96,10 @@ void weight_grad_kernel(const WgParams p) {
   const int id = ((int)blockIdx.x & 7) * p.per_xcd + ((int)blockIdx.x >> 3);
   if (id >= p.tiles * p.slices || ((int)blockIdx.x >> 3) >= p.per_xcd) return;  // uniform
   const int slice = id / p.tiles, tile = id - slice * p.tiles;
-  const int ta = tile / p.tiles_b, tb = tile - ta * p.tiles_b;
+  const bool a_first = p.tiles_a <= p.tiles_b;
+  const int side = a_first ? p.tiles_a : p.tiles_b;
+  const int tq = tile / side, tr = tile - tq * side;
+  const int ta = a_first ? tr : tq, tb = a_first ? tq : tr;
   const int wn = wave & 3, wm = wave >> 2;
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_address(smem));
 
@@ -158,11 +178,20 @@ void weight_grad_kernel(const WgParams p) {
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  f32x4 acc[NI][NJ];
+  f32x4 acc[NI][NJ], sum[NI][NJ];
 #pragma unroll
   for (int i = 0; i < NI; ++i)
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NJ; ++j) acc[i][j] = sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto fold = [&]() {
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        sum[i][j] = sum[i][j] + acc[i][j];
+        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+  };
   for (int s = 0; s < kBufs - 1 && s < stages; ++s) {
 #pragma unroll
     for (int q = 0; q < kPer; ++q) issue(q);
@@ -192,7 +221,9 @@ void weight_grad_kernel(const WgParams p) {
       }
     if (live) issue_advance();
     stage_end(live);
+    if (s % kWgFold == kWgFold - 1) fold();  // uniform
   }
+  fold();
 
   // Lane (c16, g) of (i, j): A indexes 16 i + 4 g + r of B index 16 j + c16.
   const int g = lane >> 4, c16 = lane & 15;
@@ -204,37 +235,63 @@ void weight_grad_kernel(const WgParams p) {
       const int ia = ta * WA + wm * (WA / 2) + 16 * i + 4 * g;
       const int ib = tb * WB + wn * (WB / 4) + 16 * j + c16;
       if (ia >= p.na || ib >= p.nb) continue;  // both multiples of 16
-      *reinterpret_cast<f32x4*>(out + (int64_t)ib * p.na + ia) = acc[i][j];
+      *reinterpret_cast<f32x4*>(out + (int64_t)ib * p.na + ia) = sum[i][j];
     }
 }
 
-// out = the slices' sum, in slice order.
+// out = the slices' sum: kG threads per 16-byte column group, each over
+// consecutive slices in order, then their results pairwise.  Many slices of a
+// small matrix need kG = 8 (128 slices of 128 x 128: 64 threads' worth of
+// columns would read them in a chain; the call 20.6 -> 15.2 us).
+template <int kG>
 __global__ __launch_bounds__(256) void weight_grad_sum_kernel(const float* __restrict__ part, float* __restrict__ out,
                                                               int64_t n4, int slices) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n4) return;
-  const f32x4* src = reinterpret_cast<const f32x4*>(part) + i;
-  f32x4 s = src[0];
-  int k = 1;
-  for (; k + 8 <= slices; k += 8) {
+  constexpr int kCols = 256 / kG;
+  __shared__ f32x4 s_sum[256];
+  const int c = (int)threadIdx.x % kCols, grp = (int)threadIdx.x / kCols;
+  const int64_t i = (int64_t)blockIdx.x * kCols + c;
+  const f32x4* src = reinterpret_cast<const f32x4*>(part) + (i < n4 ? i : n4 - 1);
+  const int per = (slices + kG - 1) / kG;
+  const int end = (grp + 1) * per < slices ? (grp + 1) * per : slices;
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+  int k = grp * per;
+  for (; k + 8 <= end; k += 8) {
     f32x4 v[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) v[u] = src[(int64_t)(k + u) * n4];
 #pragma unroll
     for (int u = 0; u < 8; ++u) s += v[u];
   }
-  for (; k < slices; ++k) s += src[(int64_t)k * n4];
-  reinterpret_cast<f32x4*>(out)[i] = s;
+  for (; k < end; ++k) s += src[(int64_t)k * n4];
+  if constexpr (kG > 1) {
+    s_sum[threadIdx.x] = s;
+    __syncthreads();
+#pragma unroll
+    for (int h = kG / 2; h > 0; h /= 2) {
+      if (grp < h) s_sum[threadIdx.x] = s_sum[threadIdx.x] + s_sum[threadIdx.x + h * kCols];
+      __syncthreads();
+    }
+    s = s_sum[threadIdx.x];
+  }
+  if (grp == 0 && i < n4) reinterpret_cast<f32x4*>(out)[i] = s;
 }
 
-// Tile width for n columns: the widest of 256, 192, 128 whose padding is least.
-int wg_width(int n) {
-  int best = 256, waste = (n + 255) / 256 * 256 - n;
-  for (int w : {192, 128}) {
-    const int u = (n + w - 1) / w * w - n;
-    if (u < waste) {
-      best = w;
-      waste = u;
+// Tiles, x columns by dy columns: as large as two accumulators per output and
+// the fragments fit (174 and 195 VGPRs for the first two).
+struct WgTile {
+  int wa, wb;
+};
+constexpr WgTile kWgTiles[] = {{128, 256}, {192, 192}, {192, 128}, {128, 192}, {128, 128}};
+
+// The first tile that pads na x nb least.
+WgTile wg_tile(int na, int nb) {
+  WgTile best = kWgTiles[0];
+  int64_t least = INT64_MAX;
+  for (const WgTile& t : kWgTiles) {
+    const int64_t area = (int64_t)((na + t.wa - 1) / t.wa * t.wa) * ((nb + t.wb - 1) / t.wb * t.wb);
+    if (area < least) {
+      best = t;
+      least = area;
     }
   }
   return best;
@@ -245,18 +302,28 @@ struct WgPlan {
   int64_t slice_rows;
 };
 
-// Slices: as many as give each CU one (tile, slice) pair.
+// Slices: as many (tile, slice) pairs as fill the CUs once, or, for slices of
+// kWgLong tokens, up to four times where whole tiles would leave more than a
+// tenth of them idle (96 tiles of 1024 x 3072: 192 pairs in one round, 480 in two:
+// 156672 tokens 1200 -> 1089 us, but 4096 tokens 47 -> 53).
 WgPlan wg_plan(int64_t rows, int na, int nb) {
   WgPlan q;
-  q.wa = wg_width(na);
-  q.wb = wg_width(nb);
+  const WgTile t = wg_tile(na, nb);
+  q.wa = t.wa;
+  q.wb = t.wb;
   q.tiles_a = (na + q.wa - 1) / q.wa;
   q.tiles_b = (nb + q.wb - 1) / q.wb;
-  const int tiles = q.tiles_a * q.tiles_b;
-  int64_t s = kWgCus / tiles;
+  const int64_t tiles = (int64_t)q.tiles_a * q.tiles_b;
+  int64_t s = 1, filled = 0;  // per mille of the CUs over the rounds
+  for (int64_t rounds = 1; rounds <= 4 && filled < 900; ++rounds) {
+    const int64_t n = kWgCus * rounds / tiles, f = n * tiles * 1000 / (kWgCus * rounds);
+    if (n > 0 && f > filled && (rounds == 1 || rows >= n * kWgLong)) {
+      s = n;
+      filled = f;
+    }
+  }
   const int64_t most = (rows + kWgMinTokens - 1) / kWgMinTokens;
   if (s > most) s = most;
-  if (s < 1) s = 1;
   q.slice_rows = ((rows + s - 1) / s + kWgTok - 1) / kWgTok * kWgTok;
   q.slices = (int)((rows + q.slice_rows - 1) / q.slice_rows);
   return q;
@@ -271,12 +338,6 @@ int launch_weight_grad(const WgParams& p, hipStream_t s) {
   if (attr != hipSuccess) return fail(TERRA_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(attr));
   kern<<<8 * p.per_xcd, kWgThreads, lds, s>>>(p);
   return TERRA_OK;
-}
-
-template <int WA>
-int dispatch_weight_grad(const WgParams& p, int wb, hipStream_t s) {
-  return wb == 256 ? launch_weight_grad<WA, 256>(p, s)
-                   : wb == 192 ? launch_weight_grad<WA, 192>(p, s) : launch_weight_grad<WA, 128>(p, s);
 }
 
 int wg_check(int64_t rows, int out_features, int in_features) {
@@ -323,18 +384,27 @@ extern "C" int terra_swin_weight_grad(const void* dy, const void* x, float* dw, 
   p.slice_rows = q.slice_rows;
   p.na = na;
   p.nb = nb;
+  p.tiles_a = q.tiles_a;
   p.tiles_b = q.tiles_b;
   p.tiles = q.tiles_a * q.tiles_b;
   p.slices = q.slices;
   p.per_xcd = (p.tiles * p.slices + 7) / 8;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int st = q.wa == 256 ? dispatch_weight_grad<256>(p, q.wb, s)
-                             : q.wa == 192 ? dispatch_weight_grad<192>(p, q.wb, s) : dispatch_weight_grad<128>(p, q.wb, s);
+  int st;
+  if (q.wb == 256)
+    st = launch_weight_grad<128, 256>(p, s);
+  else if (q.wb == 192)
+    st = q.wa == 192 ? launch_weight_grad<192, 192>(p, s) : launch_weight_grad<128, 192>(p, s);
+  else
+    st = q.wa == 192 ? launch_weight_grad<192, 128>(p, s) : launch_weight_grad<128, 128>(p, s);
   if (st != TERRA_OK) return st;
   if (q.slices > 1) {
     const int64_t n4 = (int64_t)na * nb / 4;
-    weight_grad_sum_kernel<<<(uint32_t)((n4 + 255) / 256), 256, 0, s>>>(static_cast<const float*>(workspace), dw, n4,
-                                                                       q.slices);
+    const float* part = static_cast<const float*>(workspace);
+    if (q.slices >= 16)
+      weight_grad_sum_kernel<8><<<(uint32_t)((n4 + 31) / 32), 256, 0, s>>>(part, dw, n4, q.slices);
+    else
+      weight_grad_sum_kernel<1><<<(uint32_t)((n4 + 255) / 256), 256, 0, s>>>(part, dw, n4, q.slices);
   }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(TERRA_ERR_LAUNCH, "terra_swin_weight_grad launch failed: %s", hipGetErrorString(e));

@@ -775,3 +775,33 @@ def test_mlp_training_takes_the_linear_kernels_where_they_pay(dev, tokens, launc
     assert _normwise(y.detach(), yr) <= 1e-2 and _normwise(xd.grad, xg) <= 1e-2
     for n, p in m.named_parameters():
         assert _normwise(p.grad, pg[n]) <= 1e-2, n
+
+
+@pytest.mark.parametrize("mean", [0.0, 0.3])
+@pytest.mark.parametrize("T,o,i", [(156672, 4096, 1024), (156673, 3072, 1024), (524288, 768, 192)])
+def test_weight_grad_sums_long_contractions_in_two_levels(dev, T, o, i, mean):
+    """Normwise error against float64 over 64 output features.  fp32 sums of n
+    independent terms in one chain are off by about 3.6e-8 sqrt(n / 32) of the
+    result (n / 32 MFMA steps, measured); 32 steps a chain and 77 chains a slice
+    leave 2.0e-7 and 1.5e-7.  One chain per slice gave 1.3e-6, 1.1e-6 and 5.2e-7,
+    the library's sums over 64 and 128 slices 3.1e-7 and 4.1e-7."""
+    g = torch.Generator(dev).manual_seed(601)
+    dy = (torch.randn(T, o, device=dev, generator=g) + mean).bfloat16()
+    x = (torch.randn(T, i, device=dev, generator=g) + mean).bfloat16()
+    got = kernels.weight_grad(dy, x)[:64].double()
+    want = dy[:, :64].double().t().contiguous() @ x.double()
+    assert ((got - want).norm() / want.norm()).item() <= 3e-7
+
+
+@pytest.mark.parametrize("T,o,i", [(1023, 256, 128), (1024, 512, 256), (1025, 192, 384), (2049, 208, 144), (5000, 3072, 1024),
+                                   (16385, 3072, 1024), (40000, 1152, 1152), (600, 16, 4096), (600, 4096, 16)])
+def test_weight_grad_tiles_and_folds(dev, T, o, i):
+    """Every tile shape, chains that end at, before and after the end of a
+    slice, one and several rounds of slices, grids of tiles longer on either
+    side: within T u of the sum of magnitudes, the same bits twice."""
+    g = torch.Generator(dev).manual_seed(602)
+    dy, x = (torch.randn(T, n, device=dev, generator=g).bfloat16() for n in (o, i))
+    got = kernels.weight_grad(dy, x)
+    want, mag = dy.double().t().contiguous() @ x.double(), dy.double().abs().t().contiguous() @ x.double().abs()
+    assert ((got.double() - want).abs() <= (T + 1) * 2.0 ** -24 * mag).all()
+    assert torch.equal(got, kernels.weight_grad(dy, x))
