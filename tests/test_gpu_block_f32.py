@@ -173,3 +173,30 @@ def test_block_f32_refuses_other_dtypes_and_outputs(dev):
     for out in (f32(1, 7, 7, 96), bf(0, 7, 7, 96)):
         with pytest.raises(ValueError):
             kernels.swin_block_f32(f32(0, 7, 7, 96), *args, out=out)
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("train", [False, True])
+def test_block_f32_keeps_a_bad_token_in_its_window(dev, bad, train):
+    """A NaN or infinity in tokens of one window (two of the same persistent
+    workgroup's among them) leaves every other window's bits alone."""
+    blk, _, x = _block(dev, (1, 140, 161, 1, (0, 0, 0, 0), 0, None, None, False, True, True))  # 20 x 23 windows
+    geom, attn, n = blk.geometry(1), blk.attn, blk.norm1
+    w, b = (torch.cat([getattr(l, p) for l in (attn.q_linear, attn.k_linear, attn.v_linear)]) for p in ("weight", "bias"))
+
+    def run(t):
+        with torch.no_grad():
+            if not train:
+                return blk(t.view(1, 140 * 161, 96)).view(140, 161, 96)
+            return kernels.swin_block_f32_train(t, geom, 3, attn.scale, w, b, attn.proj.weight, attn.proj.bias, n.weight,
+                                                n.bias, n.eps, attn._table(), blk.window_mask(geom))[0].view(140, 161, 96)
+
+    xd = x.to(dev).view(1, 140, 161, 96)
+    clean = run(xd)
+    xb = xd.clone()
+    hit = torch.zeros(140, 161, dtype=torch.bool, device=dev)
+    for wr, wc in ((0, 0), (11, 3)):  # windows 0 and 256: the first workgroup's two
+        hit[7 * wr + 3:7 * wr + 10, 7 * wc + 3:7 * wc + 10] = True  # the shifted window's tokens
+        xb[0, 7 * wr + 5, 7 * wc + 4, 7] = bad
+    got = run(xb)
+    assert torch.equal(got[~hit], clean[~hit]) and got[hit].isnan().all()
