@@ -157,8 +157,10 @@ def weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     over token slices and its sum, or for other token counts its plain product
     rounded to bf16: 524288 x 768 x 192 204 / 255, 524288 x 576 x 192 176 / 246,
     156672 x 4096 x 1024 1370 / 1562, 50176 x 512 x 128 25 / 31, 16385 x 1024 x 1024
-    49 / 140, 2001 x 1024 x 1024 25 / 22; equal at 524288 x 192 x 192 and 32768 x
-    768 x 768).  Other dtypes (and feature counts that
+    49 / 140, 2001 x 768 x 192 18 / 21; equal at 524288 x 192 x 192 and 32768 x
+    768 x 768; behind, with nothing else on the GPU's queue to wait for, at 300 to
+    1000 rows of wide layers, 1000 x 1024 x 1024 21 / 16, where the host's 24 us
+    for the library's call hide it).  Other dtypes (and feature counts that
     are no multiple of 16) take the library: for large T in fp16 k slices
     contracted as one batched GEMM with an fp32 output and then summed, since
     hipBLASLt takes no split-K tiles for a contraction this long."""
@@ -205,8 +207,10 @@ def _bias32(bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
 
 def _short_kernel(x: torch.Tensor, out_features: int) -> bool:
     """The short-row linear kernels serve and fill the chip with rows like x
-    (524288 rows, us, against the library's product: 192 -> 576 130 / 300,
-    192 -> 192 60 / 113; 50176 rows of 128 -> 384 12 / 28)."""
+    (us, against the library's product: 524288 rows of 192 -> 576 130 / 300,
+    192 -> 192 60 / 113; 50176 rows of 128 -> 384 12 / 28; with the weight's
+    packing, where 256 tiles just fill it: 16384 rows of 192 -> 192 6.0 / 8.5, 5504
+    of 192 -> 576 8.2 / 11.8, 4096 of 192 -> 768 with the GELU 9.4 / 16.6)."""
     return (kernels.linear_short_supported(x, x.shape[-1], out_features)
             and kernels.linear_short_fills(x.numel() // x.shape[-1], out_features))
 
@@ -541,8 +545,8 @@ class _AttentionHalf(torch.autograd.Function):
     instead of a chain of them: a small block's step is bound by the host
     (fp32, 56x56 tokens, C = 96: 757 us for 230 us of GPU work with separate
     functions, concatenation nodes and a fill per accumulator, 525-690 us so;
-    408-577 us with the fp32 kernel that serves that shape's whole forward in
-    one launch and keeps what the backward reads)."""
+    437-625 us, from run to run of the host, with the fp32 kernel that serves
+    that shape's whole forward in one launch and keeps what the backward reads)."""
 
     @staticmethod
     def forward(ctx, x, ln_w, ln_b, qw, kw, vw, qb, kb, vb, pw, pb, table, geom, eps, num_heads, scale, mask, fused):

@@ -225,6 +225,8 @@ int launch_short(ShortParams p, hipStream_t s) {
   return TERRA_OK;
 }
 
+// Waves: a block of 192 features where they divide the outputs, else of 128
+// (128 inputs: 512; 192 inputs: an MLP of 512 or 1024 hidden features, say).
 template <int kEpi>
 int dispatch_short(const ShortParams& p, int k, hipStream_t s) {
   if (k == 192) return p.N % 192 == 0 ? launch_short<6, 6, kEpi>(p, s) : launch_short<6, 4, kEpi>(p, s);
