@@ -127,13 +127,16 @@ class SequentialSwinTransformer(torch.nn.Module):
                 and dtype in (torch.float32, torch.float16, torch.bfloat16)
                 and row_bytes % 16 == 0 and row_bytes <= 4096 and self.embedding_dim <= 1024)
 
-    def _plain_attn(self) -> bool:
-        """attn's forward may be passed by: a WindowAttention itself, with no
-        forward of its own and no forward hooks that would see the call."""
-        attn, hooks = self.attn, torch.nn.modules.module
-        return (type(attn) is WindowAttention and "forward" not in attn.__dict__
-                and not (attn._forward_hooks or attn._forward_pre_hooks)
-                and not (hooks._global_forward_hooks or hooks._global_forward_pre_hooks))
+    @staticmethod
+    def _plain_attn(attn: torch.nn.Module, *methods: str) -> bool:
+        """attn's ``methods`` may be passed by: WindowAttention's own, neither
+        a subclass's nor the instance's, and no forward hooks that would see
+        the call."""
+        d, hooks, own = attn.__dict__, torch.nn.modules.module, type(attn)
+        return (d.keys().isdisjoint(methods) and not d["_forward_hooks"] and not d["_forward_pre_hooks"]
+                and not hooks._global_forward_hooks and not hooks._global_forward_pre_hooks
+                and (own is WindowAttention
+                     or all(getattr(own, m, None) is getattr(WindowAttention, m) for m in methods)))
 
     def _proj_scatter(self, x_windows: torch.Tensor, shortcut: torch.Tensor, geom: WindowGeometry) -> bool:
         """Whether the output projection, the window reverse and the residual
@@ -145,7 +148,9 @@ class SequentialSwinTransformer(torch.nn.Module):
         forward free to be passed by, a biased nn.Linear proj of the activation dtype (or fp32 under bf16
         autocast)."""
         C = geom.channels
-        if x_windows.dtype != torch.bfloat16 or shortcut.dtype != torch.bfloat16 or not self._plain_attn():
+        if x_windows.dtype != torch.bfloat16 or shortcut.dtype != torch.bfloat16:
+            return False
+        if not self._plain_attn(self.attn, "forward"):
             return False
         if not kernels.linear_supported(x_windows, C, C):
             return False
@@ -209,7 +214,7 @@ class SequentialSwinTransformer(torch.nn.Module):
         attn = self.attn
         if not self.use_fused_block or not kernels.swin_block_f32_supported(x, geom, attn.num_heads):
             return None
-        if not self._plain_attn():
+        if not self._plain_attn(attn, "forward", "attend", "qkv", "core"):
             return None
         if torch.is_autocast_enabled(x.device.type) or (config.use_layernorm and not self._fusable_norm(x.dtype)):
             return None
@@ -283,8 +288,8 @@ class SequentialSwinTransformer(torch.nn.Module):
             return y.view(B, H * W, C)
         f32_args = self._block_f32_args(grid, geom)
         if f32_args is not None:
-            mask = self.window_mask(geom)
-            y = kernels.swin_block_f32(grid, geom, self.attn.num_heads, self.attn.scale,
+            attn, mask = self.attn, self.window_mask(geom)
+            y = kernels.swin_block_f32(grid, geom, attn.num_heads, attn.scale,
                                        shift_mask=mask is not None and mask.shift is not None,
                                        land_bits=None if mask is None else mask.land_bits, **f32_args)
             return y.view(B, H * W, C)

@@ -306,6 +306,31 @@ def test_one_launch_blocks_keep_the_call_of_attn(dev, C, heads, ws, H, W, dtype,
     assert calls == [1]
 
 
+@pytest.mark.parametrize("C,heads,ws,H,W,dtype", ONE_LAUNCH_BLOCKS)
+@pytest.mark.parametrize("own", [None, "attend", "qkv"])
+def test_one_launch_blocks_of_a_subclass(dev, C, heads, ws, H, W, dtype, own, monkeypatch):
+    """A subclass of WindowAttention that keeps its forward takes the launches
+    that WindowAttention takes; one with an attend or qkv of its own has it
+    called (the scatter launch starts behind attend)."""
+    blk = SequentialSwinTransformer(layer_idx=0, height=H, width=W, embedding_dim=C, window_size=ws, num_heads=heads,
+                                    use_attn_mask=False, use_relative_position_bias=False)
+    blk = blk.to(dev, dtype)
+    x = workloads.activations((1, H * W, C), 91).to(dev, dtype)
+    entry = {7: "swin_block_f32", 32: "linear_scatter", 8: "linear_residual"}[ws]
+    launches, calls = [], []
+    real = getattr(kernels, entry)
+    monkeypatch.setattr(kernels, entry, lambda *a, **k: launches.append(1) or real(*a, **k))
+    methods = {}
+    if own is not None:
+        orig = getattr(blk.attn, own)
+        methods[own] = lambda self, *a, **k: calls.append(1) or orig(*a, **k)
+    blk.attn.__class__ = type("Own", (WindowAttention,), methods)
+    with torch.no_grad():
+        blk(x)
+    assert len(calls) == (own is not None)
+    assert len(launches) == (own is None or ws != 7)
+
+
 @pytest.mark.parametrize("C,heads,ws,H,W", [(512, 4, 32, 256, 128), (256, 2, 8, 16, 16)])
 def test_bf16_block_takes_x_at_any_offset(dev, C, heads, ws, H, W):
     """x two bytes off an 8-byte boundary, behind a norm that is not fused: the
